@@ -204,8 +204,9 @@ int mfc_diag_sums_noalloc(mfc_ctx* ctx, double* out6);
 /* Kinetic-energy spectrum of statistc (BOX/saveload.f90:1273-1300): u
  * transformed with forward sign and 1/n per axis (BOX/mpifft.f90:52-108);
  * ek[ik-1] = sum over modes 0 <= kx < nx/2 (weight 1/2 at kx = 0), all ky, kz,
- * with int(|k| + 0.5) = ik, for ik = 1..nek.  Uses a complex FP64 scratch
- * field of 16 bytes per node, allocated on first use. */
+ * with int(|k| + 0.5) = ik, for ik = 1..nek.  Uses an FP64 scratch
+ * field of 8 bytes per node (24 for boxes up to 128 MB of it), allocated on
+ * first use. */
 int mfc_diag_spectrum(mfc_ctx* ctx, int32_t nek, double* ek);
 
 /* ---- ensemble engine ------------------------------------------------------- */

@@ -1356,7 +1356,7 @@ int mfc_diag_spectrum(mfc_ctx* ctx, int32_t nek, double* ek) {
   if (rc) return rc;
   if ((rc = ensure_diag(ctx, nek))) return rc;
   if (!c.diag_Z) {
-    HIPCHK(hipMalloc(&c.diag_Z, sizeof(double2) * c.g.ncell));
+    HIPCHK(hipMalloc(&c.diag_Z, spectrum_scratch_bytes(c.g)));
     for (int a = 0; a < 3; ++a) {
       std::vector<double2> tw(ns[a]);
       for (int j = 0; j < ns[a]; ++j) {

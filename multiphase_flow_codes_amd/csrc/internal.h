@@ -203,7 +203,7 @@ struct Ctx {
   double* diag_part = nullptr;      // per-block partials
   double* diag_out = nullptr;       // results
   int diag_nek = 0;                 // shells the partials were sized for
-  double2* diag_Z = nullptr;        // complex FP64 field
+  double2* diag_Z = nullptr;        // half spectra (spectrum_scratch_bytes)
   double2* diag_tw[3] = {nullptr, nullptr, nullptr};   // exp(-2 pi i j / n) per axis
   void* ens = nullptr;              // the ensemble this box is a member of (its stream is on loan)
   int xcd_remap = -1;               // collide tile order over the XCDs (-1: by shape; MFC_XCD_REMAP=0/1/2)
@@ -270,6 +270,7 @@ hipError_t launch_field_sums(Ctx& c, double* part, double* out);
 // doubles and its address on the current device
 size_t sums_scratch_doubles();
 hipError_t sums_scratch(double** out);
+size_t spectrum_scratch_bytes(const Grid& g);
 hipError_t launch_spectrum(Ctx& c, int nek, double2* Z, const double2* const tw[3], double* part,
                            double* acc);
 

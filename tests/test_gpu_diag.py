@@ -40,6 +40,28 @@ def test_sums_and_spectrum_match_numpy(n):
     assert s2 == s
 
 
+# the transform's lengths: the power-of-two kernel's smallest, with a last
+# radix of 8, 4 and 2, short last tiles and its longest line; the general
+# kernel's with each factor, primes, odd row counts and its longest line
+@pytest.mark.parametrize("n", [(8, 8, 8), (16, 9, 32), (128, 4, 64), (4, 256, 6), (4, 5, 512), (1024, 5, 4),
+                               (4, 2048, 5), (4, 4, 2048), (6, 4, 25), (7, 11, 13), (9, 10, 49), (90, 77, 5),
+                               (5, 211, 7), (2047, 5, 4), (4, 4, 1458)])
+def test_spectrum_lengths_match_numpy(n):
+    from multiphase_flow_codes_amd.lbm import Lattice
+    from oracle.spectrum import spectrum
+    prm = small_params(n=n)
+    rng = np.random.default_rng(sum(n))
+    u = [rng.normal(0, 0.02, (n[2], n[1], n[0])) for _ in range(3)]
+    lat = Lattice(prm)
+    lat.upload_macro(np.zeros_like(u[0]), *u)
+    nek = max(n) // 2 + 2
+    ek = lat.diag_spectrum(nek)
+    want = spectrum(*u, nek)
+    assert np.max(np.abs(ek - want)) <= 1e-12 * np.max(want)
+    few = lat.diag_spectrum(2)
+    assert np.max(np.abs(few - want[:2])) <= 1e-12 * np.max(want)
+
+
 def test_sums_after_particle_steps_match_downloaded_fields():
     from multiphase_flow_codes_amd.lbm import Lattice
     rng = np.random.default_rng(3)
