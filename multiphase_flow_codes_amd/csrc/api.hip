@@ -658,17 +658,12 @@ int mfc_init_velocity(mfc_ctx* ctx, const double* amp, double scale) {
   if (rc) return rc;
   const size_t nk = (size_t)init_mode_k(), nkx = (size_t)init_mode_kx();
   const size_t na = 3 * nkx * nk * nk;
-  const size_t n1 = nk * nk * (size_t)c.g.nx, n2 = nk * (size_t)c.g.nx * (size_t)c.g.ny;
-  double2 *d_amp = nullptr, *B1 = nullptr, *B2 = nullptr;
-  hipError_t e = hipMalloc(&d_amp, sizeof(double2) * na);
-  if (e == hipSuccess) e = hipMalloc(&B1, sizeof(double2) * n1);
-  if (e == hipSuccess) e = hipMalloc(&B2, sizeof(double2) * n2);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_amp, amp, sizeof(double2) * na, hipMemcpyHostToDevice, c.stream);
-  if (e == hipSuccess) e = launch_init_velocity(c, d_amp, scale, B1, B2);
+  double2* d = nullptr;   // the mode table, then the scratch
+  hipError_t e = hipMalloc(&d, sizeof(double2) * (na + init_scratch(c.g)));
+  if (e == hipSuccess) e = hipMemcpyAsync(d, amp, sizeof(double2) * na, hipMemcpyHostToDevice, c.stream);
+  if (e == hipSuccess) e = launch_init_velocity(c, d, scale, d + na);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-  if (d_amp) (void)hipFree(d_amp);
-  if (B1) (void)hipFree(B1);
-  if (B2) (void)hipFree(B2);
+  if (d) (void)hipFree(d);
   if (e != hipSuccess) return fail(ctx, MFC_ERR_HIP, "mfc_init_velocity", e);
   c.mom = MOM_ARRAYS;
   return MFC_OK;

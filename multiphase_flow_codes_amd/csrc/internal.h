@@ -261,7 +261,8 @@ hipError_t launch_links_dense(Ctx& c, int32_t* ilink, int32_t* mlink, double* al
 // ---- launchers (initial.hip) ----
 int init_mode_kx();   // kx values of the mode table (0..16)
 int init_mode_k();    // ky, kz values (-16..16)
-hipError_t launch_init_velocity(Ctx& c, const double2* amp, double scale, double2* B1, double2* B2);
+size_t init_scratch(const Grid& g);   // double2 elements of launch_init_velocity's scratch
+hipError_t launch_init_velocity(Ctx& c, const double2* amp, double scale, double2* work);
 
 // ---- launchers (diag.hip) ----
 int diag_blocks();
