@@ -53,7 +53,6 @@ int fail(mfc_ctx* ctx, int code, const char* what, hipError_t e = hipSuccess) {
   if (!ctx) return MFC_ERR_ARG
 
 __global__ void k_set_status(int32_t* st, int idx, int val) { st[idx] = val; }
-__global__ void k_set_double(double* d, double v) { d[0] = v; }
 __global__ void k_fill_i32(int32_t* a, uint64_t n, int32_t v) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) a[i] = v;
@@ -436,7 +435,7 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   CK(hipMalloc(&c.d_status, sizeof(int32_t) * ST_COUNT));
   CK(hipMemsetAsync(c.d_status, 0, sizeof(int32_t) * ST_COUNT, c.stream));
   CK(hipHostMalloc((void**)&c.h_status, sizeof(int32_t) * ST_COUNT, hipHostMallocDefault));
-  CK(hipMalloc(&c.d_red, sizeof(double) * 8));
+  CK(hipMalloc(&c.d_red, sizeof(double) * (size_t)rhoupdat_blocks(c)));
   CK(hipHostMalloc((void**)&c.h_red, sizeof(double) * 8, hipHostMallocDefault));
   // this device's static scratch of the allocation-free sums
   CK(sums_scratch(&c.sums_scratch));
@@ -726,12 +725,9 @@ int mfc_rhoupdat(mfc_ctx* ctx, double* maxdiff) {
   Ctx& c = ctx->c;
   int rc = need_arrays(ctx);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_set_double, dim3(1), dim3(1), 0, c.stream, c.d_red, 0.0);
-  HIPCHK(hipGetLastError());
-  HIPCHK(launch_rhoupdat(c, c.phase == PHASE_POST_STREAM, c.d_red));
+  HIPCHK(launch_rhoupdat(c, c.phase == PHASE_POST_STREAM, c.d_red, maxdiff ? c.h_red : nullptr));
   c.mom = MOM_ARRAYS;
   if (maxdiff) {
-    HIPCHK(hipMemcpyAsync(c.h_red, c.d_red, sizeof(double), hipMemcpyDeviceToHost, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
     *maxdiff = c.h_red[0];
   }

@@ -186,7 +186,7 @@ struct Ctx {
   Particles pt;
   int32_t* d_status = nullptr;
   int32_t* h_status = nullptr;      // pinned
-  double* d_red = nullptr;          // small reduction buffer
+  double* d_red = nullptr;          // workgroup maxima of rhoupdat
   double* h_red = nullptr;          // pinned
   void* staging = nullptr;          // device staging for host transfers
   size_t staging_bytes = 0;
@@ -225,7 +225,9 @@ hipError_t launch_collide(Ctx& c, bool arrays);
 // `list`; with far set the solid mask is not read
 hipError_t launch_collide_tiles(Ctx& c, const uint32_t* list, uint32_t n, bool far);
 hipError_t launch_macro(Ctx& c, bool pulled);
-hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* d_maxdiff);
+int rhoupdat_blocks(const Ctx& c);   // workgroup maxima launch_rhoupdat leaves in `part`
+// out (device-visible, may be null): max |rho_new - rho_old|
+hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out);
 hipError_t launch_initpop(Ctx& c);
 hipError_t launch_pop_to_aos(Ctx& c, double* dst, int z0, int nzs, bool pulled);
 hipError_t launch_aos_to_pop(Ctx& c, const double* src, int z0, int nzs, bool pulled);
