@@ -31,6 +31,19 @@ constexpr int kTimingPool = 8192;
 // contact links the reference-order bounce-back can hold (48 B each)
 constexpr int64_t kOrderCap = int64_t(1) << 16;
 
+// Elements from one direction's row to the next in the row-interleaved layout:
+// nx rounded up to whole 128-B lines where that adds at most a tenth, else to
+// 64 B, so that a wavefront's run of a row starts on a line and two rows never
+// share one.  Two buffers only: in place the unwritten ends of the lines cost
+// more than the shared ones (150 x 141 x 162 FP64 240 us padded, 200 not).
+// Fluid steps, two buffers: 150 x 141 x 162 FP32 111-149 us unpadded and 98
+// padded, 1000 x 400 x 128 FP32 1562 us at 64 B and 1385 at 128 B.
+uint64_t row_pitch(uint64_t nx, size_t tsize, bool two_buffers) {
+  if (!two_buffers) return nx;
+  const uint64_t b = nx * tsize, line = (b + 127) / 128 * 128, half = (b + 63) / 64 * 64;
+  return (10 * line <= 11 * b ? line : half) / tsize;
+}
+
 int fail(mfc_ctx* ctx, int code, const char* what, hipError_t e = hipSuccess) {
   if (ctx) {
     char buf[512];
@@ -356,7 +369,7 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   }
   {
     const char* e = getenv("MFC_XCD_REMAP");
-    c.xcd_remap = (e && e[0] >= '0' && e[0] <= '2') ? e[0] - '0' : -1;
+    c.xcd_remap = (e && (e[0] == '0' || e[0] == '1')) ? e[0] - '0' : -1;
   }
   {
     // The overlapped step is opt-in: at 1024^3 with 20,000 spheres the
@@ -375,8 +388,8 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
     // 4 GB apart.  Measured against the plane-major layout, alternating in
     // one box: FP32 collide 2.6 % faster at 1024^3 and 8 % at 256^3 (step
     // 2.5 % and 5 %), FP64 in place 2.3 % faster at 1024^3, FP64 and FP32
-    // storage with FP64 collision unchanged at 256^3; padding the plane
-    // stride or the row group was slower in a probe of the access pattern.
+    // storage with FP64 collision unchanged at 256^3.  Rows are padded as
+    // row_pitch says.
     // MFC_POP_LAYOUT=planes selects plane-major planes instead, 512 B
     // further apart than the node count (a power-of-two plane size would
     // start every stream at the same offset of each page; 512 B measured
@@ -389,8 +402,8 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
       if (pad >= 0 && pad < (1L << 20)) c.g.pitch = ncell + (uint64_t)pad * (256 / c.tsize);
       c.g.rs = (uint64_t)c.g.nx;
     } else {
-      c.g.pitch = (uint64_t)c.g.nx;
-      c.g.rs = (uint64_t)NPOP * c.g.nx;
+      c.g.pitch = row_pitch((uint64_t)c.g.nx, c.tsize, c.g.lay == LAY_AB);
+      c.g.rs = (uint64_t)NPOP * c.g.pitch;
     }
   }
   c.iseedf = p->iseedf;
@@ -406,8 +419,9 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   } while (0)
   CK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
   c.own_stream = true;
-  // one past the last element: plane 18, the last row, x = nx - 1
-  const size_t pelems = (size_t)(NPOP - 1) * c.g.pitch + (size_t)(ncell / c.g.nx - 1) * c.g.rs + c.g.nx;
+  // one past the last element: plane 18, the last row, its whole pitch
+  const size_t pelems = (size_t)(NPOP - 1) * c.g.pitch + (size_t)(ncell / c.g.nx - 1) * c.g.rs +
+                        (c.g.rs == (uint64_t)c.g.nx ? (size_t)c.g.nx : (size_t)c.g.pitch);
   const size_t pb = std::max(pelems, (size_t)NPOP * (c.g.rs == (uint64_t)c.g.nx ? c.g.pitch : 0)) * c.tsize;
   CK(hipMalloc(&c.pop[0], pb));
   CK(hipMemsetAsync(c.pop[0], 0, pb, c.stream));

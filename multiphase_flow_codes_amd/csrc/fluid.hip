@@ -64,11 +64,10 @@ __device__ __forceinline__ void force_row(const double* __restrict__ t, R c1, R 
 
 // Fused stream + macro + forcing + MRT collision.
 //
-// Launch: blockIdx.z = z, blockIdx.y = y, blockIdx.x * blockDim.x + lane = x.
-// Everything that depends on (y, z) only -- the nine neighbour-row offsets,
+// One wavefront per tile of 64 consecutive x nodes of a row (kTileX):
+// everything that depends on (y, z) only -- the nine neighbour-row offsets,
 // the wall test and the forcing-table rows -- is wave-uniform and lives in
-// scalar registers; per lane only x +- 1 wraps.  Stores are non-temporal:
-// the post-collision field is not re-read until the next step.
+// scalar registers; per lane only x +- 1 wraps.
 //
 // ARR: conserved moments from the rho/u arrays (the reference's literal data
 // flow, used while they are authoritative, e.g. the pre-relaxation);
@@ -81,11 +80,9 @@ __device__ __forceinline__ void force_row(const double* __restrict__ t, R c1, R 
 // node touches exactly the locations it read and nodes never race.  From
 // LAY_AA_ODD that is all in the node's own slots; from LAY_AA_EVEN it is the
 // neighbours' (the result is in LAY_AA_ODD, and the other way round).
-// NTL: the two-buffer field is read with non-temporal loads (it is not read
-// again this step); with rows split over several x-chunks plain loads let the
-// chunks share the cache lines at their edges (1024^3: 1.2 % faster collide;
-// whole rows at 256^3: 3-8 % slower with plain loads).
-template <typename T, typename R, bool ARR, bool WALLS, int LAY, bool NTL = true>
+// NTL, NTS: non-temporal loads of the two-buffer field, non-temporal stores
+// (CollideShape says when).
+template <typename T, typename R, bool ARR, bool WALLS, int LAY, bool NTL, bool NTS>
 __device__ __forceinline__ void collide_node(const CollideArgs& a, int x, int y, int z) {
   const T* __restrict__ A = (const T*)a.A;
   T* __restrict__ B = (T*)a.B;
@@ -182,7 +179,10 @@ __device__ __forceinline__ void collide_node(const CollideArgs& a, int x, int y,
     T* q = B + own;
 #pragma unroll
     for (int i = 0; i < NPOP; ++i) {
-      __builtin_nontemporal_store((T)f[i], q);
+      if (NTS)
+        __builtin_nontemporal_store((T)f[i], q);
+      else
+        *q = (T)f[i];
       q += g.pitch;
     }
   } else {
@@ -196,58 +196,43 @@ __device__ __forceinline__ void collide_node(const CollideArgs& a, int x, int y,
   }
 }
 
-// Workgroups are dealt to the XCDs round-robin in launch order, and each XCD
-// has its own L2.  The tile (x-chunk bx, row) of launch index L:
-//   remap 0: L = bx + nbx * row (x-chunk fastest);
-//   remap 1: each XCD takes a contiguous range of tiles (rows and their chunks);
-//   remap 2: rows stay dealt round-robin (row r on XCD r % 8, so the XCDs
-//            sweep neighbouring addresses together) but all x-chunks of a
-//            row run on the row's XCD, whose L2 then holds the cache lines
-//            the chunks share at their edges.
+// Workgroups are dealt to the 8 XCDs round-robin in launch order, and each XCD
+// has its own L2.  With per = grid / 8 each XCD takes a contiguous range of
+// workgroups instead (per = 0: launch order).
 constexpr uint32_t kXcds = 8;
-__device__ __forceinline__ void xcd_tile(uint32_t L, uint32_t total, uint32_t nbx, int remap,
-                                         uint32_t& bx, uint32_t& row) {
-  if (remap == 1) {
-    const uint32_t per = total / kXcds;
-    const uint32_t t = L >= per * kXcds ? L : (L % kXcds) * per + L / kXcds;
-    bx = t % nbx;
-    row = t / nbx;
-    return;
-  }
-  if (remap == 2 && nbx > 1) {
-    const uint32_t group = kXcds * nbx;          // 8 rows, all their chunks
-    const uint32_t full = (total / group) * group;
-    if (L < full) {
-      const uint32_t q = L / group, r = L - q * group;
-      bx = r / kXcds;
-      row = q * kXcds + r % kXcds;
-      return;
-    }
-  }
-  bx = L % nbx;
-  row = L / nbx;
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t per) {
+  return b < per * kXcds ? (b % kXcds) * per + b / kXcds : b;
 }
+
+// The tiles of a lattice, `waves` per workgroup, numbered x fastest.
+struct TileGrid {
+  FastDiv tpr, ny;    // tiles per row, rows per plane
+  uint32_t ntiles, per, waves;
+};
 
 // FP32 storage with FP64 arithmetic, two buffers: 4 waves per SIMD (128
 // VGPRs, 20-28 B/lane of spills) instead of 3 (132 VGPRs) measured 6 % faster
-// at 256^3; the same bound on the FP64 kernel made it 4 % slower.
-template <typename T, typename R, bool ARR, bool WALLS, int LAY, bool NTL>
+// at 256^3; the same bound on the FP64 kernel made it 3 % slower there and at
+// 512^3 (897 against 872 us, 7.16 against 6.93 ms).
+template <typename T, typename R, bool ARR, bool WALLS, int LAY, bool NTL, bool NTS>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && sizeof(R) == 8 && LAY == LAY_AB ? 4 : 1)))
-    k_collide(CollideArgs a, int nbx, int remap) {
-  uint32_t bx, row;
-  xcd_tile(blockIdx.x, gridDim.x, (uint32_t)nbx, remap, bx, row);
-  const int x = (int)(bx * blockDim.x + threadIdx.x);
+    k_collide(CollideArgs a, TileGrid g) {
+  const uint32_t b = xcd_block(blockIdx.x, g.per);
+  // the wavefront's index is uniform: keep it (and the tile, row, y, z) scalar
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t t = b * g.waves + w;
+  if (t >= g.ntiles) return;
+  const uint32_t row = div_by(t, g.tpr);
+  const int x = (int)((t - row * g.tpr.d) * (uint32_t)kTileX + (threadIdx.x & 63u));
   if (x >= a.g.nx) return;
-  const uint32_t y = row % (uint32_t)a.g.ny, z = row / (uint32_t)a.g.ny;
-  collide_node<T, R, ARR, WALLS, LAY, NTL>(a, x, (int)y, (int)z);
+  const uint32_t z = div_by(row, g.ny);
+  collide_node<T, R, ARR, WALLS, LAY, NTL, NTS>(a, x, (int)(row - z * g.ny.d), (int)z);
 }
 
-// The collide of the tiles of a list (overlapped step): one tile (kTileX
-// nodes of a row) per wavefront, four per workgroup, the grid sized to the
-// list.  Workgroups are dealt to the XCDs round-robin (workgroup b runs on
-// XCD b % 8), so the launch index is remapped to give each XCD a contiguous
-// range of the list, in order: neighbouring rows then meet in one L2.
+// The collide of the tiles of a list (overlapped step): one tile per
+// wavefront, four per workgroup, the grid sized to the list, each XCD a
+// contiguous range of it: neighbouring rows then meet in one L2.
 // Occupancy as the plain collide reaches it: FP32 storage with FP64
 // arithmetic held to 4 waves per SIMD with two buffers; FP64 arithmetic in
 // place held to 3 (the in-place layouts with walls otherwise take 178 VGPRs,
@@ -261,10 +246,7 @@ template <typename T, typename R, bool WALLS, int LAY>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(tile_waves<T, R>(LAY))))
     k_collide_tiles(CollideArgs a, const uint32_t* __restrict__ list, uint32_t n, uint32_t tpr) {
-  uint32_t b = blockIdx.x;
-  const uint32_t per = gridDim.x / kXcds;
-  if (b < per * kXcds) b = (b % kXcds) * per + b / kXcds;
-  // the wavefront's index is uniform: keep it (and the tile, row, y, z) scalar
+  const uint32_t b = xcd_block(blockIdx.x, gridDim.x / kXcds);
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t L = b * 4u + w;
   if (L >= n) return;
@@ -272,7 +254,7 @@ __global__ void __launch_bounds__(256)
   const uint32_t row = t / tpr;
   const int x = (int)((t - row * tpr) * (uint32_t)kTileX + (threadIdx.x & 63u));
   if (x >= a.g.nx) return;
-  collide_node<T, R, false, WALLS, LAY>(a, x, (int)(row % (uint32_t)a.g.ny), (int)(row / (uint32_t)a.g.ny));
+  collide_node<T, R, false, WALLS, LAY, true, true>(a, x, (int)(row % (uint32_t)a.g.ny), (int)(row / (uint32_t)a.g.ny));
 }
 
 // Several boxes in one grid (ensemble engine): block b belongs to box c with
@@ -290,19 +272,13 @@ __device__ __forceinline__ int case_of_block(const int* __restrict__ off, int nc
 
 // ARR_ANY: some member takes its moments from the rho/u arrays (a.arr, its
 // first step after joining); without it only the recomputing path is built.
-// remap = 1 deals the grid to the 8 XCDs in contiguous ranges (workgroups are
-// dispatched to the XCDs round-robin, so launch-order block b runs on XCD
-// b % 8): consecutive node ranges, whose neighbour rows overlap, then share
-// one L2.  The block-to-nodes map is a bijection either way, so results do
+// remap = 1 deals the grid to the 8 XCDs in contiguous ranges: consecutive
+// node ranges, whose neighbour rows overlap, then share one L2.  The block-to-nodes map is a bijection either way, so results do
 // not depend on it.
 template <typename T, typename R, bool WALLS, int BS, bool ARR_ANY>
 __global__ void __launch_bounds__(BS)
     kb_collide(const CollideArgs* __restrict__ t, const int* __restrict__ off, int nc, int remap) {
-  uint32_t b = blockIdx.x;
-  if (remap) {
-    const uint32_t per = gridDim.x / kXcds;
-    if (b < per * kXcds) b = (b % kXcds) * per + b / kXcds;
-  }
+  const uint32_t b = xcd_block(blockIdx.x, remap ? gridDim.x / kXcds : 0);
   const int c = case_of_block(off, nc, (int)b);
   const CollideArgs a = t[c];
   const uint64_t n = (uint64_t)((int)b - off[c]) * BS + threadIdx.x;
@@ -311,9 +287,9 @@ __global__ void __launch_bounds__(BS)
   const uint32_t x = (uint32_t)(n % nx);
   const uint32_t r = (uint32_t)(n / nx);
   if (ARR_ANY && a.arr)
-    collide_node<T, R, true, WALLS, LAY_AB>(a, (int)x, (int)(r % ny), (int)(r / ny));
+    collide_node<T, R, true, WALLS, LAY_AB, true, true>(a, (int)x, (int)(r % ny), (int)(r / ny));
   else
-    collide_node<T, R, false, WALLS, LAY_AB>(a, (int)x, (int)(r % ny), (int)(r / ny));
+    collide_node<T, R, false, WALLS, LAY_AB, true, true>(a, (int)x, (int)(r % ny), (int)(r / ny));
 }
 
 // Forcing table of one step (force_table.h): one thread per (row, component).
@@ -526,16 +502,6 @@ hipError_t launch_force_table(Ctx& c, int slot, const ModeSet& m) {
   return hipGetLastError();
 }
 
-// x-row blocks: 64..256 lanes covering a row, one block per (x-chunk, y, z),
-// a one-dimensional grid of nbx * ny * nz tiles
-static void row_launch(const Grid& g, dim3& grid, dim3& blk, int& nbx) {
-  int bx = ((g.nx + 63) / 64) * 64;
-  if (bx > 256) bx = 256;
-  blk = dim3(bx);
-  nbx = (g.nx + bx - 1) / bx;
-  grid = dim3((unsigned)((uint64_t)nbx * g.ny * g.nz));
-}
-
 // Arguments of one box's collide launch (also used by the ensemble engine).
 CollideArgs collide_args(Ctx& c) {
   CollideArgs a;
@@ -550,39 +516,106 @@ CollideArgs collide_args(Ctx& c) {
   return a;
 }
 
-template <typename T, typename R, int LAY, bool NTL>
-static void collide_launch(Ctx& c, bool arrays, const CollideArgs& a, dim3 grid, dim3 blk, int nbx,
-                           int rm) {
+// How the collide of a box is launched.  Measured on one MI355X, us per
+// collide, in fluid-only steps (f) and in steps with spheres (s), whose other
+// kernels run between two collides:
+//  waves   4 wavefronts per workgroup, 3 where rows are a multiple of three
+//          tiles, so that workgroups hold whole rows (192 x 176 x 208 FP32 step
+//          with spheres 282 against 284); 1 where the lattice has at most
+//          16 tiles per CU (48^3 FP64 f 8.7 against 9.1).
+//  cached  plain stores where both buffers stay in the 256 MiB last-level
+//          cache between steps: from 48 MiB (64^3 FP32, 38 MiB, s 13.1 against
+//          11.6 non-temporal; 64^3 FP64, 76 MiB, s 18.6 against 20.2, f 14.0
+//          against 17.3) to 260 MiB (96^3 FP64, 257 MiB, f 43 against 47, s 49
+//          against 53; 130 x 118 x 126 FP32, 280 MiB, f 64 against 60).
+//  ntl     non-temporal loads.  Small lattices (up to 48 MiB: 48^3 FP32 f 5.6
+//          against 6.3).  FP64 with spheres (256^3 s 860 against 897, 448 x
+//          256 x 256 s 1536 against 1570; without them f 877 against 875, 262
+//          x 257 x 227 f 841 against 811).  FP32 storage with FP64 arithmetic
+//          with spheres (256^3 s 454 against 474, 262 x 257 x 227 s 486
+//          against 491) and in rows of whole workgroups (256^3 f 442 against
+//          451, but 262 x 257 x 227 f 468 against 450).  FP32 with spheres
+//          where a workgroup holds whole rows (256^3 s 430 against 443; 290 x
+//          280 x 270 s 722 against 663, where workgroups end inside rows and
+//          the next one needs the same cache lines; 256^3 f 451 against 438).
+//  per     contiguous workgroups per XCD instead of launch order.  Two
+//          buffers: when the 19 populations of a plane reach 18 MiB (512^3
+//          FP32 f 3.36 against 3.45-3.61 ms, 1024^3 26.6 against 29.1 ms; 320
+//          x 288 x 304 FP32 f 759 against 719), and in lattices up to 128 MiB,
+//          whose nodes then meet the same L2 in the next step (40^3 FP32 f 5.0
+//          against 6.2).  In place: always (1024^3 FP64 f 52.5 against 64 ms,
+//          130 x 118 x 126 FP32 47 against 58), but rows of up to four tiles
+//          that outgrow the last-level cache (200 x 190 x 210 FP64 f 461
+//          against 441).
+// One workgroup per row or 256-node chunk of a row, the shape before, left
+// half of its lanes idle where a row ends in a short chunk: 320 x 288 x 304
+// FP32 f 912 us (now 715) and FP64 in place 1790 (now 1575), 262 x 257 x 227
+// FP32 f 773 (now 436), s 785 (now 444) and FP64 f 1226 (now 800), s 1224 (now
+// 825); other rows gain from the plain loads and the padding: 150 x 141 x 162
+// FP32 f 136 (98), s 134 (97) and FP64 s 232 (195), 96^3 FP64 s 55 (49).
+struct CollideShape {
+  TileGrid t;
+  unsigned grid, block;
+  bool cached, ntl;
+};
+template <typename T, typename R>
+static CollideShape collide_shape(const Ctx& c, bool spheres) {
+  CollideShape s;
+  const uint32_t tpr = (uint32_t)((c.g.nx + kTileX - 1) / kTileX);
+  s.t.tpr = fast_div(tpr);
+  s.t.ny = fast_div((uint32_t)c.g.ny);
+  s.t.ntiles = tpr * (uint32_t)c.g.ny * (uint32_t)c.g.nz;
+  s.t.waves = s.t.ntiles <= 4096 ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
+  s.block = (unsigned)kTileX * s.t.waves;
+  s.grid = (s.t.ntiles + s.t.waves - 1) / s.t.waves;
+  const bool ab = c.g.lay == LAY_AB;
+  const uint64_t mib = (uint64_t)1 << 20;
+  const uint64_t buf = (uint64_t)NPOP * sizeof(T) * c.g.ncell;
+  const uint64_t plane = (uint64_t)NPOP * sizeof(T) * (uint64_t)c.g.nx * (uint64_t)c.g.ny;
+  const bool small = 2 * buf <= 48 * mib;
+  s.cached = ab && !small && 2 * buf <= 260 * mib;
+  if (sizeof(T) != sizeof(R))
+    s.ntl = small || spheres || c.g.nx % 256 == 0;
+  else
+    s.ntl = small || (spheres && (sizeof(T) == 8 || (c.g.nx % kTileX == 0 && s.t.waves % tpr == 0)));
+  bool ranges;
+  if (c.xcd_remap >= 0)
+    ranges = c.xcd_remap != 0;
+  else if (ab)
+    ranges = plane >= 18 * mib || 2 * buf <= 128 * mib;
+  else
+    ranges = !(tpr <= 4 && buf > 256 * mib);
+  s.t.per = ranges ? s.grid / kXcds : 0;
+  return s;
+}
+
+template <typename T, typename R, int LAY, bool NTL, bool NTS>
+static void collide_launch(Ctx& c, bool arrays, const CollideArgs& a, const CollideShape& s) {
+  const dim3 grid(s.grid), blk(s.block);
+#define MFC_COLLIDE(ARR, W) \
+  hipLaunchKernelGGL((k_collide<T, R, ARR, W, LAY, NTL, NTS>), grid, blk, 0, c.stream, a, s.t)
   if (arrays) {
-    if (c.g.walls_y)
-      hipLaunchKernelGGL((k_collide<T, R, true, true, LAY, NTL>), grid, blk, 0, c.stream, a, nbx, rm);
-    else
-      hipLaunchKernelGGL((k_collide<T, R, true, false, LAY, NTL>), grid, blk, 0, c.stream, a, nbx, rm);
+    if (c.g.walls_y) MFC_COLLIDE(true, true); else MFC_COLLIDE(true, false);
   } else {
-    if (c.g.walls_y)
-      hipLaunchKernelGGL((k_collide<T, R, false, true, LAY, NTL>), grid, blk, 0, c.stream, a, nbx, rm);
-    else
-      hipLaunchKernelGGL((k_collide<T, R, false, false, LAY, NTL>), grid, blk, 0, c.stream, a, nbx, rm);
+    if (c.g.walls_y) MFC_COLLIDE(false, true); else MFC_COLLIDE(false, false);
   }
+#undef MFC_COLLIDE
 }
 
 template <typename T, typename R, int LAY>
 static void collide_dispatch_lay(Ctx& c, bool arrays, const CollideArgs& a) {
-  dim3 grid, blk;
-  int nbx;
-  row_launch(c.g, grid, blk, nbx);
-  // rows split over several chunks (nx > 256), or FP64 arithmetic on FP64
-  // populations: contiguous tile ranges per XCD; otherwise launch order
-  // (measured best for each: at 256^3 FP64 2.3 % faster step with ranges,
-  // FP32 2.7 % slower)
-  const int rm = c.xcd_remap >= 0 ? c.xcd_remap : ((nbx > 1 || sizeof(T) == 8) ? 1 : 0);
+  const CollideShape s = collide_shape<T, R>(c, a.mask != nullptr);
   if constexpr (LAY == LAY_AB) {
-    if (nbx > 1) {   // rows in several x-chunks: plain loads
-      collide_launch<T, R, LAY, false>(c, arrays, a, grid, blk, nbx, rm);
+    if (s.cached) {
+      collide_launch<T, R, LAY, false, false>(c, arrays, a, s);
+      return;
+    }
+    if (s.ntl) {
+      collide_launch<T, R, LAY, true, true>(c, arrays, a, s);
       return;
     }
   }
-  collide_launch<T, R, LAY, true>(c, arrays, a, grid, blk, nbx, rm);
+  collide_launch<T, R, LAY, false, true>(c, arrays, a, s);
 }
 
 template <typename T, typename R>

@@ -46,8 +46,8 @@ constexpr int kScanChunk = 4096;
 // a segment's links are split over up to this many bounce-back workgroups
 constexpr int kMaxBBSplit = 4;
 constexpr int kCellCap = 16;
-// overlapped step: tiles of kTileX consecutive x nodes of a row, classified
-// near/far in chunks of kTileChunk tiles
+// the collide's tiles, kTileX consecutive x nodes of a row (one wavefront);
+// the overlapped step classifies them near/far in chunks of kTileChunk
 constexpr int kTileX = 64;
 constexpr int kTileChunk = 4096;
 
@@ -206,7 +206,7 @@ struct Ctx {
   double2* diag_Z = nullptr;        // half spectra (spectrum_scratch_bytes)
   double2* diag_tw[3] = {nullptr, nullptr, nullptr};   // exp(-2 pi i j / n) per axis
   void* ens = nullptr;              // the ensemble this box is a member of (its stream is on loan)
-  int xcd_remap = -1;               // collide tile order over the XCDs (-1: by shape; MFC_XCD_REMAP=0/1/2)
+  int xcd_remap = -1;               // collide tile order over the XCDs (-1: by shape; MFC_XCD_REMAP=0/1)
   double* sums_scratch = nullptr;   // this device's static scratch of mfc_diag_sums_noalloc
   // overlapped step (mfc_step with spheres): the particle phase of step n runs
   // on pstream while the collide of step n + 1 covers the tiles far from every

@@ -64,6 +64,30 @@ struct CollideConsts {
 // layout an upload writes and the first collide reads in place.
 enum PopLayout { LAY_AB = 0, LAY_AA_EVEN = 1, LAY_AA_ODD = 2 };
 
+// Division by a divisor known on the host: n / d for n < 2^31 as one high
+// multiply, an add and a shift (round-up method: sh = ceil(log2 d), mul =
+// floor(2^32 (2^sh - d) / d) + 1).  A 32-bit division by a kernel argument is
+// some 25 instructions, a chain that every wavefront starts with.
+struct FastDiv {
+  uint32_t d, mul, sh;
+};
+inline FastDiv fast_div(uint32_t d) {
+  FastDiv f;
+  f.d = d;
+  f.sh = 0;
+  while (((uint64_t)1 << f.sh) < d) ++f.sh;
+  f.mul = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << f.sh) - d)) / d + 1);
+  return f;
+}
+MFC_HD uint32_t div_by(uint32_t n, const FastDiv& f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t hi = __umulhi(n, f.mul);
+#else
+  const uint32_t hi = (uint32_t)(((uint64_t)n * f.mul) >> 32);
+#endif
+  return (hi + n) >> f.sh;
+}
+
 // Grid geometry handed to the kernels.
 struct Grid {
   int nx, ny, nz;

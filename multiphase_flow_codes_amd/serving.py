@@ -85,7 +85,7 @@ class BoxCase:
     def footprint_bytes(self, precision: str) -> int:
         """Device memory make_lattice allocates for the case: the sizes
         mfc_create and mfc_prt_init request (populations A/B, 19 values per
-        node each, forcing tables, moments, particle arrays, segment lists, link
+        node of padded rows each, forcing tables, moments, particle arrays, segment lists, link
         pool, refill list, node maps), each rounded up to the allocator's
         granularity (4 KiB below 1 MiB, 2 MiB above), plus 16 MiB for the
         runtime's per-context state.  An upper bound of the hipMemGetInfo
@@ -93,7 +93,9 @@ class BoxCase:
         t = 8 if precision == "fp64" else 4
         n, np_, r = self.n, self.npart, self.rad
         ncell = n ** 3
-        allocs = [19 * ncell * t] * 2 + [8 * 18 * n * n] * 4 + [8 * 6 * n, 64, 64] + [8 * ncell] * 4
+        # rows padded to whole 128-B lines where that adds at most a tenth, else to 64 B
+        line, half = -(-n * t // 128) * 128, -(-n * t // 64) * 64
+        allocs = [19 * n * n * (line if 10 * line <= 11 * n * t else half)] * 2 + [8 * 18 * n * n] * 4 + [8 * 6 * n, 64, 64] + [8 * ncell] * 4
         if np_ > 0:
             allocs += [8 * 3 * np_] * 16
             maxcnt = math.ceil(2.0 * (r + 2.0) + 1.0) + 4
