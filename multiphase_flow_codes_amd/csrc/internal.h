@@ -156,6 +156,7 @@ struct Particles {
   int32_t* cell_cnt = nullptr;
   int32_t* cell_list = nullptr;
   bool cells_ok = false;
+  bool cells_zeroed = false;   // cleared by the fused bounce-back grid for the move that follows
   // nodes to refill, found by beads_filling's first pass
   uint64_t* fill_list = nullptr;
   int32_t* fill_count = nullptr;

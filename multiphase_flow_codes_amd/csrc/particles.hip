@@ -102,22 +102,24 @@ __global__ void k_cell_zero(int32_t* __restrict__ cnt, int n) {
   if (i < n) cnt[i] = 0;
 }
 
-__global__ void __launch_bounds__(256)
-    k_cell_build(const double* __restrict__ ypglb, int np, PGeom G, CellArgs C,
-                 int32_t* __restrict__ status) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  if (!(sane_coord(ypglb[3 * p], G.nx) && sane_coord(ypglb[3 * p + 1], G.ny) &&
-        sane_coord(ypglb[3 * p + 2], G.nz)))
+// Enters particle p, centre (x, y, z), in its cell.
+__device__ __forceinline__ void cell_insert(int p, double x, double y, double z, const PGeom& G,
+                                            const CellArgs& C, int32_t* __restrict__ status) {
+  if (!(sane_coord(x, G.nx) && sane_coord(y, G.ny) && sane_coord(z, G.nz)))
     return;   // reported by the move / links kernels
-  int a, b, c;
-  cell_coords(ypglb, p, G, C, a, b, c);
-  const int cell = a + C.ncx * (b + C.ncy * c);
+  const int cell = cell_of(x, G.nx, C.ncx) + C.ncx * (cell_of(y, G.ny, C.ncy) + C.ncy * cell_of(z, G.nz, C.ncz));
   const int slot = atomicAdd(&C.cnt[cell], 1);
   if (slot < kCellCap)
     C.list[cell * kCellCap + slot] = p;
   else
     atomicAdd(&status[ST_CELL_OVERFLOW], 1);
+}
+
+__global__ void __launch_bounds__(256)
+    k_cell_build(const double* __restrict__ ypglb, int np, PGeom G, CellArgs C,
+                 int32_t* __restrict__ status) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < np) cell_insert(p, ypglb[3 * p], ypglb[3 * p + 1], ypglb[3 * p + 2], G, C, status);
 }
 
 // Overlap test of ovlpchk (partlib.f90:118-171) for the pair (p, q), q > p.
@@ -721,60 +723,79 @@ __device__ __forceinline__ bool lub_pair(const double* __restrict__ ypglb, int a
   return true;
 }
 
-// beads_lubforce of particle a from the cells: partners in the 27 cells
-// around it, summed in increasing id (a fixed order); then the walls.  One
-// pass over the cells lists the partners in range, sorted and each once (a
-// cell grid of fewer than 3 cells on an axis meets a cell twice); only a
-// sphere with more than kLubList partners falls back to finding each next
-// id by a further pass.
-constexpr int kLubList = 32;
+// beads_lubforce of particle a from the cells, by one wavefront: every lane
+// tests one (cell, slot) of the 27 cells around a at a time (at least three
+// cells on every axis: no partner is met twice), the partners in range are
+// listed in LDS with their pair forces, ranked by id and summed in increasing
+// id (a fixed order); then the walls.  Bound: three dependent loads (cell
+// count, slot, position).  One thread per particle, walking its cells serially,
+// took 39 us of a step with 900 spheres, this takes 9 us.  A sphere with more
+// than kLubList partners falls back to lane 0 finding each next id by a
+// further pass over the cells.  Called by every wavefront of a workgroup, with
+// lub_lds bytes of dynamic LDS (static LDS would cost the workgroups of boxes
+// without cells 2 us).
+constexpr int kLubList = 128;
+struct LubList {
+  int32_t id[kLubList];
+  double f[kLubList][3];
+  double sorted[kLubList][3];
+};
 __device__ void lub_cells(int a, const double* __restrict__ ypglb, int np, const PGeom& G,
-                          const LubArgs& L, int32_t* __restrict__ status) {
-  if (a >= np) return;
+                          const LubArgs& L, LubList& W) {
   const CellArgs& C = L.cells;
   const double dist0 = 2.0 * G.rad + L.mingap;
   const double pre = (dist0 + 1e-6) * (dist0 + 1e-6);
-  int ca, cb, cc;
-  cell_coords(ypglb, a, G, C, ca, cb, cc);
-  double sx = 0.0, sy = 0.0, sz = 0.0;
-  int ids[kLubList];
-  int m = 0;
-  bool full = false;
-  for (int k = 0; k < 27; ++k) {
-    const int cell = cell_neighbour(C, G, ca, cb, cc, k);
-    if (cell < 0) continue;
-    const int n = min(C.cnt[cell], kCellCap);
-    for (int e = 0; e < n; ++e) {
-      const int b = C.list[cell * kCellCap + e];
-      if (b == a) continue;
-      double fx, fy, fz;
-      if (!lub_pair(ypglb, a, b, G, L, pre, fx, fy, fz)) continue;
-      int pos = m;
-      while (pos > 0 && ids[pos - 1] > b) --pos;
-      if (pos > 0 && ids[pos - 1] == b) continue;   // met through a repeated cell
-      if (m == kLubList) {
-        full = true;
-        continue;
+  const int lane = threadIdx.x & 63;
+  int ca = 0, cb = 0, cc = 0;
+  const bool on = a < np;
+  if (on) cell_coords(ypglb, a, G, C, ca, cb, cc);
+  int m = 0;   // partners so far (the same in every lane)
+  for (int k0 = 0; k0 < 27 * kCellCap && on; k0 += 64) {
+    const int k = (k0 + lane) / kCellCap, e = (k0 + lane) % kCellCap;
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    int b = -1;
+    bool in = false;
+    if (k < 27) {
+      const int cell = cell_neighbour(C, G, ca, cb, cc, k);
+      if (cell >= 0 && e < min(C.cnt[cell], kCellCap)) {
+        b = C.list[cell * kCellCap + e];
+        in = b != a && lub_pair(ypglb, a, b, G, L, pre, fx, fy, fz);
       }
-      for (int i = m; i > pos; --i) ids[i] = ids[i - 1];
-      ids[pos] = b;
-      ++m;
+    }
+    const uint64_t bal = __ballot(in);
+    const int at = m + __popcll(bal & ((1ull << lane) - 1ull));
+    if (in && at < kLubList) {
+      W.id[at] = b;
+      W.f[at][0] = fx;
+      W.f[at][1] = fy;
+      W.f[at][2] = fz;
+    }
+    m += __popcll(bal);
+  }
+  const bool full = m > kLubList;
+  __syncthreads();
+  if (on && !full) {
+    for (int i = lane; i < m; i += 64) {
+      const int b = W.id[i];
+      int rank = 0;
+      for (int j = 0; j < m; ++j) rank += W.id[j] < b;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) W.sorted[rank][c] = W.f[i][c];
     }
   }
+  __syncthreads();
+  if (!on) return;
   if (!full) {
-    for (int i = 0; i < m; ++i) {
-      double fx, fy, fz;
-      lub_pair(ypglb, a, ids[i], G, L, pre, fx, fy, fz);
-      sx += fx;
-      sy += fy;
-      sz += fz;
+    if (lane < 3) {
+      double s = 0.0;
+      for (int i = 0; i < m; ++i) s += W.sorted[i][lane];
+      if (lane == 1 && G.walls_y) s += wall_lub(ypglb[3 * a + 1], G, L);
+      L.flubp[3 * a + lane] = s;
     }
-    if (G.walls_y) sy += wall_lub(ypglb[3 * a + 1], G, L);
-    L.flubp[3 * a] = sx;
-    L.flubp[3 * a + 1] = sy;
-    L.flubp[3 * a + 2] = sz;
     return;
   }
+  if (lane != 0) return;
+  double sx = 0.0, sy = 0.0, sz = 0.0;
   int last = -1;
   for (int guard = 0; guard < 27 * kCellCap; ++guard) {
     int next = 0x7fffffff;
@@ -805,9 +826,11 @@ __device__ void lub_cells(int a, const double* __restrict__ ypglb, int np, const
 
 __global__ void __launch_bounds__(PB)
     k_lubforce(const double* __restrict__ ypglb, int np, PGeom G, LubArgs L, int32_t* __restrict__ status) {
-  if (L.cells.cnt)
-    lub_cells((int)(blockIdx.x * PB + threadIdx.x), ypglb, np, G, L, status);
-  else if ((int)blockIdx.x < np)
+  if (L.cells.cnt) {
+    extern __shared__ double lds_f64[];
+    lub_cells((int)(blockIdx.x * (PB / 64) + (threadIdx.x >> 6)), ypglb, np, G, L,
+              ((LubList*)lds_f64)[threadIdx.x >> 6]);
+  } else if ((int)blockIdx.x < np)
     lub_block(blockIdx.x, ypglb, np, G, L);
 }
 
@@ -1016,10 +1039,13 @@ template <typename T>
 __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
   if (b_ >= a.nct) {
     const int r = b_ - a.nct;
-    if (a.lub.cells.cnt)
-      lub_cells(r * PB + (int)threadIdx.x, a.ypglb, a.np, a.G, a.lub, a.status);
-    else
+    if (a.lub.cells.cnt) {
+      extern __shared__ double lds_f64[];
+      lub_cells(r * (PB / 64) + (int)(threadIdx.x >> 6), a.ypglb, a.np, a.G, a.lub,
+                ((LubList*)lds_f64)[threadIdx.x >> 6]);
+    } else {
       lub_block(r, a.ypglb, a.np, a.G, a.lub);
+    }
     return;
   }
   if (a.ref_order) {
@@ -1050,7 +1076,8 @@ __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
 // the opposite population of the solid neighbour x + c (partlib.f90:1605-1621),
 // and the unit's momentum-exchange force and torque (FP64, fixed reduction
 // order) into seg_ft.  Blocks past the units (fused step) reset one segment
-// of the map buffer the coming beads_links rebuilds (built two steps ago).
+// of the map buffer the coming beads_links rebuilds (built two steps ago), and
+// blocks past those the counts of the pair-search cells.
 template <typename T>
 __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   __shared__ double red[6][PB / 64];
@@ -1059,7 +1086,12 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   const int u = b_;
   const int nunits = a.nsegs * a.split;
   if (u >= nunits) {
-    clear_segment(u - nunits, a.nseg, a.seg_cap, a.clr_list, a.clr_cnt, a.clr_isn, a.clr_mask);
+    if (u - nunits < a.nclr) {
+      clear_segment(u - nunits, a.nseg, a.seg_cap, a.clr_list, a.clr_cnt, a.clr_isn, a.clr_mask);
+    } else {   // the pair-search cells the coming move fills (the pre-pass has read them)
+      const int i = (u - nunits - a.nclr) * PB + (int)threadIdx.x;
+      if (i < a.ncell) a.lub.cells.cnt[i] = 0;
+    }
     return;
   }
   const int b = u / a.split, h = u - b * a.split;
@@ -1180,117 +1212,108 @@ __device__ __forceinline__ bool wrap_particle(double* yp, double* ypglb, double*
   return bad;
 }
 
-// beads_move (partlib.f90:2295-2394): second-order Newton-Euler update.  With
-// `wrap` set the periodic wrap of beads_redistribute (partlib.f90:2600-2626)
-// follows in the same thread; with seg_ft set the hydrodynamic force and
-// torque are first summed from the bounce-back segments (and stored).  Every
-// input is loaded before the first store (the argument arrays are distinct,
-// but the compiler cannot know it).
+// beads_move (partlib.f90:2295-2394): second-order Newton-Euler update, one
+// component per lane, the lanes of a particle in a quad (the fourth idles).
+// With `wrap` set the periodic wrap of beads_redistribute
+// (partlib.f90:2600-2626) follows in the same lane; with seg_ft set the
+// hydrodynamic force and torque are first summed from the bounce-back segments
+// (and stored), in unit order; with cells.cnt set the particle enters its
+// pair-search cell.  Every input is loaded before the first store (the
+// argument arrays are distinct, but the compiler cannot know it).  Bound: the
+// latency of one round of loads and stores over few lanes; one thread per
+// particle with all components took 8.7-10.8 us
+// (300 to 900 spheres), this takes 5.0.
+constexpr int kMoveBlock = 64;
 __device__ __forceinline__ void move_body(int b_, MoveArgs m, int np, int first, int wrap, PGeom G,
                                           int32_t* __restrict__ status,
-                                          const double* __restrict__ seg_ft, int nseg) {
-  const int p = b_ * blockDim.x + threadIdx.x;
-  if (p >= np) return;
+                                          const double* __restrict__ seg_ft, int nseg, CellArgs cells) {
+  const int t = b_ * kMoveBlock + (int)threadIdx.x;
+  const int p = t >> 2, c = t & 3;
+  const bool on = p < np && c < 3;
   const double dt = 1.0;
-  const double bf[3] = {m.bfx, m.bfy, m.bfz};
-  const double pf[3] = {m.pfx, m.pfy, m.pfz};
-  double yp[3], wp[3], omgp[3], fhi[3], flub[3], torq[3], fpp[3], tpp[3], dwdt[3], domgdt[3], th[3];
-  double yg[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const int q = 3 * p + c;
-    yp[c] = m.yp[q];
-    yg[c] = m.ypglb[q];
-    wp[c] = m.wp[q];
-    omgp[c] = m.omgp[q];
-    if (!seg_ft) {
-      fhi[c] = m.fHIp[q];
-      torq[c] = m.torqp[q];
+  const int q = on ? 3 * p + c : 0;
+  bool fast = false, bad = false;
+  double yg = 0.0;
+  if (on) {
+    const double bf = c == 0 ? m.bfx : (c == 1 ? m.bfy : m.bfz);
+    const double pf = c == 0 ? m.pfx : (c == 1 ? m.pfy : m.pfz);
+    double yp = m.yp[q], wp = m.wp[q], omgp = m.omgp[q], fpp = m.forcepp[q], tpp = m.torqpp[q];
+    double dwdt = m.dwdt[q], domgdt = m.domgdt[q];
+    const double flub = m.flubp[q];
+    double th = first ? 0.0 : m.thetap[q];
+    yg = m.ypglb[q];
+    double fhi, torq;
+    if (seg_ft) {
+      fhi = torq = 0.0;
+#pragma unroll 8
+      for (int s = 0; s < nseg; ++s) {
+        fhi += seg_ft[6ll * ((int64_t)p * nseg + s) + c];
+        torq += seg_ft[6ll * ((int64_t)p * nseg + s) + 3 + c];
+      }
+    } else {
+      fhi = m.fHIp[q];
+      torq = m.torqp[q];
     }
-    flub[c] = m.flubp[q];
-    fpp[c] = m.forcepp[q];
-    tpp[c] = m.torqpp[q];
-    dwdt[c] = m.dwdt[q];
-    domgdt[c] = m.domgdt[q];
-    th[c] = first ? 0.0 : m.thetap[q];
-  }
-  if (seg_ft) seg_sum(seg_ft, nseg, p, fhi, torq);
-  double wpp[3], omgpp[3], fp[3], dwn[3], don[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    wpp[c] = wp[c];
-    omgpp[c] = omgp[c];
-    double F = fhi[c] + flub[c];
+    const double wpp = wp, omgpp = omgp;
+    double F = fhi + flub;
     if (c == 1) F = F - m.volp * m.rhog;
-    if (bf[c] != 0.0) F = F + m.volp * bf[c];
-    if (pf[c] != 0.0) F = F + m.volp * pf[c];
-    fp[c] = F;
-    if (first) fpp[c] = F;
-    dwn[c] = 0.5 * (F + fpp[c]) / m.amp;
-    if (first) dwdt[c] = dwn[c];
-    wp[c] = wpp[c] + 0.5 * dt * (dwdt[c] + dwn[c]);
-  }
-  bool fast = false;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const double d = 0.5 * dt * (wp[c] + wpp[c]);
-    yp[c] = yp[c] + d;
-    fast = fast || !(fabs(d) < 1.0);
-  }
-  // the overlapped step assumes a centre moves less than one node per step
-  if (fast) atomicAdd(&status[ST_FAST], 1);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    if (first) tpp[c] = torq[c];
-    don[c] = 0.5 * (torq[c] + tpp[c]) / m.aip;
-    if (first) domgdt[c] = don[c];
-    omgp[c] = omgpp[c] + 0.5 * dt * (domgdt[c] + don[c]);
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) th[c] = th[c] + 0.5 * dt * (omgp[c] + omgpp[c]);
-  bool bad = false;
-  double ygp[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    ygp[c] = yg[c];
+    if (bf != 0.0) F = F + m.volp * bf;
+    if (pf != 0.0) F = F + m.volp * pf;
+    if (first) fpp = F;
+    const double dwn = 0.5 * (F + fpp) / m.amp;
+    if (first) dwdt = dwn;
+    wp = wpp + 0.5 * dt * (dwdt + dwn);
+    const double d = 0.5 * dt * (wp + wpp);
+    yp = yp + d;
+    // the overlapped step assumes a centre moves less than one node per step
+    fast = !(fabs(d) < 1.0);
+    if (first) tpp = torq;
+    const double don = 0.5 * (torq + tpp) / m.aip;
+    if (first) domgdt = don;
+    omgp = omgpp + 0.5 * dt * (domgdt + don);
+    th = th + 0.5 * dt * (omgp + omgpp);
+    const double ygp = yg;
     if (wrap) {
       // beads_redistribute: wrap into the periodic box (not across a wall),
       // ypglbp <- ypglb, ypglb <- yp
       const int n = c == 0 ? G.nx : (c == 1 ? G.ny : G.nz);
-      const double v = yp[c], N = (double)n;
+      const double v = yp, N = (double)n;
       if (!(G.walls_y && c == 1)) {
-        if (v >= N) yp[c] = yp[c] - N;
-        if (v < 0.0) yp[c] = yp[c] + N;
+        if (v >= N) yp = yp - N;
+        if (v < 0.0) yp = yp + N;
       }
-      if (!sane_coord(yp[c], n)) bad = true;
-      ygp[c] = yg[c];
-      yg[c] = yp[c];
+      bad = !sane_coord(yp, n);
+      yg = yp;
     }
-  }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const int q = 3 * p + c;
-    m.wpp[q] = wpp[c];
-    m.omgpp[q] = omgpp[c];
-    m.forcep[q] = fp[c];
-    m.wp[q] = wp[c];
-    m.yp[q] = yp[c];
-    m.omgp[q] = omgp[c];
-    m.thetap[q] = th[c];
-    m.dwdt[q] = dwn[c];
-    m.domgdt[q] = don[c];
-    m.forcepp[q] = fp[c];
-    m.torqpp[q] = torq[c];
+    m.wpp[q] = wpp;
+    m.omgpp[q] = omgpp;
+    m.forcep[q] = F;
+    m.wp[q] = wp;
+    m.yp[q] = yp;
+    m.omgp[q] = omgp;
+    m.thetap[q] = th;
+    m.dwdt[q] = dwn;
+    m.domgdt[q] = don;
+    m.forcepp[q] = F;
+    m.torqpp[q] = torq;
     if (seg_ft) {
-      m.fHIp[q] = fhi[c];
-      m.torqp[q] = torq[c];
+      m.fHIp[q] = fhi;
+      m.torqp[q] = torq;
     }
     if (wrap) {
-      m.ypglbp[q] = ygp[c];
-      m.ypglb[q] = yg[c];
+      m.ypglbp[q] = ygp;
+      m.ypglb[q] = yg;
     }
   }
-  if (bad) atomicAdd(&status[ST_NONFINITE], 1);
+  // once per particle: the quad's first lane speaks for it
+  const int lane = (int)threadIdx.x & 63;
+  const uint64_t quad = 7ull << (lane & ~3);
+  const uint64_t fastm = __ballot(fast), badm = __ballot(bad);
+  const double y1 = __shfl(yg, lane | 1, 64), y2 = __shfl(yg, lane | 2, 64);
+  if (!on || c != 0) return;
+  if (fastm & quad) atomicAdd(&status[ST_FAST], 1);
+  if (badm & quad) atomicAdd(&status[ST_NONFINITE], 1);
+  if (cells.cnt) cell_insert(p, yg, y1, y2, G, cells, status);
 }
 
 // beads_redistribute, one-rank content (partlib.f90:2600-2626): periodic wrap,
@@ -1621,14 +1644,14 @@ __global__ void __launch_bounds__(PB)
   bounce_back_body<T>((int)blockIdx.x - off[c], a);
 }
 
-__global__ void __launch_bounds__(256) k_move(MoveKArgs a) {
-  move_body((int)blockIdx.x, a.m, a.np, a.first, a.wrap, a.G, a.status, a.seg_ft, a.nseg);
+__global__ void __launch_bounds__(kMoveBlock) k_move(MoveKArgs a) {
+  move_body((int)blockIdx.x, a.m, a.np, a.first, a.wrap, a.G, a.status, a.seg_ft, a.nseg, a.cells);
 }
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kMoveBlock)
     kb_move(const MoveKArgs* __restrict__ t, const int* __restrict__ off, int nc) {
   const int c = case_of(off, nc, (int)blockIdx.x);
   const MoveKArgs a = t[c];
-  move_body((int)blockIdx.x - off[c], a.m, a.np, a.first, a.wrap, a.G, a.status, a.seg_ft, a.nseg);
+  move_body((int)blockIdx.x - off[c], a.m, a.np, a.first, a.wrap, a.G, a.status, a.seg_ft, a.nseg, a.cells);
 }
 
 // 4 waves per SIMD (at most 128 VGPRs): with the 1024 blocks of the grid
@@ -1795,10 +1818,12 @@ static CellArgs cell_args(const Ctx& c) {
   return C;
 }
 
+static size_t lub_lds(const Ctx& c) { return cell_args(c).cnt ? sizeof(LubList) * (PB / 64) : 0; }
+
 // Blocks of the lubrication part of a grid: one per particle (all pairs) or
-// one thread per particle (cells).
+// one wavefront per particle (cells).
 static int lub_blocks(const Ctx& c) {
-  return cell_args(c).cnt ? (c.pt.np + PB - 1) / PB : c.pt.np;
+  return cell_args(c).cnt ? (c.pt.np + PB / 64 - 1) / (PB / 64) : c.pt.np;
 }
 
 hipError_t ensure_cells(Ctx& c) {
@@ -1888,7 +1913,11 @@ BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blo
   a.seg_cap = P.seg_cap;
   a.clr_list = P.sol_list[t]; a.clr_cnt = P.sol_cnt[t]; a.clr_isn = P.isn[t]; a.clr_mask = P.mask[t];
   if (nclr) P.map_np[t] = 0;
-  *bb_blocks = a.nsegs * a.split + nclr;
+  a.nclr = nclr;
+  a.ncell = fused && a.lub.cells.cnt ? P.cell_n[0] * P.cell_n[1] * P.cell_n[2] : 0;
+  P.cells_zeroed = a.ncell > 0;
+  if (a.ncell) P.cells_ok = false;
+  *bb_blocks = a.nsegs * a.split + nclr + (a.ncell + PB - 1) / PB;
   *pre_blocks = a.nct + a.nlub;
   return a;
 }
@@ -1907,7 +1936,12 @@ MoveKArgs move_args(Ctx& c, int first, int wrap, bool from_seg, int* blocks) {
   m.pfx = c.p.particle_force[0]; m.pfy = c.p.particle_force[1]; m.pfz = c.p.particle_force[2];
   a.np = P.np; a.first = first; a.wrap = wrap; a.G = pgeom(c); a.status = c.d_status;
   a.seg_ft = from_seg ? P.seg_ft : nullptr; a.nseg = P.nseg * P.bb_split;
-  *blocks = (P.np + 255) / 256;
+  // the cells the fused bounce-back grid has cleared: filled at the new centres
+  const bool fill = wrap && from_seg && P.cells_zeroed;
+  a.cells = fill ? cell_args(c) : CellArgs{};
+  P.cells_zeroed = false;
+  if (wrap) P.cells_ok = fill;   // the wrapped positions are the new ypglb
+  *blocks = (4 * P.np + kMoveBlock - 1) / kMoveBlock;
   return a;
 }
 
@@ -2113,11 +2147,12 @@ hipError_t launch_bounce_back(Ctx& c, bool fused) {
   }
   int nb = 0, npre = 0;
   const BounceArgs ba = bounce_args(c, fused, kContactBlocks, &nb, &npre);
+  const size_t lds = fused ? lub_lds(c) : 0;
   if (c.prec == MFC_PREC_FP64) {
-    hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), lds, c.stream, ba);
     hipLaunchKernelGGL(k_bounce_back<double>, dim3(nb), dim3(PB), 0, c.stream, ba);
   } else {
-    hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), lds, c.stream, ba);
     hipLaunchKernelGGL(k_bounce_back<float>, dim3(nb), dim3(PB), 0, c.stream, ba);
   }
   if (!fused)
@@ -2130,7 +2165,7 @@ hipError_t launch_lubforce(Ctx& c) {
   Particles& P = c.pt;
   const hipError_t e = ensure_cells(c);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_lubforce, dim3(lub_blocks(c)), dim3(PB), 0, c.stream, P.ypglb, P.np, pgeom(c),
+  hipLaunchKernelGGL(k_lubforce, dim3(lub_blocks(c)), dim3(PB), lub_lds(c), c.stream, P.ypglb, P.np, pgeom(c),
                      lub_args(c), c.d_status);
   return hipGetLastError();
 }
@@ -2138,8 +2173,7 @@ hipError_t launch_lubforce(Ctx& c) {
 hipError_t launch_move(Ctx& c, int first, int wrap, bool from_seg) {
   int nb = 0;
   const MoveKArgs a = move_args(c, first, wrap, from_seg, &nb);
-  hipLaunchKernelGGL(k_move, dim3(nb), dim3(256), 0, c.stream, a);
-  if (wrap) c.pt.cells_ok = false;   // the wrapped positions are the new ypglb
+  hipLaunchKernelGGL(k_move, dim3(nb), dim3(kMoveBlock), 0, c.stream, a);
   return hipGetLastError();
 }
 
@@ -2242,7 +2276,7 @@ hipError_t launch_batched(Stage st, int prec, int walls, const void* t, const in
         hipLaunchKernelGGL(kb_bb_contact<float>, dim3(blocks), dim3(PB), 0, s, (const BounceArgs*)t, off, nc);
       break;
     case SG_MOVE:
-      hipLaunchKernelGGL(kb_move, dim3(blocks), dim3(256), 0, s, (const MoveKArgs*)t, off, nc);
+      hipLaunchKernelGGL(kb_move, dim3(blocks), dim3(kMoveBlock), 0, s, (const MoveKArgs*)t, off, nc);
       break;
     case SG_SCAN:
       hipLaunchKernelGGL(kb_links_scan, dim3(blocks), dim3(PB), lds, s, (const ScanArgs*)t, off, nc);

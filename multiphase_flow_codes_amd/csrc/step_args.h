@@ -168,6 +168,8 @@ struct BounceArgs {
   const int32_t* clr_cnt;
   int32_t* clr_isn;
   uint32_t* clr_mask;
+  int nclr;                     // blocks of the map clearing, then of the cells'
+  int ncell;                    // pair-search cells to clear (0: none)
 };
 
 struct MoveKArgs {
@@ -179,6 +181,7 @@ struct MoveKArgs {
   int32_t* status;
   const double* seg_ft;   // non-null: fHIp / torqp are first summed from the segments
   int nseg;
+  CellArgs cells;         // cnt non-null: (cleared) cells to enter the new centres in
 };
 
 struct FillApplyArgs {
