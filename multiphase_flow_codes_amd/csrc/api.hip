@@ -354,6 +354,8 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   c.g.ny = p->ny;
   c.g.nz = p->nz;
   c.g.walls_y = p->walls_y ? 1 : 0;
+  c.g.dx = fast_div((uint32_t)p->nx);
+  c.g.dy = fast_div((uint32_t)p->ny);
   c.g.ncell = ncell;
   c.g.pitch = ncell;
   // in-place storage starts with the streamed field in each node's own slots

@@ -206,7 +206,7 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t per) {
 
 // The tiles of a lattice, `waves` per workgroup, numbered x fastest.
 struct TileGrid {
-  FastDiv tpr, ny;    // tiles per row, rows per plane
+  FastDiv tpr;        // tiles per row
   uint32_t ntiles, per, waves;
 };
 
@@ -226,8 +226,8 @@ __global__ void __launch_bounds__(256)
   const uint32_t row = div_by(t, g.tpr);
   const int x = (int)((t - row * g.tpr.d) * (uint32_t)kTileX + (threadIdx.x & 63u));
   if (x >= a.g.nx) return;
-  const uint32_t z = div_by(row, g.ny);
-  collide_node<T, R, ARR, WALLS, LAY, NTL, NTS>(a, x, (int)(row - z * g.ny.d), (int)z);
+  const uint32_t z = div_by(row, a.g.dy);
+  collide_node<T, R, ARR, WALLS, LAY, NTL, NTS>(a, x, (int)(row - z * a.g.dy.d), (int)z);
 }
 
 // The collide of the tiles of a list (overlapped step): one tile per
@@ -283,13 +283,13 @@ __global__ void __launch_bounds__(BS)
   const CollideArgs a = t[c];
   const uint64_t n = (uint64_t)((int)b - off[c]) * BS + threadIdx.x;
   if (n >= a.g.ncell) return;
-  const uint32_t nx = (uint32_t)a.g.nx, ny = (uint32_t)a.g.ny;
-  const uint32_t x = (uint32_t)(n % nx);
-  const uint32_t r = (uint32_t)(n / nx);
+  int x, y, z;
+  uint32_t row;
+  node_coords((uint32_t)n, a.g, x, y, z, row);
   if (ARR_ANY && a.arr)
-    collide_node<T, R, true, WALLS, LAY_AB, true, true>(a, (int)x, (int)(r % ny), (int)(r / ny));
+    collide_node<T, R, true, WALLS, LAY_AB, true, true>(a, x, y, z);
   else
-    collide_node<T, R, false, WALLS, LAY_AB, true, true>(a, (int)x, (int)(r % ny), (int)(r / ny));
+    collide_node<T, R, false, WALLS, LAY_AB, true, true>(a, x, y, z);
 }
 
 // Forcing table of one step (force_table.h): one thread per (row, component).
@@ -563,7 +563,6 @@ static CollideShape collide_shape(const Ctx& c, bool spheres) {
   CollideShape s;
   const uint32_t tpr = (uint32_t)((c.g.nx + kTileX - 1) / kTileX);
   s.t.tpr = fast_div(tpr);
-  s.t.ny = fast_div((uint32_t)c.g.ny);
   s.t.ntiles = tpr * (uint32_t)c.g.ny * (uint32_t)c.g.nz;
   s.t.waves = s.t.ntiles <= 4096 ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
   s.block = (unsigned)kTileX * s.t.waves;

@@ -13,9 +13,9 @@ namespace mfc {
 
 __device__ __forceinline__ void node_coords(uint32_t n, const Grid& g, int& x, int& y, int& z,
                                             uint32_t& row) {
-  row = n / (uint32_t)g.nx;
+  row = div_by(n, g.dx);
   x = (int)(n - row * (uint32_t)g.nx);
-  const uint32_t zz = row / (uint32_t)g.ny;
+  const uint32_t zz = div_by(row, g.dy);
   y = (int)(row - zz * (uint32_t)g.ny);
   z = (int)zz;
 }

@@ -101,6 +101,7 @@ struct Grid {
   // rows of one (y, z) side by side).
   uint64_t pitch;     // elements from one population plane to the next
   uint64_t rs;        // elements from one row of a plane to the next row
+  FastDiv dx, dy;     // division by nx and ny
 };
 
 MFC_HD int wrapi(int a, int n) {

@@ -451,7 +451,7 @@ __device__ __forceinline__ void links_scan_body(int b_, const double* __restrict
   __shared__ int wt[2][PB / 64][2];
   __shared__ int sh[PB / 64];
   const int b = b_;
-  const int p = b / nseg, s = b - p * nseg;
+  const int p = (int)div_by((uint32_t)b, G.dseg), s = b - p * nseg;
   if (p >= np) return;
   if (ovl && s == 0) {
     // ovlpchk: flag p if any later particle is closer than 2r
@@ -496,9 +496,9 @@ __device__ __forceinline__ void links_scan_body(int b_, const double* __restrict
     const int e = e0 + (int)threadIdx.x;
     if (e < nsh) {
       const uint32_t n = shell[e];
-      const int iw = (int)(n % (uint32_t)G.nx);
-      const uint32_t rw = n / (uint32_t)G.nx;
-      const int jw = (int)(rw % (uint32_t)G.ny), kw = (int)(rw / (uint32_t)G.ny);
+      const uint32_t rw = div_by(n, G.dx);
+      const int iw = (int)(n - rw * (uint32_t)G.nx);
+      const int kw = (int)div_by(rw, G.dy), jw = (int)rw - kw * G.ny;
       LinkGeom L;
       node_geom(B, G, iw, jw, kw, L);
       uint32_t hits = 0;
@@ -585,7 +585,7 @@ __device__ __forceinline__ void links_expand_body(int b_, const double* __restri
     fill_find_segment(b - nsegs, fa, nseg, status);
     return;
   }
-  const int p = b / nseg;
+  const int p = (int)div_by((uint32_t)b, G.dseg);
   if (p >= np) return;
   box_info(ypglb, p, G, B);
   if (!B.ok) return;
@@ -618,9 +618,9 @@ __device__ __forceinline__ void links_expand_body(int b_, const double* __restri
   for (int64_t l = a + threadIdx.x; l < e; l += PB) {
     const uint32_t n = lk_node[l];
     const int q = lk_dir[l];
-    const int iw = (int)(n % (uint32_t)G.nx);
-    const uint32_t rw = n / (uint32_t)G.nx;
-    const int jw = (int)(rw % (uint32_t)G.ny), kw = (int)(rw / (uint32_t)G.ny);
+    const uint32_t rw = div_by(n, G.dx);
+    const int iw = (int)(n - rw * (uint32_t)G.nx);
+    const int kw = (int)div_by(rw, G.dy), jw = (int)rw - kw * G.ny;
     LinkGeom L;
     node_geom(B, G, iw, jw, kw, L);
     double xx1, yy1, zz1, rr1;
@@ -1094,8 +1094,8 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
     }
     return;
   }
-  const int b = u / a.split, h = u - b * a.split;
-  const int p = b / a.nseg;
+  const int b = a.split == 1 ? u : u / a.split, h = u - b * a.split;
+  const int p = (int)div_by((uint32_t)b, a.G.dseg);
   const int64_t s0 = a.off[b], s1 = min(a.off[b + 1], a.cap);
   const int64_t per = (max(s1 - s0, (int64_t)0) + a.split - 1) / a.split;
   const int64_t l0 = s0 + h * per;
@@ -1740,6 +1740,9 @@ static PGeom pgeom(const Ctx& c) {
   G.rlink2 = (c.p.rad + 1.5) * (c.p.rad + 1.5);
   G.rsolid2 = (c.p.rad + 0.5) * (c.p.rad + 0.5);
   G.slab = c.pt.slab;
+  G.dx = c.g.dx;
+  G.dy = c.g.dy;
+  G.dseg = fast_div((uint32_t)c.pt.nseg);
   return G;
 }
 

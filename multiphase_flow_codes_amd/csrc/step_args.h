@@ -36,6 +36,7 @@ struct PGeom {
   double rsolid2;
   // z planes per segment (4 or 8; Particles::slab)
   int slab;
+  FastDiv dx, dy, dseg;   // division by nx, ny and the segments per particle
 };
 
 struct FillArgs {
