@@ -32,6 +32,7 @@ SOURCES = {
     "diag.hip": [],
     "ensemble.hip": [],
     "initial.hip": [],
+    "hostcopy.hip": [],
 }
 
 

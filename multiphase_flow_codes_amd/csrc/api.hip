@@ -293,8 +293,8 @@ bool particles_on(const Ctx& c) { return c.pt.np > 0; }
 
 int check_faults(mfc_ctx* ctx) {
   Ctx& c = ctx->c;
-  HIPCHK(hipMemcpyAsync(c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part = {c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT};
+  HIPCHK(copy_to_host(c, &part, 1));
   const int32_t* s = c.h_status;
   char buf[256];
   if (s[ST_OVERLAP] > 0) {
@@ -452,9 +452,16 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   CK(hipMemsetAsync(c.d_status, 0, sizeof(int32_t) * ST_COUNT, c.stream));
   CK(hipHostMalloc((void**)&c.h_status, sizeof(int32_t) * ST_COUNT, hipHostMallocDefault));
   CK(hipMalloc(&c.d_red, sizeof(double) * (size_t)rhoupdat_blocks(c)));
-  CK(hipHostMalloc((void**)&c.h_red, sizeof(double) * 8, hipHostMallocDefault));
+  CK(hipHostMalloc((void**)&c.h_red, sizeof(double) * 8, hipHostMallocCoherent));
+  memset(c.h_red, 0, sizeof(double) * 8);
   // this device's static scratch of the allocation-free sums
   CK(sums_scratch(&c.sums_scratch));
+  int dev = -1;
+  CK(hipGetDevice(&dev));
+  if (dev >= 0 && dev < kMaxDevices) {
+    host_pipe_ref(dev);
+    c.pipe_dev = dev;
+  }
   CK(hipStreamSynchronize(c.stream));
 #undef CK
   *out = ctx;
@@ -496,6 +503,7 @@ int mfc_destroy(mfc_ctx* ctx) {
     if (c.ev_bb) (void)hipEventDestroy(c.ev_bb);
     if (c.pstream) (void)hipStreamDestroy(c.pstream);
   }
+  if (c.pipe_dev >= 0) host_pipe_unref(c.pipe_dev);
   if (c.h_status) (void)hipHostFree(c.h_status);
   if (c.h_red) (void)hipHostFree(c.h_red);
   for (auto e : c.tpool) (void)hipEventDestroy(e);
@@ -516,8 +524,8 @@ int mfc_status(mfc_ctx* ctx, int32_t* out16) {
   NEEDCTX;
   if (!out16) return MFC_ERR_ARG;
   Ctx& c = ctx->c;
-  HIPCHK(hipMemcpyAsync(c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part = {c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT};
+  HIPCHK(copy_to_host(c, &part, 1));
   memcpy(out16, c.h_status, sizeof(int32_t) * ST_COUNT);
   return MFC_OK;
 }
@@ -564,8 +572,8 @@ int mfc_download_f(mfc_ctx* ctx, double* f) {
   for (int z0 = 0; z0 < c.g.nz; z0 += ns) {
     const int nz = std::min(ns, c.g.nz - z0);
     HIPCHK(launch_pop_to_aos(c, (double*)c.staging, z0, nz, c.phase == PHASE_POST_STREAM));
-    HIPCHK(hipMemcpyAsync(f + plane * z0, c.staging, plane * nz * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    HIPCHK(hipStreamSynchronize(c.stream));
+    const HostPart part = {f + plane * z0, c.staging, plane * nz * sizeof(double)};
+    HIPCHK(copy_to_host(c, &part, 1));
   }
   return MFC_OK;
 }
@@ -595,11 +603,13 @@ int mfc_download_macro(mfc_ctx* ctx, double* rho, double* ux, double* uy, double
   int rc = need_arrays(ctx);
   if (rc) return rc;
   const size_t b = sizeof(double) * c.g.ncell;
-  if (rho) HIPCHK(hipMemcpyAsync(rho, c.rho, b, hipMemcpyDeviceToHost, c.stream));
-  if (ux) HIPCHK(hipMemcpyAsync(ux, c.ux, b, hipMemcpyDeviceToHost, c.stream));
-  if (uy) HIPCHK(hipMemcpyAsync(uy, c.uy, b, hipMemcpyDeviceToHost, c.stream));
-  if (uz) HIPCHK(hipMemcpyAsync(uz, c.uz, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  HostPart part[4];
+  int n = 0;
+  double* host[4] = {rho, ux, uy, uz};
+  const double* dev[4] = {c.rho, c.ux, c.uy, c.uz};
+  for (int k = 0; k < 4; ++k)
+    if (host[k]) part[n++] = {host[k], dev[k], b};
+  HIPCHK(copy_to_host(c, part, n));
   return MFC_OK;
 }
 
@@ -612,10 +622,8 @@ int mfc_download_force(mfc_ctx* ctx, double* fx, double* fy, double* fz) {
   if (rc) return rc;
   double* s = (double*)c.staging;
   HIPCHK(launch_force_field(c, c.ft.cur, s, s + c.g.ncell, s + 2 * c.g.ncell));
-  HIPCHK(hipMemcpyAsync(fx, s, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipMemcpyAsync(fy, s + c.g.ncell, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipMemcpyAsync(fz, s + 2 * c.g.ncell, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part[3] = {{fx, s, b}, {fy, s + c.g.ncell, b}, {fz, s + 2 * c.g.ncell, b}};
+  HIPCHK(copy_to_host(c, part, 3));
   return MFC_OK;
 }
 
@@ -741,10 +749,10 @@ int mfc_rhoupdat(mfc_ctx* ctx, double* maxdiff) {
   Ctx& c = ctx->c;
   int rc = need_arrays(ctx);
   if (rc) return rc;
-  HIPCHK(launch_rhoupdat(c, c.phase == PHASE_POST_STREAM, c.d_red, maxdiff ? c.h_red : nullptr));
+  HIPCHK(launch_rhoupdat(c, c.phase == PHASE_POST_STREAM, c.d_red, maxdiff ? c.h_red : nullptr, ++c.red_seq));
   c.mom = MOM_ARRAYS;
   if (maxdiff) {
-    HIPCHK(hipStreamSynchronize(c.stream));
+    HIPCHK(wait_flag((const uint32_t*)(c.h_red + 1), c.red_seq, c.stream));
     *maxdiff = c.h_red[0];
   }
   return MFC_OK;
@@ -933,8 +941,8 @@ int mfc_prt_get(mfc_ctx* ctx, int32_t field, double* a) {
   Particles& P = c.pt;
   double* d = pfield(P, field);
   if (!d || !a || P.np <= 0) return MFC_ERR_ARG;
-  HIPCHK(hipMemcpyAsync(a, d, sizeof(double) * 3 * P.np, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part = {a, d, sizeof(double) * 3 * P.np};
+  HIPCHK(copy_to_host(c, &part, 1));
   return MFC_OK;
 }
 
@@ -1071,9 +1079,8 @@ int mfc_get_maps(mfc_ctx* ctx, int32_t which, int32_t* ib, int32_t* is) {
   if (rc) return rc;
   int32_t* s = (int32_t*)c.staging;
   HIPCHK(launch_maps_to_host_layout(c, which, s, s + c.g.ncell));
-  HIPCHK(hipMemcpyAsync(ib, s, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipMemcpyAsync(is, s + c.g.ncell, b, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part[2] = {{ib, s, b}, {is, s + c.g.ncell, b}};
+  HIPCHK(copy_to_host(c, part, 2));
   return MFC_OK;
 }
 
@@ -1322,8 +1329,8 @@ int mfc_diag_sums(mfc_ctx* ctx, double* out6) {
   if (rc) return rc;
   if ((rc = ensure_diag(ctx, 6))) return rc;
   HIPCHK(launch_field_sums(c, c.diag_part, c.diag_out));
-  HIPCHK(hipMemcpyAsync(out6, c.diag_out, sizeof(double) * 6, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part = {out6, c.diag_out, sizeof(double) * 6};
+  HIPCHK(copy_to_host(c, &part, 1));
   return MFC_OK;
 }
 
@@ -1376,8 +1383,8 @@ int mfc_diag_spectrum(mfc_ctx* ctx, int32_t nek, double* ek) {
   }
   const double2* tw[3] = {c.diag_tw[0], c.diag_tw[1], c.diag_tw[2]};
   HIPCHK(launch_spectrum(c, nek, c.diag_Z, tw, c.diag_part, c.diag_out));
-  HIPCHK(hipMemcpyAsync(ek, c.diag_out, sizeof(double) * nek, hipMemcpyDeviceToHost, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
+  const HostPart part = {ek, c.diag_out, sizeof(double) * nek};
+  HIPCHK(copy_to_host(c, &part, 1));
   return MFC_OK;
 }
 

@@ -392,15 +392,19 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x == 0) part[blockIdx.x] = d;
 }
 
-// The maximum of the workgroups' maxima, stored where the host reads it
-// (pinned memory: no copy follows).
+// The maximum of the workgroups' maxima, stored where the host reads it, and
+// then seq in the word the host polls (pinned memory: no copy, no stream
+// synchronisation follows).
 __global__ void __launch_bounds__(256)
-    k_rho_residual(const uint64_t* __restrict__ part, int n, uint64_t* __restrict__ out) {
+    k_rho_residual(const uint64_t* __restrict__ part, int n, uint64_t* __restrict__ out, uint32_t seq) {
   uint64_t d = 0;
 #pragma unroll 8
   for (int i = threadIdx.x; i < n; i += 256) d = max(d, part[i]);
   d = block_max(d);
-  if (threadIdx.x == 0) *out = d;
+  if (threadIdx.x == 0) {
+    *out = d;
+    __hip_atomic_store((uint32_t*)(out + 1), seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 // initpop (initial.f90:3-28): deviation equilibrium with rho = 0.
@@ -717,14 +721,14 @@ static void rhoupdat_dispatch(Ctx& c, bool pulled, dim3 grid, double* part) {
 
 int rhoupdat_blocks(const Ctx& c) { return (int)std::min(nblocks(c.g.ncell), 16384u); }
 
-hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out) {
+hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out, uint32_t seq) {
   const unsigned nb = (unsigned)rhoupdat_blocks(c);
   if (c.prec == MFC_PREC_FP64)
     rhoupdat_dispatch<double>(c, pulled, dim3(nb), part);
   else
     rhoupdat_dispatch<float>(c, pulled, dim3(nb), part);
   if (out) hipLaunchKernelGGL(k_rho_residual, dim3(1), dim3(256), 0, c.stream, (const uint64_t*)part, (int)nb,
-                              (uint64_t*)out);
+                              (uint64_t*)out, seq);
   return hipGetLastError();
 }
 

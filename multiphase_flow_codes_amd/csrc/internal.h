@@ -188,9 +188,11 @@ struct Ctx {
   int32_t* d_status = nullptr;
   int32_t* h_status = nullptr;      // pinned
   double* d_red = nullptr;          // workgroup maxima of rhoupdat
-  double* h_red = nullptr;          // pinned
+  double* h_red = nullptr;          // pinned: rhoupdat's residual and the word that says it is there
+  uint32_t red_seq = 0;
   void* staging = nullptr;          // device staging for host transfers
   size_t staging_bytes = 0;
+  int pipe_dev = -1;                // device whose host-copy slots this context keeps (hostcopy.hip)
   std::string err;
   // optional timing of the collide kernel: event pairs recorded around every
   // `timing`-th launch (0: off), summed by mfc_get_timing
@@ -227,8 +229,9 @@ hipError_t launch_collide(Ctx& c, bool arrays);
 hipError_t launch_collide_tiles(Ctx& c, const uint32_t* list, uint32_t n, bool far);
 hipError_t launch_macro(Ctx& c, bool pulled);
 int rhoupdat_blocks(const Ctx& c);   // workgroup maxima launch_rhoupdat leaves in `part`
-// out (device-visible, may be null): max |rho_new - rho_old|
-hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out);
+// out (pinned, may be null): max |rho_new - rho_old|, then `seq` in the word
+// behind it
+hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out, uint32_t seq);
 hipError_t launch_initpop(Ctx& c);
 hipError_t launch_pop_to_aos(Ctx& c, double* dst, int z0, int nzs, bool pulled);
 hipError_t launch_aos_to_pop(Ctx& c, const double* src, int z0, int nzs, bool pulled);
@@ -260,6 +263,18 @@ hipError_t launch_maps_to_host_layout(Ctx& c, int which, int32_t* ib, int32_t* i
 // near/far tile lists from the current positions (c.tiles allocated)
 hipError_t launch_tiles(Ctx& c, TileLists& T);
 hipError_t launch_links_dense(Ctx& c, int32_t* ilink, int32_t* mlink, double* alink);
+
+// ---- host copies (hostcopy.hip) ----
+struct HostPart {
+  void* host;
+  const void* dev;
+  size_t bytes;
+};
+constexpr int kMaxParts = 4;
+hipError_t copy_to_host(Ctx& c, const HostPart* part, int nparts);   // waits
+hipError_t wait_flag(const uint32_t* flag, uint32_t value, hipStream_t s);
+void host_pipe_ref(int dev);     // a context of the device was created
+void host_pipe_unref(int dev);   // and destroyed
 
 // ---- launchers (initial.hip) ----
 int init_mode_kx();   // kx values of the mode table (0..16)
