@@ -320,11 +320,11 @@ int check_faults(mfc_ctx* ctx) {
 // beads_links into the map buffer that does not hold the previous step's map
 // (the one beads_filling still needs), clearing what that buffer marked
 // before.  With `overlap_check` the links pass also runs ovlpchk.
-int links_now(mfc_ctx* ctx, int overlap_check, int istep, bool with_find = false) {
+int links_now(mfc_ctx* ctx, int overlap_check, int istep, bool defer_contacts = false) {
   Ctx& c = ctx->c;
   Particles& P = c.pt;
   const int target = (P.map_cur != P.map_old) ? P.map_cur : (P.map_cur ^ 1);
-  HIPCHK(launch_links(c, target, overlap_check, istep, with_find));
+  HIPCHK(launch_links(c, target, overlap_check, istep, defer_contacts));
   P.map_cur = target;
   return MFC_OK;
 }
@@ -486,10 +486,9 @@ int mfc_destroy(mfc_ctx* ctx) {
   for (double* a : pd) F(a);
   F(P.lk_out); F(P.ct_list); F(P.ct_count);
   F(P.isn[0]); F(P.isn[1]); F(P.mask[0]); F(P.mask[1]);
-  F(P.lk_node); F(P.lk_dir); F(P.lk_cnt); F(P.lk_off); F(P.lk_part);
+  F(P.lk_node); F(P.lk_dir); F(P.lk_cnt);
   F(P.sol_list[0]); F(P.sol_list[1]); F(P.sol_cnt[0]); F(P.sol_cnt[1]);
-  F(P.sh_node); F(P.sh_hits); F(P.sh_cnt);
-  F(P.fill_list); F(P.fill_count); F(P.cell_cnt); F(P.cell_list); F(P.ord);
+  F(P.cell_cnt); F(P.cell_list); F(P.ord);
   F(c.d_status); F(c.d_red); F(c.staging);
   F(c.diag_part); F(c.diag_out); F(c.diag_Z);
   for (int a = 0; a < 3; ++a) F(c.diag_tw[a]);
@@ -524,6 +523,7 @@ int mfc_status(mfc_ctx* ctx, int32_t* out16) {
   NEEDCTX;
   if (!out16) return MFC_ERR_ARG;
   Ctx& c = ctx->c;
+  HIPCHK(launch_link_totals(c));
   const HostPart part = {c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT};
   HIPCHK(copy_to_host(c, &part, 1));
   memcpy(out16, c.h_status, sizeof(int32_t) * ST_COUNT);
@@ -796,41 +796,20 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
     P.seg_cap = segment_capacity(c.p.rad, P.slab);
     const size_t nsegs = (size_t)npart * P.nseg;
     const size_t nodes = nsegs * (size_t)P.seg_cap;
-    void** segbufs[] = {(void**)&P.lk_cnt, (void**)&P.lk_off, (void**)&P.seg_ft,
-                        (void**)&P.sol_list[0], (void**)&P.sol_list[1], (void**)&P.sol_cnt[0],
-                        (void**)&P.sol_cnt[1], (void**)&P.sh_node, (void**)&P.sh_hits,
-                        (void**)&P.sh_cnt};
+    void** segbufs[] = {(void**)&P.lk_cnt, (void**)&P.seg_ft, (void**)&P.sol_list[0], (void**)&P.sol_list[1],
+                        (void**)&P.sol_cnt[0], (void**)&P.sol_cnt[1]};
     for (void** a : segbufs) {
       if (*a) HIPCHK(hipFree(*a));
       *a = nullptr;
     }
     HIPCHK(hipMalloc(&P.lk_cnt, sizeof(int32_t) * nsegs));
-    HIPCHK(hipMalloc(&P.lk_off, sizeof(int64_t) * (nsegs + 1)));
-    if (P.lk_part) HIPCHK(hipFree(P.lk_part));
-    HIPCHK(hipMalloc(&P.lk_part, sizeof(int64_t) * 2 * (nsegs / kScanChunk + 1)));
     for (int b = 0; b < 2; ++b) {
       HIPCHK(hipMalloc(&P.sol_list[b], sizeof(uint32_t) * nodes));
       HIPCHK(hipMalloc(&P.sol_cnt[b], sizeof(int32_t) * nsegs));
     }
-    HIPCHK(hipMalloc(&P.sh_node, sizeof(uint32_t) * nodes));
-    HIPCHK(hipMalloc(&P.sh_hits, sizeof(uint32_t) * nodes));
-    HIPCHK(hipMalloc(&P.sh_cnt, sizeof(int32_t) * nsegs));
     HIPCHK(hipMalloc(&P.seg_ft, sizeof(double) * 6 * nsegs * kMaxBBSplit));
-    // every refilled node was solid: at most the solid nodes of all spheres
-    const double rs = c.p.rad + 1.0;
-    P.fill_cap = (int64_t)ceil(4.0 / 3.0 * M_PI * rs * rs * rs) * npart + 64;
-    if (P.fill_list) HIPCHK(hipFree(P.fill_list));
-    if (P.fill_count) HIPCHK(hipFree(P.fill_count));
-    HIPCHK(hipMalloc(&P.fill_list, sizeof(uint64_t) * P.fill_cap));
-    HIPCHK(hipMalloc(&P.fill_count, sizeof(int32_t)));
-    // link pool: every link's node lies in the shell r < d <= r + sqrt(2)
-    // around its centre, and a node outside a convex sphere sees it along at
-    // most 9 of the 18 directions (never along both c and -c).
-    const double r = c.p.rad, h = sqrt(3.0) / 2.0;
-    const double ro = r + sqrt(2.0) + h, ri = std::max(0.0, r - h);
-    const double shell = 4.0 / 3.0 * M_PI * (ro * ro * ro - ri * ri * ri);
-    const int64_t per = (int64_t)ceil(shell) * 9 + 64;
-    const int64_t cap = per * npart;
+    P.lk_seg = segment_links(c.p.rad, P.slab);
+    const int64_t cap = (int64_t)nsegs * P.lk_seg;
     if (P.lk_node) HIPCHK(hipFree(P.lk_node));
     if (P.lk_dir) HIPCHK(hipFree(P.lk_dir));
     if (P.lk_alpha) HIPCHK(hipFree(P.lk_alpha));
@@ -891,8 +870,7 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
     double* pd[] = {P.yp, P.ypglb, P.ypglbp, P.wp, P.wpp, P.omgp, P.omgpp, P.fHIp, P.flubp, P.torqp,
                     P.forcep, P.forcepp, P.torqpp, P.dwdt, P.domgdt, P.thetap};
     for (double* a : pd) HIPCHK(hipMemsetAsync(a, 0, sizeof(double) * 3 * npart, c.stream));
-    HIPCHK(hipMemsetAsync(P.lk_off, 0, sizeof(int64_t) * ((size_t)npart * P.nseg + 1), c.stream));
-    HIPCHK(hipMemsetAsync(P.fill_count, 0, sizeof(int32_t), c.stream));
+    HIPCHK(hipMemsetAsync(P.lk_cnt, 0, sizeof(int32_t) * (size_t)npart * P.nseg, c.stream));
   }
   HIPCHK(hipMemsetAsync(c.d_status, 0, sizeof(int32_t) * ST_COUNT, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
@@ -1207,7 +1185,7 @@ int step_overlapped(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       if ((he = launch_move(c, it == c.p.irelease ? 1 : 0, 1, true)) != hipSuccess) break;
       P.map_old = P.map_cur;
       if ((prc = links_now(ctx, 1, it, true))) break;
-      if ((he = launch_filling(c, false, nullptr)) != hipSuccess) break;
+      if ((he = launch_filling(c, true, nullptr)) != hipSuccess) break;
       c.f_version++;
       if ((prc = mfc_macrovar(ctx))) break;
       he = hipEventRecord(c.ev_part, sB);
@@ -1285,14 +1263,14 @@ int mfc_step(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       // with its overlap check fused in (reported by mfc_sync)
       HIPCHK(launch_move(c, it == c.p.irelease ? 1 : 0, 1, true));
       P.map_old = P.map_cur;
-      // links with the refill search in the expansion grid, then the refill
+      // links, then the refill with the contact links listed in its grid
       if ((rc = links_now(ctx, 1, it, true))) return rc;
       if (s + 1 < nsteps && c.p.xkf > 0.0) {
         forcing_modes_host(c);
         drawn = true;
         drawn_rc = prepare_modes(ctx, job);
       }
-      HIPCHK(launch_filling(c, false, drawn && !drawn_rc && job.nblk > 0 ? &job : nullptr));
+      HIPCHK(launch_filling(c, true, drawn && !drawn_rc && job.nblk > 0 ? &job : nullptr));
       c.f_version++;
     }
     if ((rc = mfc_macrovar(ctx))) return rc;

@@ -3,9 +3,8 @@
 // Each member is an ordinary context (its own size, spheres, rates and body
 // force; state created and initialised through the single-box API).  One
 // ensemble step runs the time-loop body of every member with one grid per
-// stage for all of them: collide, bounce-back (+ lubrication), scatter
-// (+ map clearing), move, link scan, link offsets, link expansion (+ refill
-// search), refill.  Each grid reads its members' argument blocks from a
+// stage for all of them: collide, contact links (+ lubrication), bounce-back
+// (+ map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
 // per-stage table and finds its member from a block-offset table
 // (off[c] <= blockIdx.x < off[c+1]).  The sequence and the per-member state
 // transitions are exactly those of mfc_step, so a member advanced in the
@@ -13,7 +12,7 @@
 //
 // Steps go in chunks of up to kChunk: the host builds the tables of all the
 // chunk's steps into one pinned buffer and uploads them with ONE plain copy;
-// then the chunk's stage grids (8 per step) run, in graph mode as one
+// then the chunk's stage grids (6 per step) run, in graph mode as one
 // recorded HIP graph replayed for every chunk of the same launch shapes.
 // The graphs hold kernel nodes only (their table pointers point into the
 // device table buffer); a graph is destroyed before any buffer its nodes
@@ -39,11 +38,11 @@ using namespace mfc;
 
 namespace {
 
-constexpr int kStages = 8;          // collide + the seven particle stages
+constexpr int kParts = 5;           // particle stages
+constexpr int kStages = 1 + kParts; // collide and those
 constexpr int kRing = 3;            // pinned table buffers in flight
 constexpr int kChunk = 8;           // steps per table upload and per recorded graph
 constexpr int kGraphCache = 4;      // recorded chunk graphs kept (by launch shapes)
-constexpr int kFillBlocksPerBox = 32;
 constexpr int kContactBlocksPerBox = 1;   // contact pre-pass: contacts are rare
 
 struct Member {
@@ -146,14 +145,14 @@ int drop_graphs(mfc_ens* e) {
 // One step's tables for every member, advancing each member's host-side
 // state exactly as mfc_step would.
 struct StepTabs {
-  StageTab coll, st[7];
+  StageTab coll, st[kParts];
   bool arr_any = false;
 };
-const Stage kOrder[7] = {SG_CONTACT, SG_BOUNCE, SG_MOVE, SG_SCAN, SG_COUNT, SG_EXPAND, SG_FILL};
+const Stage kOrder[kParts] = {SG_CONTACT, SG_BOUNCE, SG_MOVE, SG_SCAN, SG_FILL};
 
 int build_step(mfc_ens* e, StepTabs& T) {
   T.coll.arg_bytes = sizeof(CollideArgs);
-  for (int k = 0; k < 7; ++k) T.st[k].arg_bytes = stage_arg_bytes(kOrder[k]);
+  for (int k = 0; k < kParts; ++k) T.st[k].arg_bytes = stage_arg_bytes(kOrder[k]);
   StageTab* st = T.st;
   for (Member& mb : e->m) {
     Ctx& c = mb.box->c;
@@ -191,15 +190,11 @@ int build_step(mfc_ens* e, StepTabs& T) {
       if (P.map_np[target] != 0) return efail(e, MFC_ERR_STATE, "ensemble: link target map not cleared");
       const ScanArgs sc = scan_args(c, target, 1, it);
       st[3].add(&sc, P.np * P.nseg);
-      st[3].lds = std::max(st[3].lds, sizeof(uint32_t) * (size_t)P.seg_cap);
-      const ScanCountArgs cn = count_args(c, target);
-      st[4].add(&cn, 1);
-      const ExpandArgs ex = expand_args(c, target, true, &nb);
-      st[5].add(&ex, nb);
+      st[3].lds = std::max(st[3].lds, scan_lds(c));
       P.map_np[target] = P.np;
       P.map_cur = target;
-      FillApplyArgs fa;
-      if (fill_apply_args(c, kFillBlocksPerBox, fa)) st[6].add(&fa, kFillBlocksPerBox);
+      const FillKArgs fa = fill_args(c, true, true, &nb);
+      st[4].add(&fa, nb);
       c.f_version++;
     }
     // macrovar
@@ -223,8 +218,7 @@ int ens_chunk(mfc_ens* e, int n) {
   // lay the tables out in one buffer: per step, per stage [args][off]
   size_t pos[kChunk][kStages][2], total = 0;
   for (int s = 0; s < n; ++s) {
-    StageTab* tabs[kStages] = {&T[s].coll, &T[s].st[0], &T[s].st[1], &T[s].st[2], &T[s].st[3], &T[s].st[4],
-                               &T[s].st[5], &T[s].st[6]};
+    StageTab* tabs[kStages] = {&T[s].coll, &T[s].st[0], &T[s].st[1], &T[s].st[2], &T[s].st[3], &T[s].st[4]};
     for (int k = 0; k < kStages; ++k) {
       pos[s][k][0] = total;
       total = align_up(total + tabs[k]->args.size());
@@ -259,8 +253,7 @@ int ens_chunk(mfc_ens* e, int n) {
   }
   char* h = e->h_tab[r];
   for (int s = 0; s < n; ++s) {
-    StageTab* tabs[kStages] = {&T[s].coll, &T[s].st[0], &T[s].st[1], &T[s].st[2], &T[s].st[3], &T[s].st[4],
-                               &T[s].st[5], &T[s].st[6]};
+    StageTab* tabs[kStages] = {&T[s].coll, &T[s].st[0], &T[s].st[1], &T[s].st[2], &T[s].st[3], &T[s].st[4]};
     for (int k = 0; k < kStages; ++k) {
       if (!tabs[k]->args.empty()) memcpy(h + pos[s][k][0], tabs[k]->args.data(), tabs[k]->args.size());
       memcpy(h + pos[s][k][1], tabs[k]->off.data(), sizeof(int) * tabs[k]->off.size());
@@ -274,7 +267,7 @@ int ens_chunk(mfc_ens* e, int n) {
       EHIP(launch_batched_collide(e->prec, e->walls, e->collide_bs, e->collide_remap, d + pos[s][0][0],
                                   (const int*)(d + pos[s][0][1]), U.coll.nc, U.coll.off.back(), U.arr_any,
                                   e->stream));
-      for (int k = 0; k < 7; ++k) {
+      for (int k = 0; k < kParts; ++k) {
         const StageTab& t = U.st[k];
         EHIP(launch_batched(kOrder[k], e->prec, e->walls, d + pos[s][k + 1][0],
                             (const int*)(d + pos[s][k + 1][1]), t.nc, t.off.back(), t.lds, e->stream));
@@ -292,7 +285,7 @@ int ens_chunk(mfc_ens* e, int n) {
       sig.push_back(T[s].coll.nc);
       sig.push_back(T[s].coll.off.back());
       sig.push_back(T[s].arr_any ? 1LL : 0LL);
-      for (int k = 0; k < 7; ++k) {
+      for (int k = 0; k < kParts; ++k) {
         sig.push_back(T[s].st[k].nc);
         sig.push_back(T[s].st[k].off.back());
         sig.push_back((long long)T[s].st[k].lds);

@@ -40,9 +40,6 @@ constexpr int kMaxDevices = 64;   // device ordinals the per-device tables cover
 // (between 1 and 4/3 times 2r + mingap wide) holds at most kCellCap centres
 // (non-overlapping spheres never come close to it; more is reported)
 constexpr int kCellMinParticles = 512;
-// segment-count scans of more than kScanChunk segments run over several
-// workgroups, kScanChunk segments each
-constexpr int kScanChunk = 4096;
 // a segment's links are split over up to this many bounce-back workgroups
 constexpr int kMaxBBSplit = 4;
 constexpr int kCellCap = 16;
@@ -124,12 +121,8 @@ struct Particles {
   // later clears and what beads_filling scans for uncovered nodes
   uint32_t* sol_list[2] = {nullptr, nullptr};
   int32_t* sol_cnt[2] = {nullptr, nullptr};
-  // fluid nodes within r + 1.5 of a centre and the link directions they see
-  // (bit q set: direction q crosses the surface), per segment
-  uint32_t* sh_node = nullptr;
-  uint32_t* sh_hits = nullptr;
-  int32_t* sh_cnt = nullptr;
-  // boundary links, grouped by segment
+  // boundary links: lk_seg slots per segment, lk_cap in all
+  int lk_seg = 0;
   int64_t lk_cap = 0;
   uint32_t* lk_node = nullptr;
   uint8_t* lk_dir = nullptr;
@@ -143,8 +136,6 @@ struct Particles {
   OrderEntry* ord = nullptr;
   int64_t ord_cap = 0;
   int32_t* lk_cnt = nullptr;   // links per segment
-  int64_t* lk_part = nullptr;  // per-chunk sums of the segment counts (multi-block scan)
-  int64_t* lk_off = nullptr;   // link offset per segment (np * nseg + 1)
   double* seg_ft = nullptr;    // force and torque per bounce-back unit (6 each)
   // bounce-back units per segment (1..kMaxBBSplit, MFC_BB_SPLIT); one
   // measured best on MI355X at 256^3 and 1024^3 (more units: more blocks,
@@ -157,10 +148,6 @@ struct Particles {
   int32_t* cell_list = nullptr;
   bool cells_ok = false;
   bool cells_zeroed = false;   // cleared by the fused bounce-back grid for the move that follows
-  // nodes to refill, found by beads_filling's first pass
-  uint64_t* fill_list = nullptr;
-  int32_t* fill_count = nullptr;
-  int64_t fill_cap = 0;
 };
 
 struct Ctx {
@@ -241,9 +228,11 @@ hipError_t launch_force_field(Ctx& c, int slot, double* fx, double* fy, double* 
 int segments_per_particle(double rad, int slab);
 int segment_capacity(double rad, int slab);
 int segment_planes(double rad, int npart);
-// with_find: the first pass of beads_filling (previous map vs the new one)
-// runs in the same grid as the link expansion
-hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool with_find = false);
+int segment_links(double rad, int slab);
+// defer_contacts: the contact links are listed by the refill grid that follows
+hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool defer_contacts = false);
+// ST_NLINKS and ST_NSOLID of the current build
+hipError_t launch_link_totals(Ctx& c);
 // with `fused` set (mfc_step) the bounce-back grid also computes the
 // lubrication forces and clears the next map target, and fHIp / torqp are
 // left for the move kernel to sum from the segments
@@ -253,9 +242,9 @@ hipError_t launch_map_clear(Ctx& c, int buf);
 hipError_t launch_move(Ctx& c, int first, int wrap, bool from_seg = false);
 hipError_t launch_redistribute(Ctx& c, int istep);
 struct TableJob;
-// job: a forcing table evaluated by extra blocks of the refill grid (or by
-// its own launch when there is nothing to refill)
-hipError_t launch_filling(Ctx& c, bool find = true, const TableJob* job = nullptr);
+// contacts: the grid also lists the contact links; job: a forcing table
+// evaluated by extra blocks of it
+hipError_t launch_filling(Ctx& c, bool contacts = false, const TableJob* job = nullptr);
 hipError_t launch_initpartvel(Ctx& c);
 // (re)build the pair-search cells if they are on and stale
 hipError_t ensure_cells(Ctx& c);

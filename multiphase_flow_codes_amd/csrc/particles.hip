@@ -4,16 +4,20 @@
 //
 // Data layout.  Node maps are double-buffered (current / previous step):
 // an int32 id map (particle id, 1-based, or 0) and a 1-bit solid mask read by
-// the collide kernel.  Boundary links are a compact list grouped by particle
-// (node index, direction, wall fraction), built in a deterministic order by
-// one workgroup per particle scanning the particle's bounding box; no dense
-// 18-per-node link arrays exist.  Maps are maintained incrementally: a build
+// the collide kernel.  Boundary links (node index, direction, wall fraction)
+// are listed per segment of a particle's bounding box, each segment in a slot
+// of its own (Particles::lk_seg links), in a deterministic order by the workgroup
+// that scans the segment; no dense 18-per-node link arrays exist.  Maps are maintained incrementally: a build
 // first clears the nodes its buffer marked two steps earlier, so no pass
 // ever touches the whole lattice.  All particle state is FP64.
 //
 // Compiled with -ffp-contract=off: the geometry is evaluated exactly as the
 // reference writes it, so maps and wall fractions match the FP64 oracle bit
 // for bit.
+#include <algorithm>
+
+#include <math.h>
+
 #include "force_table.h"
 #include "internal.h"
 #include "lbm_access.h"
@@ -200,52 +204,54 @@ __device__ void box_info(const double* __restrict__ pos, int p, const PGeom& G, 
   __syncthreads();
 }
 
-// Geometry of node (iw, jw, kw) of the box.  Returns false if the node is
-// outside the reference's bounding box (partlib.f90:965-985) or beyond a wall.
-__device__ bool node_geom(const BoxInfo& B, const PGeom& G, int iw, int jw, int kw, LinkGeom& L) {
-  if (jw < 0 || jw >= G.ny) return false;
-  const double zp = (double)(kw + 1) - 0.5;
-  L.zimg = near_image(B.z0, zp, G.nz);
-  L.zz0 = zp - L.zimg;
-  if (!(fabs(L.zz0) <= G.radp2)) return false;
-  const double yp = (double)(jw + 1) - 0.5;
-  L.yimg = y_image(kw == B.kfirst ? B.y0 : B.yr, yp, G);
-  L.yy0 = yp - L.yimg;
-  if (!(fabs(L.yy0) <= G.radp2)) return false;
-  const double xp = (double)(iw + 1) - 0.5;
-  L.ximg = near_image((kw == B.kfirst && jw == B.jfirst) ? B.x0 : B.xr, xp, G.nx);
-  L.xx0 = xp - L.ximg;
-  if (!(fabs(L.xx0) <= G.radp2)) return false;
-  L.rr0 = L.xx0 * L.xx0 + L.yy0 * L.yy0 + L.zz0 * L.zz0;
-  return true;
-}
-
 __device__ __forceinline__ int block_exclusive_scan(int v, int* sh, int& total);
 
 // Rows (y, z) of one segment's walk: the x run of each row that can hold
-// nodes within r + 1.5 of the centre (a superset: the node test decides),
-// and the runs' prefix sums.  A segment has at most PB rows (one thread per
-// row): slab planes of at most PB / slab candidate rows each, which the
-// choice of slab guarantees (segment_planes).
-struct SegRows {
-  int start[PB + 1];   // first flattened index of each row
-  short xa[PB];        // first box x index of each row's run
-  int nrows;
+// nodes within r + 1.5 of the centre (a superset: the node test decides).  A
+// segment has at most PB rows (one thread per row): slab planes of at most
+// PB / slab candidate rows each, which the choice of slab guarantees
+// (segment_planes).
+struct SegRow {
+  uint32_t n0;         // node index of the row's x = 0
+  int xs;              // flattened index t of the row is at x = xs + t (unwrapped)
+  int jw, kw;
+  double yimg, zimg;   // imaged centre used for the row's nodes
 };
+
+// Geometry of the node at unwrapped x `ux` of row w (iw: its wrapped x).
+// Returns false if the node is outside the reference's bounding box
+// (partlib.f90:965-985); rows outside it or beyond a wall have no run.
+__device__ __forceinline__ bool node_geom(const BoxInfo& B, const PGeom& G, const SegRow& w, int ux, int& iw, LinkGeom& L) {
+  iw = wrap1(ux, G.nx);
+  const double zp = (double)(w.kw + 1) - 0.5;
+  L.zimg = w.zimg;
+  L.zz0 = zp - L.zimg;
+  const double yp = (double)(w.jw + 1) - 0.5;
+  L.yimg = w.yimg;
+  L.yy0 = yp - L.yimg;
+  const double xp = (double)(iw + 1) - 0.5;
+  L.ximg = near_image((w.kw == B.kfirst && w.jw == B.jfirst) ? B.x0 : B.xr, xp, G.nx);
+  L.xx0 = xp - L.ximg;
+  L.rr0 = L.xx0 * L.xx0 + L.yy0 * L.yy0 + L.zz0 * L.zz0;
+  return fabs(L.xx0) <= G.radp2;
+}
 
 // Walk of one segment (z-slab s) of the box in passes of PB candidate nodes,
 // the slab's row runs flattened x-fastest so every lane of a pass has a node.
 // Every thread runs the same number of passes (barriers are allowed in fn);
-// fn(active, iw, jw, kw) is called once per pass, in row-major, x-ascending
-// node order.
+// fn(active, row, ux) is called once per pass, in row-major, x-ascending
+// node order.  rowof: LDS bytes, one per node of the walk, for its row's
+// number (written by the row's thread; a search of the rows' starts by every
+// node is a chain of six dependent LDS reads).
 template <typename F>
-__device__ __forceinline__ void walk_segment(const BoxInfo& B, const PGeom& G, int s, SegRows& R,
-                                             int* sh, F&& fn) {
+__device__ __forceinline__ void walk_segment(const BoxInfo& B, const PGeom& G, int s, SegRow* rows,
+                                             uint8_t* rowof, int* sh, F&& fn) {
   const int z0 = s * G.slab;
   const int nzs = max(0, min(G.slab, B.az.cnt - z0));
   const int nrows = nzs * B.ay.cnt;   // <= PB
   // x run of each row (a row at most PB nodes)
-  int run = 0, xa = 0;
+  int run = 0;
+  SegRow w;
   const int r = (int)threadIdx.x;
   if (r < nrows) {
     const int tz = r / B.ay.cnt, ty = r - tz * B.ay.cnt;
@@ -253,9 +259,11 @@ __device__ __forceinline__ void walk_segment(const BoxInfo& B, const PGeom& G, i
     const int jw = G.walls_y ? B.ay.lo + ty : wrap1(B.ay.lo + ty, G.ny);
     if (jw >= 0 && jw < G.ny) {
       const double zp = (double)(kw + 1) - 0.5;
-      const double zz0 = zp - near_image(B.z0, zp, G.nz);
+      w.zimg = near_image(B.z0, zp, G.nz);
+      const double zz0 = zp - w.zimg;
       const double yp = (double)(jw + 1) - 0.5;
-      const double yy0 = yp - y_image(kw == B.kfirst ? B.y0 : B.yr, yp, G);
+      w.yimg = y_image(kw == B.kfirst ? B.y0 : B.yr, yp, G);
+      const double yy0 = yp - w.yimg;
       const double rem = G.rlink2 - yy0 * yy0 - zz0 * zz0;
       if (fabs(zz0) <= G.radp2 && fabs(yy0) <= G.radp2 && rem >= 0.0) {
         // node i (unwrapped) sits at i + 0.5; keep |i + 0.5 - x0| <= sqrt(rem) + 1
@@ -264,47 +272,58 @@ __device__ __forceinline__ void walk_segment(const BoxInfo& B, const PGeom& G, i
         const int ihi = min((int)floor(B.x0 + dx - 0.5), B.ax.lo + B.ax.cnt - 1);
         if (ihi >= ilo) {
           run = ihi - ilo + 1;
-          xa = ilo - B.ax.lo;
+          w.xs = ilo;
+          w.jw = jw;
+          w.kw = kw;
+          w.n0 = (uint32_t)G.nx * ((uint32_t)jw + (uint32_t)G.ny * (uint32_t)kw);
         }
       }
     }
   }
   int total;
   const int st = block_exclusive_scan(run, sh, total);
-  if (r < nrows) {
-    R.start[r] = st;
-    R.xa[r] = (short)xa;
+  if (run > 0) {
+    w.xs -= st;
+    rows[r] = w;
+    for (int i = 0; i < run; ++i) rowof[st + i] = (uint8_t)r;
   }
-  if (r == 0) R.start[nrows] = total;
   __syncthreads();
   for (int t0 = 0; t0 < total; t0 += PB) {
     const int t = t0 + (int)threadIdx.x;
     const bool act = t < total;
-    int iw = 0, jw = 0, kw = 0;
-    if (act) {
-      int lo = 0, hi = nrows;   // the row holding t: start[lo] <= t < start[lo + 1]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (R.start[mid] <= t) lo = mid; else hi = mid;
-      }
-      const int tz = lo / B.ay.cnt, ty = lo - tz * B.ay.cnt;
-      const int tx = R.xa[lo] + (t - R.start[lo]);
-      kw = wrap1(B.az.lo + z0 + tz, G.nz);
-      jw = G.walls_y ? B.ay.lo + ty : wrap1(B.ay.lo + ty, G.ny);
-      iw = wrap1(B.ax.lo + tx, G.nx);
-    }
-    fn(act, iw, jw, kw);
+    const int row = act ? (int)rowof[t] : 0;
+    fn(act, row, act ? rows[row].xs + t : 0);
   }
 }
 
-// Neighbour test of direction q from node (iw,jw,kw); fills rr1 and offsets.
-__device__ __forceinline__ bool link_hit(const LinkGeom& L, int iw, int jw, int kw, int q, double r2,
-                                         double& xx1, double& yy1, double& zz1, double& rr1) {
+// Directions q (bit q) along which the neighbour of a node is inside the
+// sphere (rr1 - r2 <= 0, the squares of the three possible offsets per axis
+// taken once; the sums are those of link_end).
+__device__ __forceinline__ uint32_t link_hits(const LinkGeom& L, int iw, int jw, int kw, double r2) {
+  double X[3], Y[3], Z[3];
+#pragma unroll
+  for (int o = 0; o < 3; ++o) {
+    const double x = (double)(iw + o) - 0.5 - L.ximg;
+    const double y = (double)(jw + o) - 0.5 - L.yimg;
+    const double z = (double)(kw + o) - 0.5 - L.zimg;
+    X[o] = x * x;
+    Y[o] = y * y;
+    Z[o] = z * z;
+  }
+  uint32_t hits = 0;
+#pragma unroll
+  for (int q = 1; q < NPOP; ++q)
+    if (X[cx(q) + 1] + Y[cy(q) + 1] + Z[cz(q) + 1] - r2 <= 0.0) hits |= 1u << q;
+  return hits;
+}
+
+// The neighbour of node (iw, jw, kw) along q: its offsets from the centre.
+__device__ __forceinline__ void link_end(const LinkGeom& L, int iw, int jw, int kw, int q, double& xx1,
+                                         double& yy1, double& zz1, double& rr1) {
   xx1 = (double)(iw + 1 + cx(q)) - 0.5 - L.ximg;
   yy1 = (double)(jw + 1 + cy(q)) - 0.5 - L.yimg + 0.0;
   zz1 = (double)(kw + 1 + cz(q)) - 0.5 - L.zimg + 0.0;
   rr1 = xx1 * xx1 + yy1 * yy1 + zz1 * zz1;
-  return (rr1 - r2) <= 0.0;
 }
 
 // Wavefront-wide inclusive scans through DPP lane moves (no LDS round trip):
@@ -436,23 +455,46 @@ __global__ void __launch_bounds__(PB)
 // beads_links (partlib.f90:934-1043) for one segment of a particle's box:
 // classify every box node (solid: mark the id map and mask, list it; fluid
 // within r + 1.5: keep it in LDS), then test the 18 directions of the kept
-// nodes, one node per lane, and store node and direction bits per segment.
-// With `ovl` set the first segment of each particle also performs the overlap
-// check of beads_redistribute (partlib.f90:2631-2646) on the freshly wrapped
-// positions.  Dynamic LDS: seg_cap node indices.
+// nodes, one node per lane, list their links (node, direction) in LDS and
+// write them with their wall fractions (partlib.f90:1013-1024), one link per
+// lane, into the segment's slot, in (node, direction) order.  With `ovl` set the
+// first segment of each particle also performs the overlap check of
+// beads_redistribute (partlib.f90:2631-2646) on the freshly wrapped positions.
+// Dynamic LDS: shell_bytes for the kept nodes, packed_bytes for a pass's links
+// (during the walk: its rows' numbers), then the segment's rows.
+// Bound: instructions (FP64 geometry of the candidates, then of the kept nodes
+// and the links); more waves per SIMD change nothing.  Slots of fixed size
+// need no offsets: with links placed by a prefix sum over all segments (shell
+// lists in memory, a grid for the sum, a grid to write the links and find the
+// nodes to refill) the rebuild and the refill took 88 us at 256^3 with 300
+// spheres of radius 8, 82 us with 900 of radius 4, 284 us with 2500 of radius
+// 6 and 33 us at 64^3 in FP64 with 8 of radius 4; now 68, 58, 248 and 21
+// us.  Of that the scan was 66, 52, 220 and 13.5 us while each node searched the
+// rows' starts for its row and took the image of the centre by itself and each
+// direction squared its own offsets: 44, 34, 144 and 11.3 us with the rows'
+// numbers and geometry in LDS and the squares shared.
+constexpr int kPassLinks = 9 * PB;   // a node outside a sphere has at most 9 links
+__host__ __device__ constexpr int shell_bytes(int seg_cap) { return (2 * seg_cap + 7) & ~7; }
+__host__ __device__ constexpr int packed_bytes(int seg_cap) {
+  return seg_cap > 4 * kPassLinks ? (seg_cap + 7) & ~7 : 4 * kPassLinks;
+}
 __device__ __forceinline__ void links_scan_body(int b_, const double* __restrict__ ypglb, int np, int nseg, int seg_cap, PGeom G,
                  int32_t* __restrict__ isn, uint32_t* __restrict__ mask,
                  uint32_t* __restrict__ sol_list, int32_t* __restrict__ sol_cnt,
-                 uint32_t* __restrict__ sh_node, uint32_t* __restrict__ sh_hits,
-                 int32_t* __restrict__ sh_cnt, int32_t* __restrict__ lk_cnt, int ovl, int istep,
+                 const LinkSlots& lk, int32_t* __restrict__ ct_count, int ovl, int istep,
                  int32_t* __restrict__ status, CellArgs cells) {
-  extern __shared__ uint32_t shell[];
+  extern __shared__ uint64_t scan_mem[];
+  uint16_t* shell = (uint16_t*)scan_mem;                                  // row << 8 | x in the box
+  uint32_t* packed = (uint32_t*)((char*)scan_mem + shell_bytes(seg_cap));   // shell index | direction << 24
+  uint8_t* rowof = (uint8_t*)packed;                                      // before the links
+  SegRow* rows = (SegRow*)((char*)packed + packed_bytes(seg_cap));
   __shared__ BoxInfo B;
   __shared__ int wt[2][PB / 64][2];
   __shared__ int sh[PB / 64];
   const int b = b_;
   const int p = (int)div_by((uint32_t)b, G.dseg), s = b - p * nseg;
   if (p >= np) return;
+  if (b == 0 && threadIdx.x == 0) *ct_count = 0;   // listed again once the map is complete
   if (ovl && s == 0) {
     // ovlpchk: flag p if any later particle is closer than 2r
     const bool hit = block_overlap(ypglb, p, np, G, cells);
@@ -464,178 +506,115 @@ __device__ __forceinline__ void links_scan_body(int b_, const double* __restrict
   box_info(ypglb, p, G, B);
   if (!B.ok) {
     if (threadIdx.x == 0) {
-      lk_cnt[b] = 0;
+      lk.cnt[b] = 0;
       sol_cnt[b] = 0;
-      sh_cnt[b] = 0;
       if (s == 0) atomicAdd(&status[ST_BOX_FAULT], 1);
     }
     return;
   }
   uint32_t* sol = sol_list + (size_t)b * seg_cap;
   int parity = 0, nsol = 0, nshell = 0;
-  __shared__ SegRows R;
-  walk_segment(B, G, s, R, sh, [&](bool act, int iw, int jw, int kw) {
+  walk_segment(B, G, s, rows, rowof, sh, [&](bool act, int row, int ux) {
     LinkGeom L;
-    const bool in = act && node_geom(B, G, iw, jw, kw, L) && L.rr0 <= G.rlink2;
+    int iw = 0;
+    const bool in = act && node_geom(B, G, rows[row], ux, iw, L) && L.rr0 <= G.rlink2;
     const bool solid = in && (L.rr0 - G.r2 <= 0.0);
     const bool near = in && !solid;
-    const uint32_t n = (uint32_t)iw + (uint32_t)G.nx * ((uint32_t)jw + (uint32_t)G.ny * (uint32_t)kw);
+    const uint32_t n = act ? rows[row].n0 + (uint32_t)iw : 0u;
     if (solid) atomicMax(&isn[n], p + 1);   // the highest id containing the node wins
     mask_update(mask, solid, n, true);
     int at_s, at_n;
     block_place2(solid, near, wt, parity, nsol, nshell, at_s, at_n);
     if (solid && at_s < seg_cap) sol[at_s] = n;
-    if (near && at_n < seg_cap) shell[at_n] = n;
+    if (near && at_n < seg_cap) shell[at_n] = (uint16_t)(row << 8 | (ux - B.ax.lo));
   });
   __syncthreads();
   const int nsh = min(nshell, seg_cap);
-  uint32_t* shn = sh_node + (size_t)b * seg_cap;
-  uint32_t* shh = sh_hits + (size_t)b * seg_cap;
-  int nl = 0;
+  const int64_t slot = (int64_t)b * lk.cap;
+  int nl = 0, alpha_bad = 0;
   for (int e0 = 0; e0 < nsh; e0 += PB) {
     const int e = e0 + (int)threadIdx.x;
+    uint32_t hits = 0;
     if (e < nsh) {
-      const uint32_t n = shell[e];
-      const uint32_t rw = div_by(n, G.dx);
-      const int iw = (int)(n - rw * (uint32_t)G.nx);
-      const int kw = (int)div_by(rw, G.dy), jw = (int)rw - kw * G.ny;
+      const uint32_t at = shell[e];
+      const SegRow w = rows[at >> 8];
       LinkGeom L;
-      node_geom(B, G, iw, jw, kw, L);
-      uint32_t hits = 0;
-      for (int q = 1; q < NPOP; ++q) {
-        double a1, a2, a3, a4;
-        if (link_hit(L, iw, jw, kw, q, G.r2, a1, a2, a3, a4)) hits |= 1u << q;
-      }
-      shn[e] = n;
-      shh[e] = hits;
-      nl += __popc(hits);
+      int iw;
+      node_geom(B, G, w, B.ax.lo + (int)(at & 255u), iw, L);
+      hits = link_hits(L, iw, w.jw, w.kw, G.r2);
     }
-  }
-  int tot;
-  block_exclusive_scan(nl, sh, tot);
-  if (threadIdx.x == 0) {
-    lk_cnt[b] = tot;
-    sol_cnt[b] = min(nsol, seg_cap);
-    sh_cnt[b] = nsh;
-  }
-}
-
-// Exclusive scan of the per-segment link counts (one workgroup of 1024):
-// each thread sums a contiguous run, the run totals are scanned in LDS.
-__device__ __forceinline__ void scan_counts_body(int b_, const int32_t* __restrict__ cnt, const int32_t* __restrict__ scnt, int nsegs,
-                  int64_t* __restrict__ off, int64_t cap, int32_t* __restrict__ status,
-                  int32_t* __restrict__ fill_count, int32_t* __restrict__ ct_count) {
-  if (threadIdx.x == 0) {
-    *fill_count = 0;   // the next beads_filling starts an empty list
-    *ct_count = 0;     // the expansion lists this rebuild's contact links
-  }
-  __shared__ int64_t part[1024];
-  __shared__ int64_t spart[1024];
-  const int t = threadIdx.x;
-  const int per = (nsegs + 1023) / 1024;
-  const int a = min(nsegs, t * per), e = min(nsegs, a + per);
-  int64_t s = 0, ss = 0;
-  for (int i = a; i < e; ++i) {
-    s += cnt[i];
-    ss += scnt[i];
-  }
-  part[t] = s;
-  spart[t] = ss;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int64_t v = (t >= d) ? part[t - d] : 0;
-    const int64_t w = (t >= d) ? spart[t - d] : 0;
-    __syncthreads();
-    part[t] += v;
-    spart[t] += w;
-    __syncthreads();
-  }
-  int64_t acc = part[t] - s;
-  for (int i = a; i < e; ++i) {
-    off[i] = acc;
-    acc += cnt[i];
-  }
-  if (t == 1023) {
-    off[nsegs] = part[1023];
-    status[ST_NLINKS] = (int32_t)min(part[1023], (int64_t)0x7fffffff);
-    status[ST_NSOLID] = (int32_t)min(spart[1023], (int64_t)0x7fffffff);
-    if (part[1023] > cap) atomicAdd(&status[ST_LINK_OVERFLOW], 1);
-  }
-}
-
-__device__ void fill_find_segment(int b, const FillArgs& fa, int nseg, int32_t* __restrict__ status);
-
-// Second half of beads_links: expand each segment's (node, direction bits)
-// into links at the segment's offset, in (node, direction) order, with the
-// wall fraction of every link (partlib.f90:1013-1024), one link per lane and
-// the node geometry rebuilt exactly as the scan saw it.  Blocks past the link
-// segments run the first pass of beads_filling (the new map is complete at
-// this point).
-__device__ __forceinline__ void links_expand_body(int b_, const double* __restrict__ ypglb, int np, int nseg, int seg_cap, PGeom G,
-                   const uint32_t* __restrict__ sh_node, const uint32_t* __restrict__ sh_hits,
-                   const int32_t* __restrict__ sh_cnt, const int64_t* __restrict__ off, int64_t cap,
-                   uint32_t* __restrict__ lk_node, uint8_t* __restrict__ lk_dir,
-                   double* __restrict__ lk_alpha, int32_t* __restrict__ status, int nsegs,
-                   FillArgs fa, const uint32_t* __restrict__ mask, uint64_t* __restrict__ ct_list,
-                   int32_t* __restrict__ ct_count) {
-  __shared__ BoxInfo B;
-  __shared__ int sh[PB / 64];
-  const int b = b_;
-  if (b >= nsegs) {
-    fill_find_segment(b - nsegs, fa, nseg, status);
-    return;
-  }
-  const int p = (int)div_by((uint32_t)b, G.dseg);
-  if (p >= np) return;
-  box_info(ypglb, p, G, B);
-  if (!B.ok) return;
-  const int nsh = sh_cnt[b];
-  const uint32_t* shn = sh_node + (size_t)b * seg_cap;
-  const uint32_t* shh = sh_hits + (size_t)b * seg_cap;
-  int64_t base = off[b];
-  for (int e0 = 0; e0 < nsh; e0 += PB) {
-    const int e = e0 + (int)threadIdx.x;
-    const bool act = e < nsh;
-    uint32_t hits = act ? shh[e] : 0u;
-    const uint32_t n = act ? shn[e] : 0u;
     int tot;
-    const int excl = block_exclusive_scan(__popc(hits), sh, tot);
-    int64_t w = base + excl;
+    int at = block_exclusive_scan(__popc(hits), sh, tot);
     while (hits) {
       const int q = __ffs(hits) - 1;
       hits &= hits - 1;
-      if (w < cap) {
-        lk_node[w] = n;
-        lk_dir[w] = (uint8_t)q;
+      if (at < kPassLinks) packed[at] = (uint32_t)e | ((uint32_t)q << 24);
+      ++at;
+    }
+    __syncthreads();
+    tot = min(tot, kPassLinks);
+    for (int l = (int)threadIdx.x; l < tot; l += PB) {
+      const uint32_t pk = packed[l];
+      const uint32_t from = shell[pk & 0xffffffu];
+      const int q = (int)(pk >> 24);
+      const SegRow w = rows[from >> 8];
+      LinkGeom L;
+      int iw;
+      node_geom(B, G, w, B.ax.lo + (int)(from & 255u), iw, L);
+      double xx1, yy1, zz1, rr1;
+      link_end(L, iw, w.jw, w.kw, q, xx1, yy1, zz1, rr1);
+      const double alpha = link_alpha(L, xx1, yy1, zz1, rr1, G.r2);
+      if (alpha < 0.0 || alpha > 1.0) ++alpha_bad;
+      if (nl + l < lk.cap) {
+        lk.node[slot + nl + l] = w.n0 + (uint32_t)iw;
+        lk.dir[slot + nl + l] = (uint8_t)q;
+        lk.alpha[slot + nl + l] = alpha;
       }
-      ++w;
     }
-    base += tot;
+    nl += tot;
+    __syncthreads();
   }
-  __syncthreads();   // the segment's links, written above by this block, are read below
-  const int64_t a = off[b], e = min(off[b + 1], cap);
-  int alpha_bad = 0;
-  for (int64_t l = a + threadIdx.x; l < e; l += PB) {
-    const uint32_t n = lk_node[l];
-    const int q = lk_dir[l];
-    const uint32_t rw = div_by(n, G.dx);
-    const int iw = (int)(n - rw * (uint32_t)G.nx);
-    const int kw = (int)div_by(rw, G.dy), jw = (int)rw - kw * G.ny;
-    LinkGeom L;
-    node_geom(B, G, iw, jw, kw, L);
-    double xx1, yy1, zz1, rr1;
-    link_hit(L, iw, jw, kw, q, G.r2, xx1, yy1, zz1, rr1);
-    const double alpha = link_alpha(L, xx1, yy1, zz1, rr1, G.r2);
-    if (alpha < 0.0 || alpha > 1.0) ++alpha_bad;
-    lk_alpha[l] = alpha;
-    if (bit_at(mask, n)) {   // the node is solid for another sphere: a contact link
-      const int slot = atomicAdd(ct_count, 1);
-      if (slot < cap) ct_list[slot] = ((uint64_t)(uint32_t)p << 40) | (uint64_t)l;
-    }
+  if (threadIdx.x == 0) {
+    lk.cnt[b] = min(nl, lk.cap);
+    sol_cnt[b] = min(nsol, seg_cap);
+    if (nl > lk.cap) atomicAdd(&status[ST_LINK_OVERFLOW], 1);
   }
   if (alpha_bad) atomicAdd(&status[ST_ALPHA_FAULT], alpha_bad);
 }
 
+// Links and solid nodes of the current build (status words read on demand).
+__global__ void __launch_bounds__(1024)
+    k_link_totals(const int32_t* __restrict__ cnt, const int32_t* __restrict__ scnt, int nsegs,
+                  int32_t* __restrict__ status) {
+  __shared__ unsigned long long sum[2];
+  if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned long long a = 0, b = 0;
+  for (int i = threadIdx.x; i < nsegs; i += 1024) {
+    a += (unsigned long long)cnt[i];
+    b += (unsigned long long)scnt[i];
+  }
+  atomicAdd(&sum[0], a);
+  atomicAdd(&sum[1], b);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    status[ST_NLINKS] = (int32_t)min(sum[0], 0x7fffffffull);
+    status[ST_NSOLID] = (int32_t)min(sum[1], 0x7fffffffull);
+  }
+}
+
+// Lists the contact links of one segment: links whose node is solid for
+// another sphere in the (now complete) map.
+__device__ __forceinline__ void list_contacts(int b, const ContactArgs& a) {
+  const int cnt = a.lk.cnt[b];
+  const int64_t slot = (int64_t)b * a.lk.cap;
+  for (int l = (int)threadIdx.x; l < cnt; l += PB) {
+    if (!bit_at(a.mask, a.lk.node[slot + l])) continue;
+    const int at = atomicAdd(a.ct_count, 1);
+    if (at < a.ct_cap) a.ct_list[at] = ((uint64_t)(uint32_t)div_by((uint32_t)b, a.dseg) << 40) | (uint64_t)(slot + l);
+  }
+}
+__global__ void __launch_bounds__(PB) k_contacts(ContactArgs a) { list_contacts((int)blockIdx.x, a); }
 
 // beads_lubforce (partlib.f90:2211-2292): one workgroup sums the pair forces
 // of particle a; each pair is evaluated as the reference does, from the lower
@@ -918,7 +897,7 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
   __shared__ int changed;
   const T* A = (const T*)a.A;
   const Grid& g = a.g;
-  const int64_t total = min((int64_t)*a.ct_count, a.cap);
+  const int64_t total = min((int64_t)*a.ct_count, a.ct_cap);
   if (total > a.ord_cap) {
     if (threadIdx.x == 0) atomicAdd(&a.status[ST_ORDER_CAP], 1);
     return;
@@ -930,10 +909,11 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
     OrderEntry o;
     o.dep[0] = o.dep[1] = -1;
     o.val[0] = o.val[1] = o.f9 = o.ff1 = 0.0;
-    const uint32_t n = l < a.cap ? a.lk_node[l] : 0u;
-    const int q = l < a.cap ? a.lk_dir[l] : 0;
-    if (p < a.np && l < a.cap && n < g.ncell && q >= 1 && q < NPOP) {
-      const double alpha = a.lk_alpha[l];
+    const bool in = p < a.np && l < (int64_t)a.nsegs * a.lk.cap;
+    const uint32_t n = in ? a.lk.node[l] : 0u;
+    const int q = in ? a.lk.dir[l] : 0;
+    if (in && n < g.ncell && q >= 1 && q < NPOP) {
+      const double alpha = a.lk.alpha[l];
       double ff1, f9, xx0, yy0, zz0;
       link_bounce<T>(A, g, a.G, a.mask, n, q, alpha, a.ypglb[3 * p], a.ypglb[3 * p + 1],
                      a.ypglb[3 * p + 2], a.wp[3 * p], a.wp[3 * p + 1], a.wp[3 * p + 2], a.omgp[3 * p],
@@ -951,29 +931,31 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
         const uint32_t nw = (uint32_t)wrap1(xw, g.nx) + (uint32_t)g.nx * ((uint32_t)yw + (uint32_t)g.ny * (uint32_t)zw);
         if (nw > n) continue;   // the loop runs the writer later
         const int qw = s == 0 ? opp(q) : q;
-        const int64_t lo = a.off[(int64_t)own * a.nseg];
-        const int64_t hi = min(a.off[(int64_t)(own + 1) * a.nseg], a.cap);
-        // the first match, kOrderBatch independent loads per round trip
+        // the owner's link (a writer is listed once), kOrderBatch independent
+        // loads per round trip
         int64_t lw = -1;
-        for (int64_t k0 = lo; k0 < hi && lw < 0; k0 += kOrderBatch) {
-          uint32_t nn[kOrderBatch];
-          int dd[kOrderBatch];
+        for (int sg2 = own * a.nseg; sg2 < (own + 1) * a.nseg && lw < 0; ++sg2) {
+          const int64_t lo = (int64_t)sg2 * a.lk.cap, hi = lo + a.lk.cnt[sg2];
+          for (int64_t k0 = lo; k0 < hi && lw < 0; k0 += kOrderBatch) {
+            uint32_t nn[kOrderBatch];
+            int dd[kOrderBatch];
 #pragma unroll
-          for (int j = 0; j < kOrderBatch; ++j) {
-            const bool in = k0 + j < hi;
-            nn[j] = in ? a.lk_node[k0 + j] : ~0u;
-            dd[j] = in ? (int)a.lk_dir[k0 + j] : -1;
+            for (int j = 0; j < kOrderBatch; ++j) {
+              const bool here = k0 + j < hi;
+              nn[j] = here ? a.lk.node[k0 + j] : ~0u;
+              dd[j] = here ? (int)a.lk.dir[k0 + j] : -1;
+            }
+#pragma unroll
+            for (int j = 0; j < kOrderBatch; ++j)
+              if (lw < 0 && nn[j] == nw && dd[j] == qw) lw = k0 + j;
           }
-#pragma unroll
-          for (int j = 0; j < kOrderBatch; ++j)
-            if (lw < 0 && nn[j] == nw && dd[j] == qw) lw = k0 + j;
         }
         if (lw < 0) continue;
         if (bit_at(a.mask, nw)) {
           o.dep[s] = lw | kOrderContact;
         } else {
           double wf1, wf9, wx, wy, wz;
-          link_bounce<T>(A, g, a.G, a.mask, nw, qw, a.lk_alpha[lw], a.ypglb[3 * own],
+          link_bounce<T>(A, g, a.G, a.mask, nw, qw, a.lk.alpha[lw], a.ypglb[3 * own],
                          a.ypglb[3 * own + 1], a.ypglb[3 * own + 2], a.wp[3 * own], a.wp[3 * own + 1],
                          a.wp[3 * own + 2], a.omgp[3 * own], a.omgp[3 * own + 1], a.omgp[3 * own + 2],
                          a.ww1, a.ww2, true, wf1, wf9, wx, wy, wz);
@@ -1000,7 +982,7 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
         v[s] = d < 0 ? 0.0 : ((d & kOrderContact) ? (double)(T)a.lk_out[d & ~kOrderContact].x : o.val[s]);
       }
       double ff1, f9, xx0, yy0, zz0;
-      link_bounce<T, true>(A, g, a.G, a.mask, a.lk_node[l], a.lk_dir[l], a.lk_alpha[l], a.ypglb[3 * p],
+      link_bounce<T, true>(A, g, a.G, a.mask, a.lk.node[l], a.lk.dir[l], a.lk.alpha[l], a.ypglb[3 * p],
                            a.ypglb[3 * p + 1], a.ypglb[3 * p + 2], a.wp[3 * p], a.wp[3 * p + 1],
                            a.wp[3 * p + 2], a.omgp[3 * p], a.omgp[3 * p + 1], a.omgp[3 * p + 2],
                            a.ww1, a.ww2, true, ff1, f9, xx0, yy0, zz0, o.dep[0] >= 0, v[0],
@@ -1054,17 +1036,17 @@ __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
   }
   const int nblk = a.nct;
   const T* A = (const T*)a.A;
-  const int64_t total = min((int64_t)*a.ct_count, a.cap);
+  const int64_t total = min((int64_t)*a.ct_count, a.ct_cap);
   for (int64_t e = (int64_t)b_ * PB + threadIdx.x; e < total; e += (int64_t)nblk * PB) {
     const uint64_t ent = a.ct_list[e];
     const int p = (int)(ent >> 40);
     const int64_t l = (int64_t)(ent & ((1ull << 40) - 1));
-    if (p >= a.np || l >= a.cap) continue;   // never true for a consistent list
-    const uint32_t n = a.lk_node[l];
-    const int q = a.lk_dir[l];
+    if (p >= a.np || l >= (int64_t)a.nsegs * a.lk.cap) continue;   // never true for a consistent list
+    const uint32_t n = a.lk.node[l];
+    const int q = a.lk.dir[l];
     if (n >= a.g.ncell || q < 1 || q >= NPOP) continue;
     double ff1 = 0.0, f9 = 0.0, xx0, yy0, zz0;
-    link_bounce<T>(A, a.g, a.G, a.mask, n, q, a.lk_alpha[l], a.ypglb[3 * p], a.ypglb[3 * p + 1],
+    link_bounce<T>(A, a.g, a.G, a.mask, n, q, a.lk.alpha[l], a.ypglb[3 * p], a.ypglb[3 * p + 1],
                    a.ypglb[3 * p + 2], a.wp[3 * p], a.wp[3 * p + 1], a.wp[3 * p + 2], a.omgp[3 * p],
                    a.omgp[3 * p + 1], a.omgp[3 * p + 2], a.ww1, a.ww2, true, ff1, f9, xx0, yy0, zz0);
     a.lk_out[l] = make_double2(f9, ff1);
@@ -1096,7 +1078,7 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   }
   const int b = a.split == 1 ? u : u / a.split, h = u - b * a.split;
   const int p = (int)div_by((uint32_t)b, a.G.dseg);
-  const int64_t s0 = a.off[b], s1 = min(a.off[b + 1], a.cap);
+  const int64_t s0 = (int64_t)b * a.lk.cap, s1 = s0 + a.lk.cnt[b];
   const int64_t per = (max(s1 - s0, (int64_t)0) + a.split - 1) / a.split;
   const int64_t l0 = s0 + h * per;
   const int64_t e = min(s1, l0 + per);
@@ -1106,9 +1088,9 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   double acc[6] = {0, 0, 0, 0, 0, 0};
   int contact = 0;
   for (int64_t l = l0 + threadIdx.x; l < e; l += PB) {
-    const uint32_t n = a.lk_node[l];
-    const int q = a.lk_dir[l];
-    const double alpha = a.lk_alpha[l];
+    const uint32_t n = a.lk.node[l];
+    const int q = a.lk.dir[l];
+    const double alpha = a.lk.alpha[l];
     if (n >= g.ncell || q < 1 || q >= NPOP) continue;  // never true for a consistent list
     const bool cont = bit_at(a.mask, n);
     double ff1 = 0.0, f9 = 0.0, xx0, yy0, zz0;
@@ -1341,64 +1323,30 @@ __global__ void __launch_bounds__(PB)
 }
 
 
-// beads_filling, pass 1 (partlib.f90:2846-2849): the nodes that were solid
-// for particle p in the previous map (p owns them there) and are fluid in the
-// new one, from the previous build's solid lists.  One workgroup per segment.
-__device__ void fill_find_segment(int b, const FillArgs& fa, int nseg, int32_t* __restrict__ status) {
-  const int p = b / nseg;
-  const int cnt = fa.sol_cnt_old[b];
-  const uint32_t* lst = fa.sol_old + (size_t)b * fa.seg_cap;
-  const int lane = threadIdx.x & 63;
-  int nfill = 0;
-  for (int e0 = 0; e0 < cnt; e0 += PB) {
-    const int e = e0 + (int)threadIdx.x;
-    const uint32_t n = e < cnt ? lst[e] : 0u;
-    // the new map's bit first: nearly every node stays solid, and only the
-    // uncovered ones need the owner test (a node of several spheres is
-    // listed once, by its owner)
-    const bool fill = e < cnt && !bit_at(fa.mask_new, n) && fa.isn_old[n] == p + 1;
-    // one atomic per wavefront for the list slots
-    const uint64_t bal = __ballot(fill);
-    if (bal == 0ull) continue;
-    const int leader = __ffsll((unsigned long long)bal) - 1;
-    int slot0 = 0;
-    if (lane == leader) slot0 = atomicAdd(fa.count, __popcll(bal));
-    slot0 = __builtin_amdgcn_readlane(slot0, leader);
-    if (fill) {
-      const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-      const int slot = slot0 + __popcll(bal & below);
-      if (slot < fa.cap) fa.list[slot] = ((uint64_t)(uint32_t)p << 32) | n;
-      ++nfill;
-    }
-  }
-  if (nfill) atomicAdd(&status[ST_REFILL], nfill);
-}
-
-__global__ void __launch_bounds__(PB)
-    k_fill_find(FillArgs fa, int nseg, int32_t* __restrict__ status) {
-  fill_find_segment(blockIdx.x, fa, nseg, status);
-}
-
-// beads_filling, pass 2 (partlib.f90:2851-3089): one wavefront per listed
-// node; lane l examines neighbour l+1 (fluid in both maps?  its density; the
-// non-equilibrium part if it lies along the back-traced normal), then lane i
+// beads_filling for one segment of the previous build (partlib.f90:2846-3089).
+// First the nodes that were solid for particle p in the previous map (p owns
+// them there) and are fluid in the new one, from the previous build's solid
+// list, kFillPass listed entries at a time; then one wavefront per such node: lane
+// l examines neighbour l+1 (fluid in both maps?  its density; the
+// non-equilibrium part if it lies along the back-traced normal), and lane i
 // writes population i of the node: equilibrium at the rigid-body velocity
 // (new w, omega; old centre) and the neighbours' mean density, plus the
-// non-equilibrium part.  Written into the pull sources of the node.
+// non-equilibrium part.  Written into the pull sources of the node.  The
+// neighbours read are fluid in both maps, so no refilled node is read and the
+// order of the refills does not matter.  Bound: two rounds of dependent loads
+// (list, new map), then two more for the few nodes uncovered.
+constexpr int kFillPass = 4 * PB;
 template <typename T, bool WALLS>
-__device__ __forceinline__ void fill_apply_body(int b_, T* __restrict__ A, Grid g, FillArgs fa, int nblk) {
+__device__ __forceinline__ void refill_nodes(const uint32_t* todo, int total, int id, T* __restrict__ A,
+                                             const Grid& g, const FillArgs& fa) {
   __shared__ double fneq[4][NPOP];
   __shared__ double srho[4][NPOP];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t nwaves = (int64_t)nblk * 4;
-  const int64_t total = min((int64_t)*fa.count, fa.cap);
   // the trip count is the same for every wavefront of the block (barriers inside)
-  for (int64_t base = (int64_t)b_ * 4; base < total; base += nwaves) {
-    const int64_t e = base + w;
+  for (int base = 0; base < total; base += 4) {
+    const int e = base + w;
     const bool active = e < total;
-    const uint64_t ent = active ? fa.list[e] : 0ull;
-    const int id = (int)(ent >> 32);
-    const uint32_t n = (uint32_t)(ent & 0xffffffffu);
+    const uint32_t n = active ? todo[e] : 0u;
     int i, j, k;
     uint32_t row;
     node_coords(n, g, i, j, k, row);
@@ -1479,6 +1427,39 @@ __device__ __forceinline__ void fill_apply_body(int b_, T* __restrict__ A, Grid 
   }
 }
 
+template <typename T, bool WALLS>
+__device__ __forceinline__ void fill_segment(int b, T* __restrict__ A, const Grid& g, const FillArgs& fa, FastDiv dseg) {
+  __shared__ uint32_t todo[kFillPass];
+  __shared__ int ntodo;
+  const int id = (int)div_by((uint32_t)b, dseg);
+  const int cnt = fa.sol_cnt_old[b];
+  const uint32_t* lst = fa.sol_old + (size_t)b * fa.seg_cap;
+  for (int e0 = 0; e0 < cnt; e0 += kFillPass) {
+    __syncthreads();   // the previous pass's list has been refilled
+    if (threadIdx.x == 0) ntodo = 0;
+    __syncthreads();
+    constexpr int kEach = kFillPass / PB;
+    uint32_t cand[kEach];
+    bool open[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+      const int e = e0 + k * PB + (int)threadIdx.x;
+      cand[k] = e < cnt ? lst[e] : ~0u;
+    }
+    // the new map's bit first: nearly every node stays solid
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) open[k] = cand[k] != ~0u && !bit_at(fa.mask_new, cand[k]);
+    // (a node of several spheres is refilled by its owner)
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+      if (open[k] && fa.isn_old[cand[k]] == id + 1) todo[atomicAdd(&ntodo, 1)] = cand[k];
+    __syncthreads();
+    const int total = ntodo;
+    if (threadIdx.x == 0 && total) atomicAdd(&fa.status[ST_REFILL], total);
+    refill_nodes<T, WALLS>(todo, total, id, A, g, fa);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Launch forms of the step kernels.  Each kernel body takes its block index;
 // k_* launches one box (arguments by value), kb_* one grid over several boxes
@@ -1493,119 +1474,14 @@ __device__ __forceinline__ int case_of(const int* __restrict__ off, int nc, int 
   return lo;
 }
 
-// 8 waves per SIMD (the compiler fits the scan in 64 VGPRs without spills):
-// a box of a few hundred spheres then runs its segments in one round
-__global__ void __launch_bounds__(PB) __attribute__((amdgpu_waves_per_eu(8))) k_links_scan(ScanArgs a) {
-  links_scan_body((int)blockIdx.x, a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.isn, a.mask, a.sol_list, a.sol_cnt, a.sh_node, a.sh_hits, a.sh_cnt, a.lk_cnt, a.ovl, a.istep, a.status, a.cells);
+__global__ void __launch_bounds__(PB) k_links_scan(ScanArgs a) {
+  links_scan_body((int)blockIdx.x, a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.isn, a.mask, a.sol_list, a.sol_cnt, a.lk, a.ct_count, a.ovl, a.istep, a.status, a.cells);
 }
-__global__ void __launch_bounds__(PB) __attribute__((amdgpu_waves_per_eu(8)))
+__global__ void __launch_bounds__(PB)
     kb_links_scan(const ScanArgs* __restrict__ t, const int* __restrict__ off, int nc) {
   const int c = case_of(off, nc, (int)blockIdx.x);
   const ScanArgs a = t[c];
-  links_scan_body((int)blockIdx.x - off[c], a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.isn, a.mask, a.sol_list, a.sol_cnt, a.sh_node, a.sh_hits, a.sh_cnt, a.lk_cnt, a.ovl, a.istep, a.status, a.cells);
-}
-
-// The same scan over many segments, in two grids of kScanChunk-segment
-// chunks: each chunk's sums, then each chunk scans itself after adding the
-// chunks before it.  Integer sums: the result equals the one-block scan.
-constexpr int kScanPer = kScanChunk / PB;
-__global__ void __launch_bounds__(PB) k_count_partials(ScanCountArgs a) {
-  __shared__ int sh[PB / 64];
-  const int b = blockIdx.x;
-  int s = 0, ss = 0;
-  for (int k = 0; k < kScanPer; ++k) {
-    const int i = b * kScanChunk + k * PB + (int)threadIdx.x;
-    if (i < a.nsegs) {
-      s += a.cnt[i];
-      ss += a.scnt[i];
-    }
-  }
-  int t1, t2;
-  block_exclusive_scan(s, sh, t1);
-  block_exclusive_scan(ss, sh, t2);
-  if (threadIdx.x == 0) {
-    a.part[2 * b] = t1;
-    a.part[2 * b + 1] = t2;
-  }
-}
-
-__global__ void __launch_bounds__(PB) k_count_offsets(ScanCountArgs a) {
-  __shared__ int sh[PB / 64];
-  __shared__ int64_t red[2][PB];
-  const int b = blockIdx.x;
-  if (b == 0 && threadIdx.x == 0) {
-    *a.fill_count = 0;   // the next beads_filling starts an empty list
-    *a.ct_count = 0;     // the expansion lists this rebuild's contact links
-  }
-  // chunks before this one (and all chunks, for the totals)
-  const int nb = gridDim.x;
-  int64_t before = 0, tot = 0, stot = 0;
-  for (int k = threadIdx.x; k < nb; k += PB) {
-    const int64_t v = a.part[2 * k];
-    tot += v;
-    stot += a.part[2 * k + 1];
-    if (k < b) before += v;
-  }
-  red[0][threadIdx.x] = before;
-  red[1][threadIdx.x] = tot;
-  __syncthreads();
-  for (int o = PB / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + o];
-      red[1][threadIdx.x] += red[1][threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  const int64_t base = red[0][0], total = red[1][0];
-  __syncthreads();
-  // this chunk: thread t owns segments [t * kScanPer, (t + 1) * kScanPer)
-  const int i0 = b * kScanChunk + (int)threadIdx.x * kScanPer;
-  int s = 0;
-  for (int k = 0; k < kScanPer; ++k)
-    if (i0 + k < a.nsegs) s += a.cnt[i0 + k];
-  int ct;
-  int64_t acc = base + block_exclusive_scan(s, sh, ct);
-  for (int k = 0; k < kScanPer; ++k) {
-    if (i0 + k < a.nsegs) {
-      a.off[i0 + k] = acc;
-      acc += a.cnt[i0 + k];
-    }
-  }
-  if (b == nb - 1) {
-    // every chunk's solid count, by the same reduction
-    red[1][threadIdx.x] = stot;
-    __syncthreads();
-    for (int o = PB / 2; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) red[1][threadIdx.x] += red[1][threadIdx.x + o];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      a.off[a.nsegs] = total;
-      a.status[ST_NLINKS] = (int32_t)min(total, (int64_t)0x7fffffff);
-      a.status[ST_NSOLID] = (int32_t)min(red[1][0], (int64_t)0x7fffffff);
-      if (total > a.cap) atomicAdd(&a.status[ST_LINK_OVERFLOW], 1);
-    }
-  }
-}
-
-__global__ void __launch_bounds__(1024) k_scan_counts(ScanCountArgs a) {
-  scan_counts_body((int)blockIdx.x, a.cnt, a.scnt, a.nsegs, a.off, a.cap, a.status, a.fill_count, a.ct_count);
-}
-__global__ void __launch_bounds__(1024)
-    kb_scan_counts(const ScanCountArgs* __restrict__ t, const int* __restrict__ off, int nc) {
-  const int c = case_of(off, nc, (int)blockIdx.x);
-  const ScanCountArgs a = t[c];
-  scan_counts_body((int)blockIdx.x - off[c], a.cnt, a.scnt, a.nsegs, a.off, a.cap, a.status, a.fill_count, a.ct_count);
-}
-
-__global__ void __launch_bounds__(PB) k_links_expand(ExpandArgs a) {
-  links_expand_body((int)blockIdx.x, a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.sh_node, a.sh_hits, a.sh_cnt, a.off, a.cap, a.lk_node, a.lk_dir, a.lk_alpha, a.status, a.nsegs, a.fa, a.mask, a.ct_list, a.ct_count);
-}
-__global__ void __launch_bounds__(PB)
-    kb_links_expand(const ExpandArgs* __restrict__ t, const int* __restrict__ off, int nc) {
-  const int c = case_of(off, nc, (int)blockIdx.x);
-  const ExpandArgs a = t[c];
-  links_expand_body((int)blockIdx.x - off[c], a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.sh_node, a.sh_hits, a.sh_cnt, a.off, a.cap, a.lk_node, a.lk_dir, a.lk_alpha, a.status, a.nsegs, a.fa, a.mask, a.ct_list, a.ct_count);
+  links_scan_body((int)blockIdx.x - off[c], a.ypglb, a.np, a.nseg, a.seg_cap, a.G, a.isn, a.mask, a.sol_list, a.sol_cnt, a.lk, a.ct_count, a.ovl, a.istep, a.status, a.cells);
 }
 
 template <typename T>
@@ -1654,24 +1530,36 @@ __global__ void __launch_bounds__(kMoveBlock)
   move_body((int)blockIdx.x - off[c], a.m, a.np, a.first, a.wrap, a.G, a.status, a.seg_ft, a.nseg, a.cells);
 }
 
-// 4 waves per SIMD (at most 128 VGPRs): with the 1024 blocks of the grid
-// every wavefront is resident at once
+// The refill of the previous build's segments, the contact links of the new
+// build's and, in blocks past those, the next step's forcing table.  4 waves
+// per SIMD (at most 128 VGPRs; 5 or more spill: 24 to 31 us with 900 spheres of
+// radius 4).  The search in a grid of its own that lists the nodes for a refill
+// grid was no faster but with 15,000 segments (12 + 12 us against 24 with 900
+// spheres, 3.6 + 9.2 against 9.8 with 8, 58 + 26 against 105 with 2500).
 template <typename T, bool WALLS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-    k_fill_apply(FillApplyArgs a, TableJob tj) {
-  if ((int)blockIdx.x >= a.nblk) {   // blocks past the refill: the next step's forcing table
-    force_table_block(tj.M, tj.phy, tj.phz, tj.ny, tj.nz, tj.G, blockIdx.x - (uint32_t)a.nblk);
-    return;
+__device__ __forceinline__ bool fill_block(int b, const FillKArgs& a) {
+  if (b < a.nfill) {
+    fill_segment<T, WALLS>(b, (T*)a.A, a.g, a.fa, a.ct.dseg);
+  } else if (b < a.nfill + a.nct) {
+    list_contacts(b - a.nfill, a.ct);
+  } else {
+    return false;
   }
-  fill_apply_body<T, WALLS>((int)blockIdx.x, (T*)a.A, a.g, a.fa, a.nblk);
+  return true;
 }
-static_assert(sizeof(FillApplyArgs) + sizeof(TableJob) <= 4096, "refill kernel arguments over 4 KB");
 template <typename T, bool WALLS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-    kb_fill_apply(const FillApplyArgs* __restrict__ t, const int* __restrict__ off, int nc) {
+    k_fill(FillKArgs a, TableJob tj) {
+  if (!fill_block<T, WALLS>((int)blockIdx.x, a))
+    force_table_block(tj.M, tj.phy, tj.phz, tj.ny, tj.nz, tj.G, blockIdx.x - (uint32_t)(a.nfill + a.nct));
+}
+static_assert(sizeof(FillKArgs) + sizeof(TableJob) <= 4096, "refill kernel arguments over 4 KB");
+template <typename T, bool WALLS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+    kb_fill(const FillKArgs* __restrict__ t, const int* __restrict__ off, int nc) {
   const int c = case_of(off, nc, (int)blockIdx.x);
-  const FillApplyArgs a = t[c];
-  fill_apply_body<T, WALLS>((int)blockIdx.x - off[c], (T*)a.A, a.g, a.fa, a.nblk);
+  const FillKArgs a = t[c];
+  fill_block<T, WALLS>((int)blockIdx.x - off[c], a);
 }
 
 // trilinear velocity at the particle centres (initpartvel,
@@ -1711,19 +1599,17 @@ __global__ void k_maps_dense(Grid g, const int32_t* __restrict__ isn, const uint
   is[n] = (isn != nullptr && isn[n] > 0) ? isn[n] : -1;
 }
 
-__global__ void k_links_dense(Grid g, int nseg, const int64_t* __restrict__ off, int64_t cap,
-                              const uint32_t* __restrict__ lk_node, const uint8_t* __restrict__ lk_dir,
-                              const double* __restrict__ lk_alpha, int32_t* __restrict__ ilink,
+__global__ void k_links_dense(Grid g, FastDiv dseg, LinkSlots lk, int32_t* __restrict__ ilink,
                               int32_t* __restrict__ mlink, double* __restrict__ alink) {
   const int b = blockIdx.x;
-  const int p = b / nseg;
-  const int64_t a = off[b], e = min(off[b + 1], cap);
+  const int p = (int)div_by((uint32_t)b, dseg);
+  const int64_t a = (int64_t)b * lk.cap, e = a + lk.cnt[b];
   for (int64_t l = a + threadIdx.x; l < e; l += blockDim.x) {
-    if (lk_node[l] >= g.ncell || lk_dir[l] < 1 || lk_dir[l] >= NPOP) continue;
-    const uint64_t d = (uint64_t)(lk_dir[l] - 1) + 18ull * lk_node[l];
+    if (lk.node[l] >= g.ncell || lk.dir[l] < 1 || lk.dir[l] >= NPOP) continue;
+    const uint64_t d = (uint64_t)(lk.dir[l] - 1) + 18ull * lk.node[l];
     ilink[d] = 1;
     mlink[d] = p + 1;
-    alink[d] = lk_alpha[l];
+    alink[d] = lk.alpha[l];
   }
 }
 
@@ -1740,8 +1626,6 @@ static PGeom pgeom(const Ctx& c) {
   G.rlink2 = (c.p.rad + 1.5) * (c.p.rad + 1.5);
   G.rsolid2 = (c.p.rad + 0.5) * (c.p.rad + 0.5);
   G.slab = c.pt.slab;
-  G.dx = c.g.dx;
-  G.dy = c.g.dy;
   G.dseg = fast_div((uint32_t)c.pt.nseg);
   return G;
 }
@@ -1761,13 +1645,28 @@ int segment_capacity(double rad, int slab) {
   return slab * maxcnt * maxcnt;
 }
 
+// Links a segment can hold: a lattice line along a direction enters a sphere
+// once, so a direction within the planes has at most as many links as lines
+// meet the disc of each plane (2r + 1 along an axis, 2 sqrt(2) r + 1 along a
+// diagonal), and a direction across the planes as many as lines meet the sphere
+// or the part of its surface in the segment, whichever is fewer (a band of
+// height h has the projected area pi r h, a cap 2 pi r h; sqrt(2) lines per unit
+// area along a diagonal), each with a margin of a node.  1.9 to 3 times the
+// largest count met over radii from 2 to 27 and random centres.
+int segment_links(double rad, int slab) {
+  const double r = rad + 1.0, disc = M_PI * r * r, h = slab + 1.0;
+  const double in_plane = slab * (4.0 * (2.0 * r) + 4.0 * (2.0 * sqrt(2.0) * rad + 2.0));
+  const double across = 2.0 * std::min(disc, 2.0 * M_PI * r * h) + 8.0 * sqrt(2.0) * std::min(disc, M_PI * r * h);
+  return (int)ceil(in_plane + across) + 64;
+}
+
 // Planes per segment.  8 when the spheres are many (the segment grids of the
 // link rebuild and the bounce-back still fill the GPU several times over
 // with half as many, twice as large workgroups: at 1024^3 with 20,000
 // spheres of radius 6 the three kernels take 0.5 ms less per step), else 4
 // (300 spheres of radius 8 at 256^3 need the parallelism: 0.06 ms more per
 // step with 8).  8 also needs at most PB / 8 candidate rows per plane and
-// keeps the scan's shell list within 20 KB of LDS, so only for
+// keeps the scan's shell list within 10 KB of LDS, so only for
 // box_candidates <= 25 (rad <= 8).  MFC_SEG_PLANES=4 or 8 forces one (8 only
 // where it fits).
 constexpr int64_t kSlab8MinSegments = 8192;
@@ -1802,9 +1701,7 @@ static bool make_fill_args(Ctx& c, int old, int neu, FillArgs& fa) {
   fa.mask_new = P.mask[neu];
   fa.mask_old = P.mask[old];
   fa.rad = c.p.rad; fa.rho0 = c.p.rho0; fa.ww0 = c.p.ww0; fa.ww1 = c.p.ww1; fa.ww2 = c.p.ww2;
-  fa.list = P.fill_list;
-  fa.count = P.fill_count;
-  fa.cap = P.fill_cap;
+  fa.status = c.d_status;
   return true;
 }
 
@@ -1854,6 +1751,21 @@ static LubArgs lub_args(Ctx& c) {
   return L;
 }
 
+static LinkSlots link_slots(const Particles& P) {
+  return LinkSlots{P.lk_node, P.lk_dir, P.lk_alpha, P.lk_cnt, P.lk_seg};
+}
+
+static ContactArgs contact_args(const Particles& P) {
+  ContactArgs a;
+  a.lk = link_slots(P);
+  a.mask = P.mask[P.map_cur];
+  a.ct_list = P.ct_list;
+  a.ct_count = P.ct_count;
+  a.ct_cap = P.lk_cap;
+  a.dseg = fast_div((uint32_t)P.nseg);
+  return a;
+}
+
 // ---- argument builders: one box's arguments of each step kernel ------------
 // (used by the single-box launchers below and by the ensemble engine)
 
@@ -1862,35 +1774,14 @@ ScanArgs scan_args(Ctx& c, int target, int ovl, int istep) {
   ScanArgs a;
   a.ypglb = P.ypglb; a.np = P.np; a.nseg = P.nseg; a.seg_cap = P.seg_cap; a.G = pgeom(c);
   a.isn = P.isn[target]; a.mask = P.mask[target]; a.sol_list = P.sol_list[target];
-  a.sol_cnt = P.sol_cnt[target]; a.sh_node = P.sh_node; a.sh_hits = P.sh_hits; a.sh_cnt = P.sh_cnt;
-  a.lk_cnt = P.lk_cnt; a.ovl = ovl; a.istep = istep; a.status = c.d_status;
+  a.sol_cnt = P.sol_cnt[target]; a.lk = link_slots(P); a.ct_count = P.ct_count; a.ovl = ovl; a.istep = istep; a.status = c.d_status;
   a.cells = cell_args(c);
   return a;
 }
 
-ScanCountArgs count_args(Ctx& c, int target) {
-  Particles& P = c.pt;
-  ScanCountArgs a;
-  a.cnt = P.lk_cnt; a.scnt = P.sol_cnt[target]; a.nsegs = P.np * P.nseg; a.off = P.lk_off;
-  a.cap = P.lk_cap; a.status = c.d_status; a.fill_count = P.fill_count; a.ct_count = P.ct_count;
-  a.part = P.lk_part;
-  return a;
-}
-
-// with_find: the refill search (previous map P.map_old vs `target`) rides in
-// the same grid; *blocks gets the grid size
-ExpandArgs expand_args(Ctx& c, int target, bool with_find, int* blocks) {
-  Particles& P = c.pt;
-  ExpandArgs a;
-  a.ypglb = P.ypglb; a.np = P.np; a.nseg = P.nseg; a.seg_cap = P.seg_cap; a.G = pgeom(c);
-  a.sh_node = P.sh_node; a.sh_hits = P.sh_hits; a.sh_cnt = P.sh_cnt; a.off = P.lk_off; a.cap = P.lk_cap;
-  a.lk_node = P.lk_node; a.lk_dir = P.lk_dir; a.lk_alpha = P.lk_alpha; a.status = c.d_status;
-  a.nsegs = P.np * P.nseg;
-  a.mask = P.mask[target]; a.ct_list = P.ct_list; a.ct_count = P.ct_count;
-  a.fa = FillArgs{};
-  const int nfind = (with_find && make_fill_args(c, P.map_old, target, a.fa)) ? P.map_np[P.map_old] * P.nseg : 0;
-  *blocks = a.nsegs + nfind;
-  return a;
+size_t scan_lds(const Ctx& c) {
+  return (size_t)shell_bytes(c.pt.seg_cap) + packed_bytes(c.pt.seg_cap) +
+         sizeof(SegRow) * (size_t)(c.pt.slab * box_candidates(c.p.rad));
 }
 
 // fused: the lubrication forces ride in the same grid
@@ -1901,8 +1792,8 @@ BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blo
   Particles& P = c.pt;
   BounceArgs a;
   a.A = c.pop[c.cur]; a.g = c.g; a.G = pgeom(c); a.mask = P.mask[P.map_cur]; a.nseg = P.nseg;
-  a.off = P.lk_off; a.cap = P.lk_cap; a.lk_node = P.lk_node; a.lk_dir = P.lk_dir;
-  a.lk_alpha = P.lk_alpha; a.lk_out = P.lk_out; a.ct_list = P.ct_list; a.ct_count = P.ct_count;
+  a.lk = link_slots(P); a.lk_out = P.lk_out;
+  a.ct_list = P.ct_list; a.ct_count = P.ct_count; a.ct_cap = P.lk_cap;
   a.ypglb = P.ypglb; a.wp = P.wp; a.omgp = P.omgp;
   a.ww1 = c.p.ww1; a.ww2 = c.p.ww2; a.seg_ft = P.seg_ft; a.status = c.d_status;
   a.nsegs = P.np * P.nseg; a.np = P.np; a.lub = lub_args(c);
@@ -1948,12 +1839,19 @@ MoveKArgs move_args(Ctx& c, int first, int wrap, bool from_seg, int* blocks) {
   return a;
 }
 
-// false if there is nothing to refill
-bool fill_apply_args(Ctx& c, int nblk, FillApplyArgs& a) {
+// refill: beads_filling between the maps map_old and map_cur (no blocks if there
+// is nothing to refill); contacts: list the contact links of the current build
+FillKArgs fill_args(Ctx& c, bool refill, bool contacts, int* blocks) {
   Particles& P = c.pt;
-  if (!make_fill_args(c, P.map_old, P.map_cur, a.fa)) return false;
-  a.A = c.pop[c.cur]; a.g = c.g; a.nblk = nblk;
-  return true;
+  FillKArgs a;
+  a.fa = FillArgs{};
+  a.nfill = refill && make_fill_args(c, P.map_old, P.map_cur, a.fa) ? P.map_np[P.map_old] * P.nseg : 0;
+  a.nct = contacts ? P.np * P.nseg : 0;
+  a.ct = contact_args(P);
+  a.A = c.pop[c.cur];
+  a.g = c.g;
+  *blocks = a.nfill + a.nct;
+  return a;
 }
 
 // ---- far and near tiles of the overlapped step ----------------------------------
@@ -2113,30 +2011,32 @@ hipError_t launch_tiles(Ctx& c, TileLists& T) {
 }
 
 // ---- single-box launchers -------------------------------------------------------
-hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool with_find) {
+hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool defer_contacts) {
   Particles& P = c.pt;
   const int nsegs = P.np * P.nseg;
   hipError_t e = launch_map_clear(c, target);
   if (e != hipSuccess) return e;
   if (P.np <= 0) return hipGetLastError();
-  int nexp = 0;
   if (overlap_check) {
     e = ensure_cells(c);
     if (e != hipSuccess) return e;
   }
-  const ExpandArgs ea = expand_args(c, target, with_find, &nexp);
-  hipLaunchKernelGGL(k_links_scan, dim3(nsegs), dim3(PB), sizeof(uint32_t) * (size_t)P.seg_cap,
-                     c.stream, scan_args(c, target, overlap_check, istep));
-  if (nsegs > kScanChunk) {
-    const int nb = (nsegs + kScanChunk - 1) / kScanChunk;
-    const ScanCountArgs ca = count_args(c, target);
-    hipLaunchKernelGGL(k_count_partials, dim3(nb), dim3(PB), 0, c.stream, ca);
-    hipLaunchKernelGGL(k_count_offsets, dim3(nb), dim3(PB), 0, c.stream, ca);
-  } else {
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, c.stream, count_args(c, target));
+  hipLaunchKernelGGL(k_links_scan, dim3(nsegs), dim3(PB), scan_lds(c), c.stream,
+                     scan_args(c, target, overlap_check, istep));
+  if (!defer_contacts) {
+    ContactArgs ca = contact_args(P);
+    ca.mask = P.mask[target];
+    hipLaunchKernelGGL(k_contacts, dim3(nsegs), dim3(PB), 0, c.stream, ca);
   }
-  hipLaunchKernelGGL(k_links_expand, dim3(nexp), dim3(PB), 0, c.stream, ea);
   P.map_np[target] = P.np;
+  return hipGetLastError();
+}
+
+hipError_t launch_link_totals(Ctx& c) {
+  Particles& P = c.pt;
+  if (P.np <= 0 || P.map_np[P.map_cur] == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_link_totals, dim3(1), dim3(1024), 0, c.stream, P.lk_cnt, P.sol_cnt[P.map_cur],
+                     P.np * P.nseg, c.d_status);
   return hipGetLastError();
 }
 
@@ -2192,31 +2092,26 @@ hipError_t launch_redistribute(Ctx& c, int istep) {
   return hipGetLastError();
 }
 
-constexpr int kFillBlocks = 1024;
-
-hipError_t launch_filling(Ctx& c, bool find, const TableJob* job) {
-  Particles& P = c.pt;
-  FillApplyArgs a;
-  if (!fill_apply_args(c, kFillBlocks, a)) return job ? launch_force_table(c, job->slot, job->M) : hipSuccess;
-  if (find)
-    hipLaunchKernelGGL(k_fill_find, dim3(P.map_np[P.map_old] * P.nseg), dim3(PB), 0, c.stream, a.fa,
-                       P.nseg, c.d_status);
+hipError_t launch_filling(Ctx& c, bool contacts, const TableJob* job) {
+  int nb = 0;
+  const FillKArgs a = fill_args(c, true, contacts, &nb);
   TableJob tj;
   if (job)
     tj = *job;
   else
     tj.nblk = 0;
-  const dim3 grid(kFillBlocks + tj.nblk), blk(256);
+  const dim3 grid(nb + tj.nblk), blk(256);
+  if (grid.x == 0) return hipSuccess;
   if (c.prec == MFC_PREC_FP64) {
     if (c.g.walls_y)
-      hipLaunchKernelGGL((k_fill_apply<double, true>), grid, blk, 0, c.stream, a, tj);
+      hipLaunchKernelGGL((k_fill<double, true>), grid, blk, 0, c.stream, a, tj);
     else
-      hipLaunchKernelGGL((k_fill_apply<double, false>), grid, blk, 0, c.stream, a, tj);
+      hipLaunchKernelGGL((k_fill<double, false>), grid, blk, 0, c.stream, a, tj);
   } else {
     if (c.g.walls_y)
-      hipLaunchKernelGGL((k_fill_apply<float, true>), grid, blk, 0, c.stream, a, tj);
+      hipLaunchKernelGGL((k_fill<float, true>), grid, blk, 0, c.stream, a, tj);
     else
-      hipLaunchKernelGGL((k_fill_apply<float, false>), grid, blk, 0, c.stream, a, tj);
+      hipLaunchKernelGGL((k_fill<float, false>), grid, blk, 0, c.stream, a, tj);
   }
   return hipGetLastError();
 }
@@ -2239,8 +2134,8 @@ hipError_t launch_maps_to_host_layout(Ctx& c, int which, int32_t* ib, int32_t* i
 
 hipError_t launch_links_dense(Ctx& c, int32_t* ilink, int32_t* mlink, double* alink) {
   Particles& P = c.pt;
-  hipLaunchKernelGGL(k_links_dense, dim3(P.np * P.nseg), dim3(256), 0, c.stream, c.g, P.nseg, P.lk_off,
-                     P.lk_cap, P.lk_node, P.lk_dir, P.lk_alpha, ilink, mlink, alink);
+  hipLaunchKernelGGL(k_links_dense, dim3(P.np * P.nseg), dim3(256), 0, c.stream, c.g,
+                     fast_div((uint32_t)P.nseg), link_slots(P), ilink, mlink, alink);
   return hipGetLastError();
 }
 
@@ -2254,9 +2149,7 @@ size_t stage_arg_bytes(Stage st) {
     case SG_CONTACT: return sizeof(BounceArgs);
     case SG_MOVE: return sizeof(MoveKArgs);
     case SG_SCAN: return sizeof(ScanArgs);
-    case SG_COUNT: return sizeof(ScanCountArgs);
-    case SG_EXPAND: return sizeof(ExpandArgs);
-    case SG_FILL: return sizeof(FillApplyArgs);
+    case SG_FILL: return sizeof(FillKArgs);
   }
   return 0;
 }
@@ -2284,23 +2177,17 @@ hipError_t launch_batched(Stage st, int prec, int walls, const void* t, const in
     case SG_SCAN:
       hipLaunchKernelGGL(kb_links_scan, dim3(blocks), dim3(PB), lds, s, (const ScanArgs*)t, off, nc);
       break;
-    case SG_COUNT:
-      hipLaunchKernelGGL(kb_scan_counts, dim3(blocks), dim3(1024), 0, s, (const ScanCountArgs*)t, off, nc);
-      break;
-    case SG_EXPAND:
-      hipLaunchKernelGGL(kb_links_expand, dim3(blocks), dim3(PB), 0, s, (const ExpandArgs*)t, off, nc);
-      break;
     case SG_FILL:
       if (f64) {
         if (walls)
-          hipLaunchKernelGGL((kb_fill_apply<double, true>), dim3(blocks), dim3(256), 0, s, (const FillApplyArgs*)t, off, nc);
+          hipLaunchKernelGGL((kb_fill<double, true>), dim3(blocks), dim3(256), 0, s, (const FillKArgs*)t, off, nc);
         else
-          hipLaunchKernelGGL((kb_fill_apply<double, false>), dim3(blocks), dim3(256), 0, s, (const FillApplyArgs*)t, off, nc);
+          hipLaunchKernelGGL((kb_fill<double, false>), dim3(blocks), dim3(256), 0, s, (const FillKArgs*)t, off, nc);
       } else {
         if (walls)
-          hipLaunchKernelGGL((kb_fill_apply<float, true>), dim3(blocks), dim3(256), 0, s, (const FillApplyArgs*)t, off, nc);
+          hipLaunchKernelGGL((kb_fill<float, true>), dim3(blocks), dim3(256), 0, s, (const FillKArgs*)t, off, nc);
         else
-          hipLaunchKernelGGL((kb_fill_apply<float, false>), dim3(blocks), dim3(256), 0, s, (const FillApplyArgs*)t, off, nc);
+          hipLaunchKernelGGL((kb_fill<float, false>), dim3(blocks), dim3(256), 0, s, (const FillKArgs*)t, off, nc);
       }
       break;
   }

@@ -36,7 +36,7 @@ struct PGeom {
   double rsolid2;
   // z planes per segment (4 or 8; Particles::slab)
   int slab;
-  FastDiv dx, dy, dseg;   // division by nx, ny and the segments per particle
+  FastDiv dseg;   // division by the segments per particle
 };
 
 struct FillArgs {
@@ -47,9 +47,26 @@ struct FillArgs {
   const int32_t* sol_cnt_old;
   int seg_cap;
   double rad, rho0, ww0, ww1, ww2;
-  uint64_t* list;       // (particle << 32) | node of every node to refill
-  int32_t* count;       // list length (reset by k_scan_counts of the links pass)
-  int64_t cap;
+  int32_t* status;
+};
+
+// Boundary links: segment b's are the cnt[b] entries from b * cap on.
+struct LinkSlots {
+  uint32_t* node;
+  uint8_t* dir;
+  double* alpha;
+  int32_t* cnt;
+  int cap;
+};
+
+// Contact links (node solid for another sphere) of the current build.
+struct ContactArgs {
+  LinkSlots lk;
+  const uint32_t* mask;
+  uint64_t* ct_list;    // (particle << 40) | link
+  int32_t* ct_count;    // cleared by the links scan
+  int64_t ct_cap;
+  FastDiv dseg;
 };
 
 // Uniform cell grid of the particle pair searches (lubrication, overlap
@@ -86,48 +103,12 @@ struct ScanArgs {
   uint32_t* mask;
   uint32_t* sol_list;
   int32_t* sol_cnt;
-  uint32_t* sh_node;
-  uint32_t* sh_hits;
-  int32_t* sh_cnt;
-  int32_t* lk_cnt;
+  LinkSlots lk;
+  int32_t* ct_count;
   int ovl;
   int istep;
   int32_t* status;
   CellArgs cells;
-};
-
-struct ScanCountArgs {
-  const int32_t* cnt;
-  const int32_t* scnt;
-  int nsegs;
-  int64_t* off;
-  int64_t cap;
-  int32_t* status;
-  int32_t* fill_count;
-  int32_t* ct_count;
-  int64_t* part;          // per-chunk sums of the multi-block form (2 per chunk)
-};
-
-struct ExpandArgs {
-  const double* ypglb;
-  int np;
-  int nseg;
-  int seg_cap;
-  PGeom G;
-  const uint32_t* sh_node;
-  const uint32_t* sh_hits;
-  const int32_t* sh_cnt;
-  const int64_t* off;
-  int64_t cap;
-  uint32_t* lk_node;
-  uint8_t* lk_dir;
-  double* lk_alpha;
-  int32_t* status;
-  int nsegs;
-  FillArgs fa;
-  const uint32_t* mask;   // the map being built: links whose node is solid are contact links
-  uint64_t* ct_list;
-  int32_t* ct_count;
 };
 
 // Arguments of the bounce-back grid (link segments, then the map-clearing
@@ -139,14 +120,11 @@ struct BounceArgs {
   PGeom G;
   const uint32_t* mask;
   int nseg;
-  const int64_t* off;
-  int64_t cap;
-  const uint32_t* lk_node;
-  const uint8_t* lk_dir;
-  const double* lk_alpha;
+  LinkSlots lk;
   double2* lk_out;              // (f9, ff1) of the contact links
   const uint64_t* ct_list;      // contact links: (particle << 40) | link
   const int32_t* ct_count;
+  int64_t ct_cap;
   const double* ypglb;
   const double* wp;
   const double* omgp;
@@ -185,27 +163,29 @@ struct MoveKArgs {
   CellArgs cells;         // cnt non-null: (cleared) cells to enter the new centres in
 };
 
-struct FillApplyArgs {
+// Arguments of the refill grid: nfill blocks of beads_filling (segments of the
+// previous build), then nct blocks listing contact links.
+struct FillKArgs {
   void* A;
   Grid g;
   FillArgs fa;
-  int nblk;
+  ContactArgs ct;
+  int nfill, nct;
 };
 
 // ---- argument builders (fluid.hip, particles.hip) ----
 CollideArgs collide_args(Ctx& c);
 ScanArgs scan_args(Ctx& c, int target, int ovl, int istep);
-ScanCountArgs count_args(Ctx& c, int target);
-ExpandArgs expand_args(Ctx& c, int target, bool with_find, int* blocks);
+size_t scan_lds(const Ctx& c);   // dynamic LDS of the links scan
 // bb_blocks: the bounce-back grid; pre_blocks: the pre-pass grid (nct
 // contact blocks + lubrication)
 BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blocks);
 MoveKArgs move_args(Ctx& c, int first, int wrap, bool from_seg, int* blocks);
-bool fill_apply_args(Ctx& c, int nblk, FillApplyArgs& a);
+FillKArgs fill_args(Ctx& c, bool refill, bool contacts, int* blocks);
 
 // ---- launches over several boxes: t = device table of the stage's argument
 // blocks (one per box), off = device block offsets (nc + 1), `blocks` = off[nc]
-enum Stage { SG_CONTACT, SG_BOUNCE, SG_MOVE, SG_SCAN, SG_COUNT, SG_EXPAND, SG_FILL };
+enum Stage { SG_CONTACT, SG_BOUNCE, SG_MOVE, SG_SCAN, SG_FILL };
 hipError_t launch_batched(Stage st, int prec, int walls, const void* t, const int* off, int nc,
                           int blocks, size_t lds, hipStream_t s);
 // arr_any: some member's CollideArgs::arr is set

@@ -86,7 +86,7 @@ class BoxCase:
         """Device memory make_lattice allocates for the case: the sizes
         mfc_create and mfc_prt_init request (populations A/B, 19 values per
         node of padded rows each, forcing tables, moments, particle arrays, segment lists, link
-        pool, refill list, node maps), each rounded up to the allocator's
+        slots, node maps), each rounded up to the allocator's
         granularity (4 KiB below 1 MiB, 2 MiB above), plus 16 MiB for the
         runtime's per-context state.  An upper bound of the hipMemGetInfo
         difference around make_lattice (checked by the serving test)."""
@@ -102,12 +102,12 @@ class BoxCase:
             nseg, seg_cap = (maxcnt + 3) // 4, 4 * maxcnt * maxcnt
             nsegs = np_ * nseg
             nodes = nsegs * seg_cap
-            allocs += [4 * nsegs, 8 * (nsegs + 1), 16 * (nsegs // 4096 + 1)]
-            allocs += [4 * nodes, 4 * nsegs] * 2 + [4 * nodes, 4 * nodes, 4 * nsegs, 8 * 6 * nsegs * 4]
-            allocs += [8 * (math.ceil(4.0 / 3.0 * math.pi * (r + 1.0) ** 3) * np_ + 64), 4]
-            h = math.sqrt(3.0) / 2.0
-            ro, ri = r + math.sqrt(2.0) + h, max(0.0, r - h)
-            cap = (math.ceil(4.0 / 3.0 * math.pi * (ro ** 3 - ri ** 3)) * 9 + 64) * np_
+            allocs += [4 * nsegs, 8 * 6 * nsegs * 4] + [4 * nodes, 4 * nsegs] * 2
+            # links per segment of four planes (segment_links)
+            q, root2 = r + 1.0, math.sqrt(2.0)
+            disc = math.pi * q * q
+            cap = 4 * (8.0 * q + 4.0 * (2.0 * root2 * r + 2.0)) + 2.0 * min(disc, 10.0 * math.pi * q)
+            cap = (math.ceil(cap + 8.0 * root2 * min(disc, 5.0 * math.pi * q)) + 65) * nsegs
             allocs += [4, 4 * cap, cap, 8 * cap, 16 * cap, 8 * cap]
             allocs += [4 * ncell, 4 * ((ncell + 31) // 32)] * 2
         total = 16 << 20
