@@ -125,6 +125,10 @@ int mfc_streaming(mfc_ctx* ctx);        /* BOX/streaming.f90:2-171 */
 /* rhoupdat (BOX/collision.f90:213-229); optionally also returns
  * max|rho_new - rho_old|, the pre-relaxation residual of BOX/main.f90:91-96. */
 int mfc_rhoupdat(mfc_ctx* ctx, double* max_abs_change);
+/* The pre-relaxation loop (BOX/main.f90:86-108): collision_MRT, streaming and
+ * rhoupdat until its residual is at most eps or the iteration count, from 0,
+ * passes max_iter; the count and the residual are returned. */
+int mfc_prerelax(mfc_ctx* ctx, double eps, int32_t max_iter, int32_t* iterations, double* residual);
 int mfc_macrovar(mfc_ctx* ctx);         /* BOX/collision.f90:232-332 */
 
 /* ---- particles (BOX/partlib.f90) ----------------------------------------- */

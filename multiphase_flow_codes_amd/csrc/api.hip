@@ -451,7 +451,7 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   CK(hipMalloc(&c.d_status, sizeof(int32_t) * ST_COUNT));
   CK(hipMemsetAsync(c.d_status, 0, sizeof(int32_t) * ST_COUNT, c.stream));
   CK(hipHostMalloc((void**)&c.h_status, sizeof(int32_t) * ST_COUNT, hipHostMallocDefault));
-  CK(hipMalloc(&c.d_red, sizeof(double) * (size_t)rhoupdat_blocks(c)));
+  CK(hipMalloc(&c.d_red, sizeof(double) * (size_t)(rhoupdat_blocks(c) + relax_slots())));
   CK(hipHostMalloc((void**)&c.h_red, sizeof(double) * 8, hipHostMallocCoherent));
   memset(c.h_red, 0, sizeof(double) * 8);
   // this device's static scratch of the allocation-free sums
@@ -756,6 +756,46 @@ int mfc_rhoupdat(mfc_ctx* ctx, double* maxdiff) {
     *maxdiff = c.h_red[0];
   }
   return MFC_OK;
+}
+
+// The pre-relaxation loop (main.f90:86-108): collide, stream, rhoupdat until the
+// largest density change is at most `eps` or `max_iter` is passed.  With two
+// buffers and no spheres the rhoupdat of an iteration runs in the grid of the
+// next one's collide (its result is dropped when the loop ends there: the
+// buffers are not swapped); the last iteration of all has no next one.
+int mfc_prerelax(mfc_ctx* ctx, double eps, int32_t max_iter, int32_t* iters, double* residual) {
+  NEEDCTX;
+  Ctx& c = ctx->c;
+  if (!iters || !residual) return MFC_ERR_ARG;
+  int rc = mfc_collision_mrt(ctx);
+  if (rc || (rc = mfc_streaming(ctx))) return rc;
+  const bool fused = c.g.lay == LAY_AB && !(c.pt.np > 0 && c.pt.map_np[c.pt.map_cur] > 0) && !c.timing;
+  double* slots = c.d_red + rhoupdat_blocks(c);
+  if (fused) {
+    if ((rc = need_arrays(ctx))) return rc;
+    HIPCHK(hipMemsetAsync(slots, 0, sizeof(double) * (size_t)relax_slots(), c.stream));
+  }
+  int32_t it = 0;
+  for (;;) {
+    const bool ahead = fused && it <= max_iter;
+    if (ahead) {
+      HIPCHK(launch_collide_relax(c, slots, c.h_red, ++c.red_seq));
+      c.mom = MOM_ARRAYS;
+      HIPCHK(wait_flag((const uint32_t*)(c.h_red + 1), c.red_seq, c.stream));
+      *residual = c.h_red[0];
+    } else if ((rc = mfc_rhoupdat(ctx, residual))) {
+      return rc;
+    }
+    *iters = it;
+    if (*residual <= eps || it > max_iter) return MFC_OK;
+    ++it;
+    if (ahead) {   // that iteration has collided already
+      c.cur ^= 1;
+      c.f_version += 2;
+    } else if ((rc = mfc_collision_mrt(ctx)) || (rc = mfc_streaming(ctx))) {
+      return rc;
+    }
+  }
 }
 
 int mfc_macrovar(mfc_ctx* ctx) {

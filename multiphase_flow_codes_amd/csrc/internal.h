@@ -174,7 +174,7 @@ struct Ctx {
   Particles pt;
   int32_t* d_status = nullptr;
   int32_t* h_status = nullptr;      // pinned
-  double* d_red = nullptr;          // workgroup maxima of rhoupdat
+  double* d_red = nullptr;          // workgroup maxima of rhoupdat, then the words of the pre-relaxation
   double* h_red = nullptr;          // pinned: rhoupdat's residual and the word that says it is there
   uint32_t red_seq = 0;
   void* staging = nullptr;          // device staging for host transfers
@@ -219,6 +219,10 @@ int rhoupdat_blocks(const Ctx& c);   // workgroup maxima launch_rhoupdat leaves 
 // out (pinned, may be null): max |rho_new - rho_old|, then `seq` in the word
 // behind it
 hipError_t launch_rhoupdat(Ctx& c, bool pulled, double* part, double* out, uint32_t seq);
+// rhoupdat and the collide after it in one grid (two buffers, no spheres);
+// slots: relax_slots() words, zero before and after
+int relax_slots();
+hipError_t launch_collide_relax(Ctx& c, double* slots, double* out, uint32_t seq);
 hipError_t launch_initpop(Ctx& c);
 hipError_t launch_pop_to_aos(Ctx& c, double* dst, int z0, int nzs, bool pulled);
 hipError_t launch_aos_to_pop(Ctx& c, const double* src, int z0, int nzs, bool pulled);

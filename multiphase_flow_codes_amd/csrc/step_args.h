@@ -21,7 +21,8 @@ struct CollideArgs {
   Grid g;
   CollideConsts k;
   ForceArgs fa;
-  const double *rho, *ux, *uy, *uz;
+  double* rho;
+  const double *ux, *uy, *uz;
   int arr;   // batched launches: conserved moments from the arrays (else recomputed)
 };
 

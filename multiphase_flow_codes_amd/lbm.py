@@ -10,6 +10,7 @@ module raises -- there is no CPU fallback.
 from __future__ import annotations
 
 import ctypes as C
+import math
 import os
 
 import numpy as np
@@ -84,6 +85,7 @@ SIGNATURES = {
     "mfc_collision_mrt": [C.c_void_p],
     "mfc_streaming": [C.c_void_p],
     "mfc_rhoupdat": [C.c_void_p, _D],
+    "mfc_prerelax": [C.c_void_p, C.c_double, C.c_int32, _I, _D],
     "mfc_macrovar": [C.c_void_p],
     "mfc_prt_init": [C.c_void_p, C.c_int32],
     "mfc_prt_set": [C.c_void_p, C.c_int32, _D],
@@ -283,16 +285,10 @@ class Lattice:
         collision_MRT, streaming, rhoupdat until max|rho - rho_prev| <= rhoepsl or
         the iteration count passes max_iter; then macrovar.  Returns
         (iterations, final residual)."""
-        it = 0
-        while True:
-            self.collision_mrt()
-            self.streaming()
-            err = self.rhoupdat()
-            if err <= rhoepsl or it > max_iter:
-                break
-            it += 1
+        it, err = C.c_int32(), C.c_double()
+        self._chk(lib().mfc_prerelax(self.h, float(rhoepsl), math.floor(min(max(max_iter, -1), 2**31 - 2)), C.byref(it), C.byref(err)))
         self.macrovar()
-        return it, err
+        return it.value, err.value
 
     # -- particles ---------------------------------------------------------------
     def prt_init(self, npart: int):
