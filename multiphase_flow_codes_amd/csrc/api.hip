@@ -19,6 +19,7 @@
 #include <new>
 #include <vector>
 
+#include "field_sums.h"
 #include "force_table.h"
 #include "internal.h"
 
@@ -252,7 +253,8 @@ int ensure_macro(mfc_ctx* ctx) {
 // arrays are a copy for the caller, and the next collide still recomputes
 // the moments itself, so a step's result (in FP32 arithmetic too) does not
 // depend on whether the host looked at rho/u before it.
-int need_arrays(mfc_ctx* ctx) {
+// With `fill` a pass that would materialise is left to the caller (*fill set).
+int need_arrays(mfc_ctx* ctx, bool* fill = nullptr) {
   Ctx& c = ctx->c;
   if (c.mom == MOM_ARRAYS) return MFC_OK;
   if (c.mom == MOM_VIRTUAL) {
@@ -261,7 +263,10 @@ int need_arrays(mfc_ctx* ctx) {
     if (c.rho && c.arrays_version == c.mom_version) return MFC_OK;
     int rc = ensure_macro(ctx);
     if (rc) return rc;
-    HIPCHK(launch_macro(c, c.phase == PHASE_POST_STREAM));
+    if (fill)
+      *fill = true;
+    else
+      HIPCHK(launch_macro(c, c.phase == PHASE_POST_STREAM));
     c.arrays_version = c.mom_version;
     return MFC_OK;
   }
@@ -1332,7 +1337,7 @@ static int ensure_diag(mfc_ctx* ctx, int nek) {
     c.diag_out = nullptr;
   }
   if (!c.diag_part) {
-    HIPCHK(hipMalloc(&c.diag_part, sizeof(double) * (size_t)nb * need));
+    HIPCHK(hipMalloc(&c.diag_part, sizeof(double) * std::max((size_t)nb * need, 6 * (size_t)kSumBlocksMax)));
     HIPCHK(hipMalloc(&c.diag_out, sizeof(double) * need));
     c.diag_nek = need;
   }
@@ -1343,10 +1348,11 @@ int mfc_diag_sums(mfc_ctx* ctx, double* out6) {
   NEEDCTX;
   if (!out6) return MFC_ERR_ARG;
   Ctx& c = ctx->c;
-  int rc = need_arrays(ctx);
+  int rc = ensure_diag(ctx, 6);
   if (rc) return rc;
-  if ((rc = ensure_diag(ctx, 6))) return rc;
-  HIPCHK(launch_field_sums(c, c.diag_part, c.diag_out));
+  bool fill = false;
+  if ((rc = need_arrays(ctx, &fill))) return rc;
+  HIPCHK(launch_field_sums(c, fill, c.diag_part, c.diag_out));
   const HostPart part = {out6, c.diag_out, sizeof(double) * 6};
   HIPCHK(copy_to_host(c, &part, 1));
   return MFC_OK;
@@ -1359,20 +1365,16 @@ int mfc_diag_sums_noalloc(mfc_ctx* ctx, double* out6) {
   if (!c.rho) return fail(ctx, MFC_ERR_STATE, "diag_sums_noalloc: the rho/u arrays do not exist yet "
                                                "(a call that returns them allocates them first)");
   if (!c.sums_scratch) return fail(ctx, MFC_ERR_STATE, "diag_sums_noalloc: device scratch not resolved");
-  const size_t need = 6 * (size_t)diag_blocks() + 6;
+  const size_t nsum = 6 * (size_t)sum_blocks(c.g.ncell), need = nsum + 6;
   if (need > sums_scratch_doubles())
     return fail(ctx, MFC_ERR_CAPACITY, "diag_sums_noalloc: the partial sums exceed the static scratch");
-  if (c.mom != MOM_ARRAYS) {
-    if (c.mom != MOM_VIRTUAL || c.mom_version != c.f_version)
-      return fail(ctx, MFC_ERR_STATE, "rho/u requested after the field changed since macrovar");
-    if (c.arrays_version != c.mom_version) {
-      HIPCHK(launch_macro(c, c.phase == PHASE_POST_STREAM));
-      c.arrays_version = c.mom_version;
-    }
-  }
+  if (c.mom != MOM_ARRAYS && (c.mom != MOM_VIRTUAL || c.mom_version != c.f_version))
+    return fail(ctx, MFC_ERR_STATE, "rho/u requested after the field changed since macrovar");
+  const bool fill = c.mom != MOM_ARRAYS && c.arrays_version != c.mom_version;
+  if (fill) c.arrays_version = c.mom_version;
   double* part = c.sums_scratch;
-  double* res = part + 6 * (size_t)diag_blocks();
-  HIPCHK(launch_field_sums(c, part, res));
+  double* res = part + nsum;
+  HIPCHK(launch_field_sums(c, fill, part, res));
   HIPCHK(hipMemcpyAsync(out6, res, sizeof(double) * 6, hipMemcpyDeviceToDevice, c.stream));
   return MFC_OK;
 }

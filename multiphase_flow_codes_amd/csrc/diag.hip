@@ -11,59 +11,31 @@
 #include <algorithm>
 #include <mutex>
 
+#include "field_sums.h"
 #include "internal.h"
 
 namespace mfc {
 
-constexpr int DB = 256;          // threads per reduction block
-constexpr int kSumBlocks = 1024; // partial sums of the first level
-
 // Scratch of the allocation-free field sums (mfc_diag_sums_noalloc): the
-// kSumBlocks x 6 first-level partials, then the 6 results it leaves before
+// kSumBlocksMax x 6 first-level partials, then the 6 results it leaves before
 // they are copied out.  Every GPU the library runs on holds its own copy
 // until the process ends.  The host resolves its address once per device
 // (sums_scratch) and passes that pointer to the kernels; the array's name in
 // host code is only a stand-in.  Each call overwrites every word it reads,
 // so nothing is cleared between calls; calls that overlap on one GPU share
 // the array and race.
-constexpr size_t kSumsScratchDoubles = 6 * (size_t)kSumBlocks + 8;
+constexpr size_t kSumsScratchDoubles = 6 * (size_t)kSumBlocksMax + 8;
 static __device__ __align__(256) double scratch[kSumsScratchDoubles];
 
 // Per-block partial sums of rho, ux, uy, uz and u.u, and the block's max |u|^2.
-__global__ void __launch_bounds__(DB)
+__global__ void __launch_bounds__(kSumThreads)
     k_field_sums(const double* __restrict__ rho, const double* __restrict__ ux,
                  const double* __restrict__ uy, const double* __restrict__ uz, uint64_t n,
                  double* __restrict__ part) {
-  __shared__ double red[6][DB / 64];
-  double s[6] = {0, 0, 0, 0, 0, 0};
-  for (uint64_t i = (uint64_t)blockIdx.x * DB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * DB) {
-    const double a = ux[i], b = uy[i], c = uz[i];
-    const double q = a * a + b * b + c * c;
-    s[0] += rho[i];
-    s[1] += a;
-    s[2] += b;
-    s[3] += c;
-    s[4] += q;
-    s[5] = fmax(s[5], q);
-  }
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    double v = s[k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const double t = __shfl_down(v, o, 64);
-      v = (k == 5) ? fmax(v, t) : v + t;
-    }
-    if (lane == 0) red[k][w] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 6) {
-    const int k = threadIdx.x;
-    double v = red[k][0];
-    for (int q = 1; q < DB / 64; ++q) v = (k == 5) ? fmax(v, red[k][q]) : v + red[k][q];
-    part[6 * blockIdx.x + k] = v;
-  }
+  FieldSums f;
+  for (uint64_t i = (uint64_t)blockIdx.x * kSumThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kSumThreads)
+    f.add(rho[i], ux[i], uy[i], uz[i]);
+  f.store(part);
 }
 
 // The final sums: wavefront k adds component k's partials, each lane every
@@ -497,10 +469,16 @@ __global__ void __launch_bounds__(1024)
 }
 
 // ---------------------------------------------------------------------------
-hipError_t launch_field_sums(Ctx& c, double* part, double* out) {
-  hipLaunchKernelGGL(k_field_sums, dim3(kSumBlocks), dim3(DB), 0, c.stream, c.rho, c.ux, c.uy, c.uz,
-                     (uint64_t)c.g.ncell, part);
-  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(6 * 64), 0, c.stream, part, kSumBlocks, out);
+hipError_t launch_field_sums(Ctx& c, bool fill, double* part, double* out) {
+  const int nb = sum_blocks(c.g.ncell);
+  if (fill) {
+    const hipError_t e = launch_macro_sums(c, c.phase == PHASE_POST_STREAM, part);
+    if (e != hipSuccess) return e;
+  } else {
+    hipLaunchKernelGGL(k_field_sums, dim3(nb), dim3(kSumThreads), 0, c.stream, c.rho, c.ux, c.uy, c.uz,
+                       (uint64_t)c.g.ncell, part);
+  }
+  hipLaunchKernelGGL(k_sums_final, dim3(1), dim3(6 * 64), 0, c.stream, part, nb, out);
   return hipGetLastError();
 }
 

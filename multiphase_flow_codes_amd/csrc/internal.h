@@ -215,6 +215,8 @@ hipError_t launch_collide(Ctx& c, bool arrays);
 // `list`; with far set the solid mask is not read
 hipError_t launch_collide_tiles(Ctx& c, const uint32_t* list, uint32_t n, bool far);
 hipError_t launch_macro(Ctx& c, bool pulled);
+// with the first level of the field sums in `part`
+hipError_t launch_macro_sums(Ctx& c, bool pulled, double* part);
 int rhoupdat_blocks(const Ctx& c);   // workgroup maxima launch_rhoupdat leaves in `part`
 // out (pinned, may be null): max |rho_new - rho_old|, then `seq` in the word
 // behind it
@@ -277,7 +279,8 @@ hipError_t launch_init_velocity(Ctx& c, const double2* amp, double scale, double
 
 // ---- launchers (diag.hip) ----
 int diag_blocks();
-hipError_t launch_field_sums(Ctx& c, double* part, double* out);
+// fill: the rho/u arrays are filled by the same pass
+hipError_t launch_field_sums(Ctx& c, bool fill, double* part, double* out);
 // the static device scratch of the allocation-free sums: its size in
 // doubles and its address on the current device
 size_t sums_scratch_doubles();
