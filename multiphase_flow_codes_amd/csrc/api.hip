@@ -836,7 +836,7 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
       *a = nullptr;
       HIPCHK(hipMalloc(a, sizeof(double) * 3 * npart));
     }
-    P.slab = segment_planes(c.p.rad, npart);
+    P.slab = segment_planes(c.p.rad, npart, P.want_slab);
     P.nseg = segments_per_particle(c.p.rad, P.slab);
     P.seg_cap = segment_capacity(c.p.rad, P.slab);
     const size_t nsegs = (size_t)npart * P.nseg;
@@ -1420,6 +1420,16 @@ int mfc_set_bb_order(mfc_ctx* ctx, int32_t order) {
     P.ord_cap = kOrderCap;
   }
   P.bb_order = order;
+  return MFC_OK;
+}
+
+int mfc_set_segment_planes(mfc_ctx* ctx, int32_t planes) {
+  NEEDCTX;
+  Ctx& c = ctx->c;
+  if (planes != 0 && planes != 1 && planes != 2 && planes != 4 && planes != 8)
+    return fail(ctx, MFC_ERR_ARG, "segment planes must be 1, 2, 4, 8 or 0 (by size)");
+  if (c.pt.np_max > 0) return fail(ctx, MFC_ERR_STATE, "segment planes are chosen before the spheres are set");
+  c.pt.want_slab = planes;
   return MFC_OK;
 }
 

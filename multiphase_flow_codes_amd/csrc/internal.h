@@ -123,6 +123,7 @@ struct Particles {
   int32_t* sol_cnt[2] = {nullptr, nullptr};
   // boundary links: lk_seg slots per segment, lk_cap in all
   int lk_seg = 0;
+  int want_slab = 0;   // mfc_set_segment_planes
   int64_t lk_cap = 0;
   uint32_t* lk_node = nullptr;
   uint8_t* lk_dir = nullptr;
@@ -233,7 +234,7 @@ hipError_t launch_force_field(Ctx& c, int slot, double* fx, double* fy, double* 
 // ---- launchers (particles.hip) ----
 int segments_per_particle(double rad, int slab);
 int segment_capacity(double rad, int slab);
-int segment_planes(double rad, int npart);
+int segment_planes(double rad, int npart, int want);
 int segment_links(double rad, int slab);
 // defer_contacts: the contact links are listed by the refill grid that follows
 hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool defer_contacts = false);

@@ -1660,22 +1660,35 @@ int segment_links(double rad, int slab) {
   return (int)ceil(in_plane + across) + 64;
 }
 
-// Planes per segment.  8 when the spheres are many (the segment grids of the
-// link rebuild and the bounce-back still fill the GPU several times over
-// with half as many, twice as large workgroups: at 1024^3 with 20,000
-// spheres of radius 6 the three kernels take 0.5 ms less per step), else 4
-// (300 spheres of radius 8 at 256^3 need the parallelism: 0.06 ms more per
-// step with 8).  8 also needs at most PB / 8 candidate rows per plane and
+// Planes per segment.  The fewer planes, the shorter a workgroup's chain of
+// passes; the more, the fewer workgroups.  1 or 2 where the spheres are few:
+// their workgroups fit the 256 CUs at once, five or six each (step at 64^3 FP32
+// with 8 spheres of radius 4: 46.0 us with 1, 47.7 with 2, 54.1 with 4; 96^3 with
+// 20 of radius 6 69.6, 72.0, 82.9; 100^3 with 4 of radius 13 81, 91, 118; 128^3
+// with 60 of radius 6 (1260 segments of 1 plane) 107.3, 109.7, 117.7; with 100
+// of radius 4 (1700) 106.6, 105.0, 107.0; 150 x 141 x 162 with 140 of radius 6
+// (1540 of 2 planes) 178.9, 171.8, 177.4; 160^3 with 250 of radius 4 (2250)
+// 189.1, 180.2, 175.1).  Many small boxes in one grid fill the GPU anyhow (32
+// boxes 1003 us a step with 1, 953 with 2, 939 with 4): their contexts ask for
+// 4.  8 when the spheres are many (the segment grids of the link rebuild and the bounce-back still fill the GPU
+// several times over with half as many, twice as large workgroups: at 1024^3
+// with 20,000 spheres of radius 6 the three kernels take 0.5 ms less per step),
+// else 4 (300 spheres of radius 8 at 256^3 need the parallelism: 0.06 ms more
+// per step with 8).  8 also needs at most PB / 8 candidate rows per plane and
 // keeps the scan's shell list within 10 KB of LDS, so only for
-// box_candidates <= 25 (rad <= 8).  MFC_SEG_PLANES=4 or 8 forces one (8 only
-// where it fits).
-constexpr int64_t kSlab8MinSegments = 8192;
-int segment_planes(double rad, int npart) {
+// box_candidates <= 25 (rad <= 8).  `want` (a context's own choice) and
+// MFC_SEG_PLANES = 1, 2, 4 or 8 force one (8 only where it fits).
+constexpr int64_t kSlab1MaxSegments = 1280, kSlab2MaxSegments = 1600, kSlab8MinSegments = 8192;
+int segment_planes(double rad, int npart, int want) {
   const bool fits8 = box_candidates(rad) <= 25;
   const char* e = getenv("MFC_SEG_PLANES");
-  if (e && e[0] == '4') return 4;
-  if (e && e[0] == '8') return fits8 ? 8 : 4;
-  return (fits8 && (int64_t)npart * segments_per_particle(rad, 8) >= kSlab8MinSegments) ? 8 : 4;
+  if (e && (e[0] == '1' || e[0] == '2' || e[0] == '4' || e[0] == '8')) want = e[0] - '0';
+  if (want == 8 && !fits8) want = 4;
+  if (want) return want;
+  auto segs = [&](int planes) { return (int64_t)npart * segments_per_particle(rad, planes); };
+  if (segs(1) <= kSlab1MaxSegments) return 1;
+  if (segs(2) <= kSlab2MaxSegments) return 2;
+  return fits8 && segs(8) >= kSlab8MinSegments ? 8 : 4;
 }
 
 // Reset map buffer `buf` to empty (no-op if it is empty already).

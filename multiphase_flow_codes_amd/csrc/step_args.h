@@ -35,7 +35,7 @@ struct PGeom {
   double rlink2;
   // (r + 0.5)^2: no solid node lies farther out than this
   double rsolid2;
-  // z planes per segment (4 or 8; Particles::slab)
+  // z planes per segment (Particles::slab)
   int slab;
   FastDiv dseg;   // division by the segments per particle
 };

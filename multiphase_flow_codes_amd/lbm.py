@@ -96,6 +96,7 @@ SIGNATURES = {
     "mfc_beads_links": [C.c_void_p],
     "mfc_beads_collision": [C.c_void_p],
     "mfc_set_bb_order": [C.c_void_p, C.c_int32],
+    "mfc_set_segment_planes": [C.c_void_p, C.c_int32],
     "mfc_beads_lubforce": [C.c_void_p],
     "mfc_beads_move": [C.c_void_p, C.c_int32],
     "mfc_beads_redistribute": [C.c_void_p, C.c_int32],
@@ -372,6 +373,14 @@ class Lattice:
         if order not in codes:
             raise ValueError(f"bounce-back order must be one of {sorted(codes)}")
         self._chk(lib().mfc_set_bb_order(self.h, codes[order]))
+
+    def set_segment_planes(self, planes: int):
+        """Lattice planes per unit of particle work (1, 2, 4 or 8; 0, the
+        default: by size), to be chosen before prt_init.  By size, few spheres
+        are cut into many units so that they fill the GPU on their own; 4 suits a
+        box that shares it with many others.  The forces' sums over units differ
+        in rounding."""
+        self._chk(lib().mfc_set_segment_planes(self.h, int(planes)))
 
     def set_timing(self, every):
         """Time every `every`-th collide launch with HIP events (True: each

@@ -150,6 +150,7 @@ def make_lattice(case: BoxCase, precision: str) -> Lattice:
     lat.rhoupdat()
     lat.macrovar()
     if case.npart:
+        lat.set_segment_planes(4)   # many such boxes share the GPU
         lat.prt_init(case.npart)
         lat.initpartpos(case.seed, mingap_check=True)
         lat.initpartomg()
