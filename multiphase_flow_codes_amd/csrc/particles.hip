@@ -1670,25 +1670,29 @@ int segment_links(double rad, int slab) {
 // (1540 of 2 planes) 178.9, 171.8, 177.4; 160^3 with 250 of radius 4 (2250)
 // 189.1, 180.2, 175.1).  Many small boxes in one grid fill the GPU anyhow (32
 // boxes 1003 us a step with 1, 953 with 2, 939 with 4): their contexts ask for
-// 4.  8 when the spheres are many (the segment grids of the link rebuild and the bounce-back still fill the GPU
-// several times over with half as many, twice as large workgroups: at 1024^3
-// with 20,000 spheres of radius 6 the three kernels take 0.5 ms less per step),
-// else 4 (300 spheres of radius 8 at 256^3 need the parallelism: 0.06 ms more
-// per step with 8).  8 also needs at most PB / 8 candidate rows per plane and
-// keeps the scan's shell list within 10 KB of LDS, so only for
-// box_candidates <= 25 (rad <= 8).  `want` (a context's own choice) and
-// MFC_SEG_PLANES = 1, 2, 4 or 8 force one (8 only where it fits).
-constexpr int64_t kSlab1MaxSegments = 1280, kSlab2MaxSegments = 1600, kSlab8MinSegments = 8192;
+// 4.  8 where the spheres are many and small, whose segments of 4 leave most of
+// a pass idle: radius up to 4 from 500 segments of 8 (160^3 with 400 of radius 3
+// 175 us against 193 with 4; 192^3 with 400 of radius 4 259 against 264; 128^3
+// with 150 of radius 3, 300 segments, 105 against 109), up to 6 from 2048 (352^3
+// with 1500 of radius 6 1667 against 1684, 256^3 with 700 637 against 640; 224^3
+// with 350, 1050 segments, 435 against 437 with 4 but 428 with 2).  Larger
+// spheres have enough in 4 (radius 7 at 400^3 2420 and 2418; radius 8 at 288^3
+// 899 against 1002, at 448^3 with 8400 segments of 8 3298 against 3683).  8 also
+// needs at most PB / 8 candidate rows per plane and keeps the scan's shell list
+// within 10 KB of LDS, so only for box_candidates <= 25 (rad <= 8).  `want` (a
+// context's own choice) and MFC_SEG_PLANES = 1, 2, 4 or 8 force one (8 only
+// where it fits).
+constexpr int64_t kSlab1MaxSegments = 1280, kSlab2MaxSegments = 1600;
 int segment_planes(double rad, int npart, int want) {
-  const bool fits8 = box_candidates(rad) <= 25;
+  const int rows = box_candidates(rad);
   const char* e = getenv("MFC_SEG_PLANES");
   if (e && (e[0] == '1' || e[0] == '2' || e[0] == '4' || e[0] == '8')) want = e[0] - '0';
-  if (want == 8 && !fits8) want = 4;
+  if (want == 8 && rows > 25) want = 4;
   if (want) return want;
   auto segs = [&](int planes) { return (int64_t)npart * segments_per_particle(rad, planes); };
+  if (segs(8) >= (rows <= 17 ? 500 : 2048) && rows <= 21) return 8;   // radius up to 4, 6
   if (segs(1) <= kSlab1MaxSegments) return 1;
-  if (segs(2) <= kSlab2MaxSegments) return 2;
-  return fits8 && segs(8) >= kSlab8MinSegments ? 8 : 4;
+  return segs(2) <= kSlab2MaxSegments ? 2 : 4;
 }
 
 // Reset map buffer `buf` to empty (no-op if it is empty already).
