@@ -199,7 +199,7 @@ int mfc_diag_sums(mfc_ctx* ctx, double* out6);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops that must not call
  * hipMalloc): mfc_diag_sums with its first-level partials and results in a
- * static device array of the library (6 x 1024 + 8 doubles per GPU,
+ * static device array of the library (6 x 4096 + 8 doubles per GPU,
  * resolved when a context is created) instead of buffers allocated on first
  * use.  out6 is DEVICE memory for the six values (same order as
  * mfc_diag_sums); the work is queued on the context's stream without

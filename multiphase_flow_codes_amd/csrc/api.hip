@@ -896,7 +896,7 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
   if (P.cell_list) HIPCHK(hipFree(P.cell_list));
   P.cell_cnt = nullptr;
   P.cell_list = nullptr;
-  P.cells_ok = false;
+  P.cells_ok = P.cells_zeroed = false;
   if (npart > kCellMinParticles) {
     const double h = 2.0 * c.p.rad + std::max(c.p.mingap, 0.0) + 1e-3;
     const int ns[3] = {c.g.nx, c.g.ny, c.g.nz};
@@ -907,7 +907,7 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
     }
     if (ok) {
       const size_t ncell = (size_t)P.cell_n[0] * P.cell_n[1] * P.cell_n[2];
-      HIPCHK(hipMalloc(&P.cell_cnt, sizeof(int32_t) * ncell));
+      HIPCHK(hipMalloc(&P.cell_cnt, sizeof(int32_t) * ncell * 2));
       HIPCHK(hipMalloc(&P.cell_list, sizeof(int32_t) * ncell * kCellCap));
     }
   }

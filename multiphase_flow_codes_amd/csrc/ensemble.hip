@@ -3,8 +3,8 @@
 // Each member is an ordinary context (its own size, spheres, rates and body
 // force; state created and initialised through the single-box API).  One
 // ensemble step runs the time-loop body of every member with one grid per
-// stage for all of them: collide, contact links (+ lubrication), bounce-back
-// (+ map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
+// stage for all of them: collide, contact links, bounce-back
+// (+ lubrication, map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
 // per-stage table and finds its member from a block-offset table
 // (off[c] <= blockIdx.x < off[c+1]).  The sequence and the per-member state
 // transitions are exactly those of mfc_step, so a member advanced in the

@@ -145,7 +145,8 @@ struct Particles {
   // cell grid of the pair searches (on for many particles): per-cell counts
   // and particle lists, valid for the positions at the last build
   int cell_n[3] = {0, 0, 0};
-  int32_t* cell_cnt = nullptr;
+  int32_t* cell_cnt = nullptr;   // two halves: the current counts and those the next move fills
+  int cell_half = 0;
   int32_t* cell_list = nullptr;
   bool cells_ok = false;
   bool cells_zeroed = false;   // cleared by the fused bounce-back grid for the move that follows

@@ -1014,22 +1014,10 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
 // node, which the bounce-back grid overwrites: their values are taken first,
 // from the untouched field, into lk_out (f9, ff1).  Every other link reads
 // fluid nodes only and writes only solid ones, so the bounce-back grid can
-// scatter as it goes; all links see the one post-collision snapshot.  The
-// first nct blocks stride over the contact list; the blocks after them
-// compute beads_lubforce (which the bounce-back does not read).
+// scatter as it goes; all links see the one post-collision snapshot.  nct
+// blocks stride over the contact list.
 template <typename T>
 __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
-  if (b_ >= a.nct) {
-    const int r = b_ - a.nct;
-    if (a.lub.cells.cnt) {
-      extern __shared__ double lds_f64[];
-      lub_cells(r * (PB / 64) + (int)(threadIdx.x >> 6), a.ypglb, a.np, a.G, a.lub,
-                ((LubList*)lds_f64)[threadIdx.x >> 6]);
-    } else {
-      lub_block(r, a.ypglb, a.np, a.G, a.lub);
-    }
-    return;
-  }
   if (a.ref_order) {
     if (b_ == 0) bb_contact_ordered<T>(a);
     return;
@@ -1053,11 +1041,26 @@ __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
   }
 }
 
+// Workgroups are dealt to the 8 XCDs round-robin in launch order.  Launch
+// index L of the first nsegs blocks is mapped so that all segments of a
+// particle run on one XCD (particle p on XCD p % 8): neighbouring segments
+// read overlapping stencils and that XCD's L2 then holds them once.
+__device__ __forceinline__ int xcd_segment(int L, int nsegs, int nseg) {
+  const int group = 8 * nseg;
+  const int full = (nsegs / group) * group;
+  if (L >= full) return L;
+  const int q = L / group, r = L - q * group;
+  return (q * 8 + r % 8) * nseg + r / 8;
+}
+
 // beads_collision (partlib.f90:1363-1703), one unit (1/split of a segment's
 // links) per block: the bounce-back value of every link, written at once into
 // the opposite population of the solid neighbour x + c (partlib.f90:1605-1621),
 // and the unit's momentum-exchange force and torque (FP64, fixed reduction
-// order) into seg_ft.  Blocks past the units (fused step) reset one segment
+// order) into seg_ft.  In the fused step nlub blocks before the units compute
+// beads_lubforce: beside the links they cost nothing, in the pre-pass 5 us (900
+// spheres at 192 x 176 x 208: pre-pass 9.2 to 4.6 us, this grid 62 to 63 us, a step
+// 299 to 293 us; 64^3 FP64 with 8 49 to 48 us).  Blocks past the units reset one segment
 // of the map buffer the coming beads_links rebuilds (built two steps ago), and
 // blocks past those the counts of the pair-search cells.
 template <typename T>
@@ -1065,14 +1068,24 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   __shared__ double red[6][PB / 64];
   T* A = (T*)a.A;
   const Grid& g = a.g;
-  const int u = b_;
+  if (b_ < a.nlub) {   // beads_lubforce, which no link reads
+    if (a.lub.cells.cnt) {
+      extern __shared__ double lds_f64[];
+      lub_cells(b_ * (PB / 64) + (int)(threadIdx.x >> 6), a.ypglb, a.np, a.G, a.lub,
+                ((LubList*)lds_f64)[threadIdx.x >> 6]);
+    } else {
+      lub_block(b_, a.ypglb, a.np, a.G, a.lub);
+    }
+    return;
+  }
   const int nunits = a.nsegs * a.split;
+  const int u = b_ - a.nlub;
   if (u >= nunits) {
     if (u - nunits < a.nclr) {
       clear_segment(u - nunits, a.nseg, a.seg_cap, a.clr_list, a.clr_cnt, a.clr_isn, a.clr_mask);
-    } else {   // the pair-search cells the coming move fills (the pre-pass has read them)
+    } else {   // the counts of the pair-search cells the coming move fills
       const int i = (u - nunits - a.nclr) * PB + (int)threadIdx.x;
-      if (i < a.ncell) a.lub.cells.cnt[i] = 0;
+      if (i < a.ncell) a.clr_cells[i] = 0;
     }
     return;
   }
@@ -1496,21 +1509,10 @@ __global__ void __launch_bounds__(PB)
   bb_contact_body<T>((int)blockIdx.x - off[c], a);
 }
 
-// Workgroups are dealt to the 8 XCDs round-robin in launch order.  Launch
-// index L of the first nsegs blocks is mapped so that all segments of a
-// particle run on one XCD (particle p on XCD p % 8): neighbouring segments
-// read overlapping stencils and that XCD's L2 then holds them once.
-__device__ __forceinline__ int xcd_segment(int L, int nsegs, int nseg) {
-  const int group = 8 * nseg;
-  const int full = (nsegs / group) * group;
-  if (L >= full) return L;
-  const int q = L / group, r = L - q * group;
-  return (q * 8 + r % 8) * nseg + r / 8;
-}
-
 template <typename T>
 __global__ void __launch_bounds__(PB) k_bounce_back(BounceArgs a) {
-  bounce_back_body<T>(xcd_segment((int)blockIdx.x, a.nsegs * a.split, a.nseg * a.split), a);
+  const int b = (int)blockIdx.x;
+  bounce_back_body<T>(b < a.nlub ? b : a.nlub + xcd_segment(b - a.nlub, a.nsegs * a.split, a.nseg * a.split), a);
 }
 template <typename T>
 __global__ void __launch_bounds__(PB)
@@ -1722,12 +1724,14 @@ static bool make_fill_args(Ctx& c, int old, int neu, FillArgs& fa) {
   return true;
 }
 
+static int cell_count(const Particles& P) { return P.cell_n[0] * P.cell_n[1] * P.cell_n[2]; }
+
 // The cell grid if it is on (else cnt = nullptr: all pairs).  The lists must
 // be current (ensure_cells) before a kernel reads them.
 static CellArgs cell_args(const Ctx& c) {
   const Particles& P = c.pt;
   CellArgs C;
-  C.cnt = c.ens ? nullptr : P.cell_cnt;   // ensemble members search all pairs
+  C.cnt = c.ens || !P.cell_cnt ? nullptr : P.cell_cnt + P.cell_half * cell_count(P);   // ensemble members search all pairs
   C.list = P.cell_list;
   C.ncx = P.cell_n[0];
   C.ncy = P.cell_n[1];
@@ -1746,8 +1750,8 @@ static int lub_blocks(const Ctx& c) {
 hipError_t ensure_cells(Ctx& c) {
   Particles& P = c.pt;
   if (!cell_args(c).cnt || P.cells_ok) return hipSuccess;
-  const int ncell = P.cell_n[0] * P.cell_n[1] * P.cell_n[2];
-  hipLaunchKernelGGL(k_cell_zero, dim3((ncell + 255) / 256), dim3(256), 0, c.stream, P.cell_cnt, ncell);
+  const int ncell = cell_count(P);
+  hipLaunchKernelGGL(k_cell_zero, dim3((ncell + 255) / 256), dim3(256), 0, c.stream, cell_args(c).cnt, ncell);
   hipLaunchKernelGGL(k_cell_build, dim3((P.np + 255) / 256), dim3(256), 0, c.stream, P.ypglb, P.np,
                      pgeom(c), cell_args(c), c.d_status);
   P.cells_ok = true;
@@ -1825,11 +1829,11 @@ BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blo
   a.clr_list = P.sol_list[t]; a.clr_cnt = P.sol_cnt[t]; a.clr_isn = P.isn[t]; a.clr_mask = P.mask[t];
   if (nclr) P.map_np[t] = 0;
   a.nclr = nclr;
-  a.ncell = fused && a.lub.cells.cnt ? P.cell_n[0] * P.cell_n[1] * P.cell_n[2] : 0;
+  a.ncell = fused && a.lub.cells.cnt ? cell_count(P) : 0;
+  a.clr_cells = a.ncell ? P.cell_cnt + (P.cell_half ^ 1) * a.ncell : nullptr;
   P.cells_zeroed = a.ncell > 0;
-  if (a.ncell) P.cells_ok = false;
-  *bb_blocks = a.nsegs * a.split + nclr + (a.ncell + PB - 1) / PB;
-  *pre_blocks = a.nct + a.nlub;
+  *bb_blocks = a.nlub + a.nsegs * a.split + nclr + (a.ncell + PB - 1) / PB;
+  *pre_blocks = a.nct;
   return a;
 }
 
@@ -1849,6 +1853,7 @@ MoveKArgs move_args(Ctx& c, int first, int wrap, bool from_seg, int* blocks) {
   a.seg_ft = from_seg ? P.seg_ft : nullptr; a.nseg = P.nseg * P.bb_split;
   // the cells the fused bounce-back grid has cleared: filled at the new centres
   const bool fill = wrap && from_seg && P.cells_zeroed;
+  if (fill) P.cell_half ^= 1;
   a.cells = fill ? cell_args(c) : CellArgs{};
   P.cells_zeroed = false;
   if (wrap) P.cells_ok = fill;   // the wrapped positions are the new ypglb
@@ -2069,11 +2074,11 @@ hipError_t launch_bounce_back(Ctx& c, bool fused) {
   const BounceArgs ba = bounce_args(c, fused, kContactBlocks, &nb, &npre);
   const size_t lds = fused ? lub_lds(c) : 0;
   if (c.prec == MFC_PREC_FP64) {
-    hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), lds, c.stream, ba);
-    hipLaunchKernelGGL(k_bounce_back<double>, dim3(nb), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bounce_back<double>, dim3(nb), dim3(PB), lds, c.stream, ba);
   } else {
-    hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), lds, c.stream, ba);
-    hipLaunchKernelGGL(k_bounce_back<float>, dim3(nb), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    hipLaunchKernelGGL(k_bounce_back<float>, dim3(nb), dim3(PB), lds, c.stream, ba);
   }
   if (!fused)
     hipLaunchKernelGGL(k_seg_reduce, dim3((P.np + 255) / 256), dim3(256), 0, c.stream, P.seg_ft,

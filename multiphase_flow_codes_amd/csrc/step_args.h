@@ -112,9 +112,9 @@ struct ScanArgs {
   CellArgs cells;
 };
 
-// Arguments of the bounce-back grid (link segments, then the map-clearing
-// blocks) and of its pre-pass grid (nct blocks for the contact links, then
-// nlub lubrication blocks).
+// Arguments of the bounce-back grid (nlub lubrication blocks, the link
+// segments, the map-clearing blocks and those of the pair-search cells) and of
+// its pre-pass grid (nct blocks for the contact links).
 struct BounceArgs {
   void* A;
   Grid g;
@@ -141,7 +141,7 @@ struct BounceArgs {
   OrderEntry* ord;              // its table (ord_cap entries) and the current owner map
   int64_t ord_cap;
   const int32_t* isn;
-  int nlub;                     // lubrication blocks of the pre-pass grid (fused step, else 0)
+  int nlub;                     // lubrication blocks (fused step, else 0)
   LubArgs lub;
   int seg_cap;                  // map clearing (clr_* of map buffer map_cur ^ 1)
   const uint32_t* clr_list;
@@ -150,6 +150,7 @@ struct BounceArgs {
   uint32_t* clr_mask;
   int nclr;                     // blocks of the map clearing, then of the cells'
   int ncell;                    // pair-search cells to clear (0: none)
+  int32_t* clr_cells;
 };
 
 struct MoveKArgs {
@@ -178,8 +179,7 @@ struct FillKArgs {
 CollideArgs collide_args(Ctx& c);
 ScanArgs scan_args(Ctx& c, int target, int ovl, int istep);
 size_t scan_lds(const Ctx& c);   // dynamic LDS of the links scan
-// bb_blocks: the bounce-back grid; pre_blocks: the pre-pass grid (nct
-// contact blocks + lubrication)
+// bb_blocks: the bounce-back grid; pre_blocks: the pre-pass grid
 BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blocks);
 MoveKArgs move_args(Ctx& c, int first, int wrap, bool from_seg, int* blocks);
 FillKArgs fill_args(Ctx& c, bool refill, bool contacts, int* blocks);
