@@ -202,7 +202,7 @@ def run_ensemble_bench(ncases, steps):
                         f"nu=0.01, from rest, {steps} steps",
             "cells": int(sum(c.cells for c in cases)), "spheres": int(sum(c.npart for c in cases)),
             "step_launch": ("chunks of 8 steps: one table upload and one recorded HIP graph "
-                            "(6 stage grids per step) per chunk") if r32.get("graph") else "6 stage grids per step",
+                            "(5 stage grids per step) per chunk") if r32.get("graph") else "5 stage grids per step",
             "pencil": "collide block = `block` consecutive x nodes of one box; tile order 1 = blocks dealt "
                       "to the 8 XCDs in contiguous ranges",
             "fp32": {k: (round(r32[k], 4) if isinstance(r32[k], float) else r32[k]) for k in keep}

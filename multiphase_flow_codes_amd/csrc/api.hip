@@ -325,12 +325,13 @@ int check_faults(mfc_ctx* ctx) {
 // beads_links into the map buffer that does not hold the previous step's map
 // (the one beads_filling still needs), clearing what that buffer marked
 // before.  With `overlap_check` the links pass also runs ovlpchk.
-int links_now(mfc_ctx* ctx, int overlap_check, int istep, bool defer_contacts = false) {
+int links_now(mfc_ctx* ctx, int overlap_check, int istep) {
   Ctx& c = ctx->c;
   Particles& P = c.pt;
   const int target = (P.map_cur != P.map_old) ? P.map_cur : (P.map_cur ^ 1);
-  HIPCHK(launch_links(c, target, overlap_check, istep, defer_contacts));
+  HIPCHK(launch_links(c, target, overlap_check, istep));
   P.map_cur = target;
+  c.old_version = 0;   // the collide copied the old map's solid nodes
   return MFC_OK;
 }
 
@@ -736,7 +737,7 @@ int mfc_collision_mrt(mfc_ctx* ctx) {
   else
     c.g.lay = c.g.lay == LAY_AA_ODD ? LAY_AA_EVEN : LAY_AA_ODD;
   c.phase = PHASE_PRE_STREAM;
-  c.f_version++;
+  c.old_version = ++c.f_version;
   return MFC_OK;
 }
 
@@ -916,6 +917,8 @@ int mfc_prt_init(mfc_ctx* ctx, int32_t npart) {
                     P.forcep, P.forcepp, P.torqpp, P.dwdt, P.domgdt, P.thetap};
     for (double* a : pd) HIPCHK(hipMemsetAsync(a, 0, sizeof(double) * 3 * npart, c.stream));
     HIPCHK(hipMemsetAsync(P.lk_cnt, 0, sizeof(int32_t) * (size_t)npart * P.nseg, c.stream));
+    HIPCHK(hipMemsetAsync(P.ct_count, 0, sizeof(int32_t), c.stream));
+    P.ct_ok = true;
   }
   HIPCHK(hipMemsetAsync(c.d_status, 0, sizeof(int32_t) * ST_COUNT, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
@@ -1223,13 +1226,14 @@ int step_overlapped(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       }
       if ((he = hipStreamWaitEvent(sB, c.ev_coll, 0)) != hipSuccess) break;
       // beads_collision with beads_lubforce and the map clearing in its grid
+      c.old_version = 0;   // the next collide is writing the other buffer
       if ((he = launch_bounce_back(c, true)) != hipSuccess) break;
       if ((he = hipEventRecord(c.ev_bb, sB)) != hipSuccess) break;
       c.f_version++;
       if ((prc = mfc_streaming(ctx))) break;
       if ((he = launch_move(c, it == c.p.irelease ? 1 : 0, 1, true)) != hipSuccess) break;
       P.map_old = P.map_cur;
-      if ((prc = links_now(ctx, 1, it, true))) break;
+      if ((prc = links_now(ctx, 1, it))) break;
       if ((he = launch_filling(c, true, nullptr)) != hipSuccess) break;
       c.f_version++;
       if ((prc = mfc_macrovar(ctx))) break;
@@ -1309,7 +1313,7 @@ int mfc_step(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       HIPCHK(launch_move(c, it == c.p.irelease ? 1 : 0, 1, true));
       P.map_old = P.map_cur;
       // links, then the refill with the contact links listed in its grid
-      if ((rc = links_now(ctx, 1, it, true))) return rc;
+      if ((rc = links_now(ctx, 1, it))) return rc;
       if (s + 1 < nsteps && c.p.xkf > 0.0) {
         forcing_modes_host(c);
         drawn = true;

@@ -3,8 +3,8 @@
 // Each member is an ordinary context (its own size, spheres, rates and body
 // force; state created and initialised through the single-box API).  One
 // ensemble step runs the time-loop body of every member with one grid per
-// stage for all of them: collide, contact links, bounce-back
-// (+ lubrication, map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
+// stage for all of them: collide, contact links (members in the
+// reference's order only), bounce-back (+ lubrication, map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
 // per-stage table and finds its member from a block-offset table
 // (off[c] <= blockIdx.x < off[c+1]).  The sequence and the per-member state
 // transitions are exactly those of mfc_step, so a member advanced in the
@@ -12,7 +12,7 @@
 //
 // Steps go in chunks of up to kChunk: the host builds the tables of all the
 // chunk's steps into one pinned buffer and uploads them with ONE plain copy;
-// then the chunk's stage grids (6 per step) run, in graph mode as one
+// then the chunk's stage grids (5 or 6 per step) run, in graph mode as one
 // recorded HIP graph replayed for every chunk of the same launch shapes.
 // The graphs hold kernel nodes only (their table pointers point into the
 // device table buffer); a graph is destroyed before any buffer its nodes
@@ -170,12 +170,15 @@ int build_step(mfc_ens* e, StepTabs& T) {
       T.coll.add(&a, (int)((c.g.ncell + e->collide_bs - 1) / e->collide_bs));
       c.cur ^= 1;
       c.phase = PHASE_PRE_STREAM;
-      c.f_version++;
+      c.old_version = ++c.f_version;
     }
     if (on) {
       int nb = 0, npre = 0;
       const BounceArgs ba = bounce_args(c, true, kContactBlocksPerBox, &nb, &npre);
-      st[0].add(&ba, npre);
+      if (npre) {
+        EHIP(ensure_contacts(c));   // before the chunk; its later steps list their own
+        st[0].add(&ba, npre);
+      }
       st[1].add(&ba, nb);
       c.f_version++;
     }

@@ -131,6 +131,7 @@ struct Particles {
   double2* lk_out = nullptr;   // (f9, ff1) of contact links, taken before the scatter
   uint64_t* ct_list = nullptr; // contact links of the last build: (particle << 40) | link
   int32_t* ct_count = nullptr;
+  bool ct_ok = false;          // the list holds the current map's contact links
   // bounce-back order (MFC_BB_SNAPSHOT or MFC_BB_REFERENCE) and, for the
   // reference order, the per-contact-link table of its evaluation
   int bb_order = 0;
@@ -164,6 +165,7 @@ struct Ctx {
   int cur = 0;
   int phase = PHASE_POST_STREAM;
   uint64_t f_version = 1;
+  uint64_t old_version = 0;   // f_version right after a collide of the current map from the other buffer
   // macroscopic arrays (reference rho/ux/uy/uz), FP64
   double *rho = nullptr, *ux = nullptr, *uy = nullptr, *uz = nullptr;
   int mom = MOM_NONE;
@@ -237,8 +239,10 @@ int segments_per_particle(double rad, int slab);
 int segment_capacity(double rad, int slab);
 int segment_planes(double rad, int npart, int want);
 int segment_links(double rad, int slab);
-// defer_contacts: the contact links are listed by the refill grid that follows
-hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool defer_contacts = false);
+hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep);
+// does the bounce-back need the list of contact links (else it may)?
+bool wants_contacts(const Ctx& c);
+hipError_t ensure_contacts(Ctx& c);
 // ST_NLINKS and ST_NSOLID of the current build
 hipError_t launch_link_totals(Ctx& c);
 // with `fused` set (mfc_step) the bounce-back grid also computes the
@@ -250,7 +254,7 @@ hipError_t launch_map_clear(Ctx& c, int buf);
 hipError_t launch_move(Ctx& c, int first, int wrap, bool from_seg = false);
 hipError_t launch_redistribute(Ctx& c, int istep);
 struct TableJob;
-// contacts: the grid also lists the contact links; job: a forcing table
+// contacts: the grid also lists the contact links, if they are wanted; job: a forcing table
 // evaluated by extra blocks of it
 hipError_t launch_filling(Ctx& c, bool contacts = false, const TableJob* job = nullptr);
 hipError_t launch_initpartvel(Ctx& c);

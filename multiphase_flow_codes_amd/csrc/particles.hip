@@ -1009,13 +1009,32 @@ __device__ void bb_contact_ordered(const BounceArgs& a) {
   }
 }
 
+// Streamed value of direction i at node n of a two-buffer field.
+template <typename T>
+__device__ __forceinline__ double pulled_value(const T* A, const Grid& g, int i, uint32_t n) {
+  int x, y, z, pl;
+  uint32_t row;
+  uint64_t s;
+  node_coords(n, g, x, y, z, row);
+  if (g.walls_y)
+    pull_src_lay<true>(LAY_AB, i, x, y, z, g, pl, s);
+  else
+    pull_src_lay<false>(LAY_AB, i, x, y, z, g, pl, s);
+  return (double)A[(uint64_t)pl * g.pitch + s];
+}
+
 // Pre-pass of the bounce-back.  Contact links (node x solid for another
 // sphere, spheres almost touching) read post-collision values at a solid
 // node, which the bounce-back grid overwrites: their values are taken first,
 // from the untouched field, into lk_out (f9, ff1).  Every other link reads
 // fluid nodes only and writes only solid ones, so the bounce-back grid can
 // scatter as it goes; all links see the one post-collision snapshot.  nct
-// blocks stride over the contact list.
+// blocks stride over the contact list.  With two buffers neither is needed: a
+// solid node's post-collision values are the streamed ones the collide copied,
+// which the other buffer still holds, and a contact link reads them there
+// (one launch less, and the refill grid lists no contact links: 192 x 176 x 208
+// FP32 with 900 spheres 293 to 290 us a step, 64^3 FP64 with 8 48.2 to 46.3, 512^3
+// with 2500 4154 to 4137, 32 boxes in one grid 938 to 932).
 template <typename T>
 __device__ __forceinline__ void bb_contact_body(int b_, const BounceArgs& a) {
   if (a.ref_order) {
@@ -1106,13 +1125,20 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
     const double alpha = a.lk.alpha[l];
     if (n >= g.ncell || q < 1 || q >= NPOP) continue;  // never true for a consistent list
     const bool cont = bit_at(a.mask, n);
-    double ff1 = 0.0, f9 = 0.0, xx0, yy0, zz0;
-    link_bounce<T>(A, g, a.G, a.mask, n, q, alpha, xcp, ycp, zcp, w1, w2, w3, o1, o2, o3, a.ww1,
-                   a.ww2, !cont, ff1, f9, xx0, yy0, zz0);
+    const bool own = cont && a.old;
+    double ff1 = 0.0, f9 = 0.0, xx0, yy0, zz0, was_q = 0.0, was_qbar = 0.0;
+    if (own) {
+      was_q = pulled_value((const T*)a.old, g, q, n);
+      was_qbar = pulled_value((const T*)a.old, g, opp(q), n);
+    }
+    link_bounce<T, true>(A, g, a.G, a.mask, n, q, alpha, xcp, ycp, zcp, w1, w2, w3, o1, o2, o3, a.ww1,
+                         a.ww2, own || !cont, ff1, f9, xx0, yy0, zz0, own, was_q, own, was_qbar);
     if (cont) {
-      const double2 v = a.lk_out[l];
-      f9 = v.x;
-      ff1 = v.y;
+      if (!own) {
+        const double2 v = a.lk_out[l];
+        f9 = v.x;
+        ff1 = v.y;
+      }
       ++contact;
     }
     // scatter: the post-collision value of opp(q) at the solid node x + c
@@ -1533,7 +1559,7 @@ __global__ void __launch_bounds__(kMoveBlock)
 }
 
 // The refill of the previous build's segments, the contact links of the new
-// build's and, in blocks past those, the next step's forcing table.  4 waves
+// build's (where the bounce-back wants their list) and, in blocks past those, the next step's forcing table.  4 waves
 // per SIMD (at most 128 VGPRs; 5 or more spill: 24 to 31 us with 900 spheres of
 // radius 4).  The search in a grid of its own that lists the nodes for a refill
 // grid was no faster but with 15,000 segments (12 + 12 us against 24 with 900
@@ -1791,6 +1817,7 @@ static ContactArgs contact_args(const Particles& P) {
 // (used by the single-box launchers below and by the ensemble engine)
 
 ScanArgs scan_args(Ctx& c, int target, int ovl, int istep) {
+  c.pt.ct_ok = false;   // the scan empties the contact list
   Particles& P = c.pt;
   ScanArgs a;
   a.ypglb = P.ypglb; a.np = P.np; a.nseg = P.nseg; a.seg_cap = P.seg_cap; a.G = pgeom(c);
@@ -1820,7 +1847,8 @@ BounceArgs bounce_args(Ctx& c, bool fused, int nct, int* bb_blocks, int* pre_blo
   a.nsegs = P.np * P.nseg; a.np = P.np; a.lub = lub_args(c);
   a.split = P.bb_split;
   a.ref_order = P.bb_order == MFC_BB_REFERENCE;
-  a.nct = a.ref_order ? 1 : nct;
+  a.old = !a.ref_order && c.g.lay == LAY_AB && c.old_version == c.f_version ? c.pop[c.cur ^ 1] : nullptr;
+  a.nct = a.old ? 0 : (a.ref_order ? 1 : nct);
   a.ord = P.ord; a.ord_cap = P.ord_cap; a.isn = P.isn[P.map_cur];
   a.nlub = fused ? lub_blocks(c) : 0;
   const int t = P.map_cur ^ 1;
@@ -1868,7 +1896,8 @@ FillKArgs fill_args(Ctx& c, bool refill, bool contacts, int* blocks) {
   FillKArgs a;
   a.fa = FillArgs{};
   a.nfill = refill && make_fill_args(c, P.map_old, P.map_cur, a.fa) ? P.map_np[P.map_old] * P.nseg : 0;
-  a.nct = contacts ? P.np * P.nseg : 0;
+  a.nct = contacts && wants_contacts(c) ? P.np * P.nseg : 0;
+  if (a.nct) P.ct_ok = true;
   a.ct = contact_args(P);
   a.A = c.pop[c.cur];
   a.g = c.g;
@@ -2033,7 +2062,7 @@ hipError_t launch_tiles(Ctx& c, TileLists& T) {
 }
 
 // ---- single-box launchers -------------------------------------------------------
-hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool defer_contacts) {
+hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep) {
   Particles& P = c.pt;
   const int nsegs = P.np * P.nseg;
   hipError_t e = launch_map_clear(c, target);
@@ -2045,12 +2074,17 @@ hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep, bool d
   }
   hipLaunchKernelGGL(k_links_scan, dim3(nsegs), dim3(PB), scan_lds(c), c.stream,
                      scan_args(c, target, overlap_check, istep));
-  if (!defer_contacts) {
-    ContactArgs ca = contact_args(P);
-    ca.mask = P.mask[target];
-    hipLaunchKernelGGL(k_contacts, dim3(nsegs), dim3(PB), 0, c.stream, ca);
-  }
   P.map_np[target] = P.np;
+  return hipGetLastError();
+}
+
+bool wants_contacts(const Ctx& c) { return c.g.lay != LAY_AB || c.pt.bb_order == MFC_BB_REFERENCE; }
+
+hipError_t ensure_contacts(Ctx& c) {
+  Particles& P = c.pt;
+  if (P.ct_ok || P.np <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_contacts, dim3(P.np * P.nseg), dim3(PB), 0, c.stream, contact_args(P));
+  P.ct_ok = true;
   return hipGetLastError();
 }
 
@@ -2073,11 +2107,15 @@ hipError_t launch_bounce_back(Ctx& c, bool fused) {
   int nb = 0, npre = 0;
   const BounceArgs ba = bounce_args(c, fused, kContactBlocks, &nb, &npre);
   const size_t lds = fused ? lub_lds(c) : 0;
+  if (npre) {
+    const hipError_t e = ensure_contacts(c);
+    if (e != hipSuccess) return e;
+  }
   if (c.prec == MFC_PREC_FP64) {
-    hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    if (npre) hipLaunchKernelGGL(k_bb_contact<double>, dim3(npre), dim3(PB), 0, c.stream, ba);
     hipLaunchKernelGGL(k_bounce_back<double>, dim3(nb), dim3(PB), lds, c.stream, ba);
   } else {
-    hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), 0, c.stream, ba);
+    if (npre) hipLaunchKernelGGL(k_bb_contact<float>, dim3(npre), dim3(PB), 0, c.stream, ba);
     hipLaunchKernelGGL(k_bounce_back<float>, dim3(nb), dim3(PB), lds, c.stream, ba);
   }
   if (!fused)

@@ -117,6 +117,7 @@ struct ScanArgs {
 // its pre-pass grid (nct blocks for the contact links).
 struct BounceArgs {
   void* A;
+  const void* old;              // the field before the collide, if the other buffer holds it
   Grid g;
   PGeom G;
   const uint32_t* mask;
