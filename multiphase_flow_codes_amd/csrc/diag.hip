@@ -358,9 +358,10 @@ __device__ __forceinline__ void small_pass(const FftArgs& a, const double2* src,
 }
 
 // Any length: passes over the factors of n (4, 2, 3, 5, then the remaining
-// primes by their direct sums) between two LDS buffers.  150 x 141 x 162 nodes
-// (141 = 3 x 47), three components: 0.33 ms; direct sums over whole lines
-// took 4.6 ms.
+// primes by their sums, outputs m and r - m together) between two LDS buffers.
+// Bound: those sums.  A spectrum of 150 x 141 x 162 nodes (141 = 3 x 47) takes
+// 0.25 ms, 0.35 with every output summed by itself, 4.6 with direct sums over
+// whole lines; 139 x 151 x 149 0.50 ms (1.33), 98 x 121 x 169 0.18 (0.26).
 template <int AXIS>
 __global__ void __launch_bounds__(256)
     k_fft_any(FftArgs a) {
@@ -394,24 +395,37 @@ __global__ void __launch_bounds__(256)
       } else if (r == 5) {
         small_pass<5>(a, src, dst, ns, slot);
       } else {
-        // output m of butterfly i: sum over q of entry i + q n/r times
-        // exp(-2 pi i q (k0 / (ns r) + m / r))
-        const int nr = n / r, st = nr / ns;
-        for (int w = threadIdx.x; w < n * a.tx; w += blockDim.x) {
+        // x_q: entry i + q n/r of butterfly i, turned by exp(-2 pi i q k0 / (ns r)).
+        // Outputs m and r - m share the sums over q <= (r - 1) / 2 of cos(2 pi q m / r)
+        // (x_q + x_{r-q}) and sin(2 pi q m / r) (x_q - x_{r-q}): first those sums and
+        // differences in place, then a pair of outputs per thread.
+        const int nr = n / r, st = nr / ns, h = r / 2;
+        for (int w = threadIdx.x; w < nr * h * a.tx; w += blockDim.x) {
+          const int t = w & (a.tx - 1), iq = w >> a.ltx;
+          const int q = iq / nr, i = iq - q * nr, k0 = i % ns;
+          double2 &lo = src[slot(i + (q + 1) * nr, t)], &hi = src[slot(i + (r - 1 - q) * nr, t)];
+          const double2 u = cmul(lo, a.tw[(q + 1) * k0 * st]), v = cmul(hi, a.tw[(r - 1 - q) * k0 * st]);
+          lo = u + v;
+          hi = u - v;
+        }
+        __syncthreads();
+        for (int w = threadIdx.x; w < nr * (h + 1) * a.tx; w += blockDim.x) {
           const int t = w & (a.tx - 1), im = w >> a.ltx;
-          const int m = im / nr, i = im - m * nr, k0 = i % ns;
-          int step = k0 * st + m * nr;
-          if (step >= n) step -= n;
-          double2 s = src[slot(i, t)];
+          const int m = im / nr, i = im - m * nr, k0 = i % ns, step = m * nr;
+          double2 c = src[slot(i, t)], d = make_double2(0.0, 0.0);
           int e = 0;
-          for (int q = 1; q < r; ++q) {
+          for (int q = 1; q <= h; ++q) {
             e += step;
             if (e >= n) e -= n;
-            const double2 v = src[slot(i + q * nr, t)], w1 = a.tw[e];
-            s.x += v.x * w1.x - v.y * w1.y;
-            s.y += v.x * w1.y + v.y * w1.x;
+            const double2 s = src[slot(i + q * nr, t)], f = src[slot(i + (r - q) * nr, t)], cs = a.tw[e];
+            c.x += cs.x * s.x;
+            c.y += cs.x * s.y;
+            d.x -= cs.y * f.y;   // cs.y = -sin
+            d.y += cs.y * f.x;
           }
-          dst[slot((i - k0) * r + k0 + m * ns, t)] = s;
+          const int o = (i - k0) * r + k0;
+          dst[slot(o + m * ns, t)] = c + d;
+          if (m) dst[slot(o + (r - m) * ns, t)] = c - d;
         }
       }
       __syncthreads();
