@@ -147,6 +147,7 @@ int drop_graphs(mfc_ens* e) {
 struct StepTabs {
   StageTab coll, st[kParts];
   bool arr_any = false;
+  int64_t whole_lines = 0;   // nodes in rows of whole 64-B half lines, less those in other rows
 };
 const Stage kOrder[kParts] = {SG_CONTACT, SG_BOUNCE, SG_MOVE, SG_SCAN, SG_FILL};
 
@@ -167,6 +168,7 @@ int build_step(mfc_ens* e, StepTabs& T) {
       CollideArgs a = collide_args(c);
       a.arr = c.mom == MOM_ARRAYS ? 1 : 0;
       T.arr_any = T.arr_any || a.arr;
+      T.whole_lines += (size_t)c.g.nx * c.tsize % 64 == 0 ? (int64_t)c.g.ncell : -(int64_t)c.g.ncell;
       T.coll.add(&a, (int)((c.g.ncell + e->collide_bs - 1) / e->collide_bs));
       c.cur ^= 1;
       c.phase = PHASE_PRE_STREAM;
@@ -269,7 +271,7 @@ int ens_chunk(mfc_ens* e, int n) {
       const StepTabs& U = T[s];
       EHIP(launch_batched_collide(e->prec, e->walls, e->collide_bs, e->collide_remap, d + pos[s][0][0],
                                   (const int*)(d + pos[s][0][1]), U.coll.nc, U.coll.off.back(), U.arr_any,
-                                  e->stream));
+                                  U.whole_lines >= 0, e->stream));
       for (int k = 0; k < kParts; ++k) {
         const StageTab& t = U.st[k];
         EHIP(launch_batched(kOrder[k], e->prec, e->walls, d + pos[s][k + 1][0],
@@ -287,7 +289,7 @@ int ens_chunk(mfc_ens* e, int n) {
     for (int s = 0; s < n; ++s) {
       sig.push_back(T[s].coll.nc);
       sig.push_back(T[s].coll.off.back());
-      sig.push_back(T[s].arr_any ? 1LL : 0LL);
+      sig.push_back((T[s].arr_any ? 1LL : 0LL) + (T[s].whole_lines >= 0 ? 2LL : 0LL));
       for (int k = 0; k < kParts; ++k) {
         sig.push_back(T[s].st[k].nc);
         sig.push_back(T[s].st[k].off.back());

@@ -315,7 +315,13 @@ __device__ __forceinline__ int case_of_block(const int* __restrict__ off, int nc
 // remap = 1 deals the grid to the 8 XCDs in contiguous ranges: consecutive
 // node ranges, whose neighbour rows overlap, then share one L2.  The block-to-nodes map is a bijection either way, so results do
 // not depend on it.
-template <typename T, typename R, bool WALLS, int BS, bool ARR_ANY>
+// NTL: non-temporal loads, where most nodes lie in rows of whole 64-B half lines (32
+// boxes of 32 to 128 nodes an edge FP64 1697 us a step against 1748 plain, FP32 928
+// against 935).  In other rows neighbouring blocks need the same lines: plain
+// loads (100 x 90 x 96 FP32 44 to 35 us, 262 x 257 x 227 774 to 683, FP64 1066 to
+// 1026; 130 x 118 x 126 FP32 99 to 72).  One grid, one kind: with both in one
+// kernel it needs 99 instead of 71 VGPRs (FP64 176 instead of 132) and loses.
+template <typename T, typename R, bool WALLS, int BS, bool ARR_ANY, bool NTL>
 __global__ void __launch_bounds__(BS)
     kb_collide(const CollideArgs* __restrict__ t, const int* __restrict__ off, int nc, int remap) {
   const uint32_t b = xcd_block(blockIdx.x, remap ? gridDim.x / kXcds : 0);
@@ -327,9 +333,9 @@ __global__ void __launch_bounds__(BS)
   uint32_t row;
   node_coords((uint32_t)n, a.g, x, y, z, row);
   if (ARR_ANY && a.arr)
-    collide_node<T, R, true, WALLS, LAY_AB, true, true>(a, x, y, z);
+    collide_node<T, R, true, WALLS, LAY_AB, NTL, true>(a, x, y, z);
   else
-    collide_node<T, R, false, WALLS, LAY_AB, true, true>(a, x, y, z);
+    collide_node<T, R, false, WALLS, LAY_AB, NTL, true>(a, x, y, z);
 }
 
 // Forcing table of one step (force_table.h): one thread per (row, component).
@@ -918,43 +924,46 @@ hipError_t launch_force_field(Ctx& c, int slot, double* fx, double* fy, double* 
 namespace mfc {
 
 template <typename T, typename R, int BS, bool ARR_ANY>
-static void batched_collide_k(int walls, const CollideArgs* tab, const int* off, int nc, int blocks,
-                              int remap, hipStream_t s) {
-  if (walls)
-    hipLaunchKernelGGL((kb_collide<T, R, true, BS, ARR_ANY>), dim3(blocks), dim3(BS), 0, s, tab, off, nc,
-                       remap);
-  else
-    hipLaunchKernelGGL((kb_collide<T, R, false, BS, ARR_ANY>), dim3(blocks), dim3(BS), 0, s, tab, off, nc,
-                       remap);
+static void batched_collide_k(int walls, const CollideArgs* t, const int* off, int nc, int blocks, int remap,
+                              bool ntl, hipStream_t s) {
+#define MFC_BATCHED(W, N) \
+  hipLaunchKernelGGL((kb_collide<T, R, W, BS, ARR_ANY, N>), dim3(blocks), dim3(BS), 0, s, t, off, nc, remap)
+  // a first step after joining (ARR_ANY) is rare: non-temporal only
+  if (ARR_ANY || ntl) {
+    if (walls) MFC_BATCHED(true, true); else MFC_BATCHED(false, true);
+  } else {
+    if (walls) MFC_BATCHED(true, ARR_ANY); else MFC_BATCHED(false, ARR_ANY);
+  }
+#undef MFC_BATCHED
 }
 
 template <int BS, bool ARR_ANY>
 static void batched_collide_bs(int prec, int walls, const void* t, const int* off, int nc, int blocks,
-                               int remap, hipStream_t s) {
+                               int remap, bool ntl, hipStream_t s) {
   const CollideArgs* tab = (const CollideArgs*)t;
   if (prec == MFC_PREC_FP64)
-    batched_collide_k<double, double, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, s);
+    batched_collide_k<double, double, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, ntl, s);
   else if (prec == MFC_PREC_FP32_F64MATH)
-    batched_collide_k<float, double, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, s);
+    batched_collide_k<float, double, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, ntl, s);
   else
-    batched_collide_k<float, float, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, s);
+    batched_collide_k<float, float, BS, ARR_ANY>(walls, tab, off, nc, blocks, remap, ntl, s);
 }
 
 hipError_t launch_batched_collide(int prec, int walls, int bs, int remap, const void* t, const int* off,
-                                  int nc, int blocks, bool arr_any, hipStream_t s) {
+                                  int nc, int blocks, bool arr_any, bool ntl, hipStream_t s) {
   if (nc <= 0 || blocks <= 0) return hipSuccess;
   switch (bs) {
     case 64:
-      arr_any ? batched_collide_bs<64, true>(prec, walls, t, off, nc, blocks, remap, s)
-              : batched_collide_bs<64, false>(prec, walls, t, off, nc, blocks, remap, s);
+      arr_any ? batched_collide_bs<64, true>(prec, walls, t, off, nc, blocks, remap, ntl, s)
+              : batched_collide_bs<64, false>(prec, walls, t, off, nc, blocks, remap, ntl, s);
       break;
     case 128:
-      arr_any ? batched_collide_bs<128, true>(prec, walls, t, off, nc, blocks, remap, s)
-              : batched_collide_bs<128, false>(prec, walls, t, off, nc, blocks, remap, s);
+      arr_any ? batched_collide_bs<128, true>(prec, walls, t, off, nc, blocks, remap, ntl, s)
+              : batched_collide_bs<128, false>(prec, walls, t, off, nc, blocks, remap, ntl, s);
       break;
     case 256:
-      arr_any ? batched_collide_bs<256, true>(prec, walls, t, off, nc, blocks, remap, s)
-              : batched_collide_bs<256, false>(prec, walls, t, off, nc, blocks, remap, s);
+      arr_any ? batched_collide_bs<256, true>(prec, walls, t, off, nc, blocks, remap, ntl, s)
+              : batched_collide_bs<256, false>(prec, walls, t, off, nc, blocks, remap, ntl, s);
       break;
     default: return hipErrorInvalidValue;
   }

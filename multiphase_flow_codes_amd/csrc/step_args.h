@@ -192,7 +192,7 @@ hipError_t launch_batched(Stage st, int prec, int walls, const void* t, const in
                           int blocks, size_t lds, hipStream_t s);
 // arr_any: some member's CollideArgs::arr is set
 hipError_t launch_batched_collide(int prec, int walls, int bs, int remap, const void* t, const int* off,
-                                  int nc, int blocks, bool arr_any, hipStream_t s);
+                                  int nc, int blocks, bool arr_any, bool ntl, hipStream_t s);
 size_t stage_arg_bytes(Stage st);
 
 }  // namespace mfc
