@@ -263,10 +263,11 @@ int need_arrays(mfc_ctx* ctx, bool* fill = nullptr) {
     if (c.rho && c.arrays_version == c.mom_version) return MFC_OK;
     int rc = ensure_macro(ctx);
     if (rc) return rc;
-    if (fill)
+    if (fill) {
       *fill = true;
-    else
-      HIPCHK(launch_macro(c, c.phase == PHASE_POST_STREAM));
+      return MFC_OK;
+    }
+    HIPCHK(launch_macro(c, c.phase == PHASE_POST_STREAM));
     c.arrays_version = c.mom_version;
     return MFC_OK;
   }
@@ -1357,6 +1358,7 @@ int mfc_diag_sums(mfc_ctx* ctx, double* out6) {
   bool fill = false;
   if ((rc = need_arrays(ctx, &fill))) return rc;
   HIPCHK(launch_field_sums(c, fill, c.diag_part, c.diag_out));
+  if (fill) c.arrays_version = c.mom_version;
   const HostPart part = {out6, c.diag_out, sizeof(double) * 6};
   HIPCHK(copy_to_host(c, &part, 1));
   return MFC_OK;
@@ -1375,10 +1377,10 @@ int mfc_diag_sums_noalloc(mfc_ctx* ctx, double* out6) {
   if (c.mom != MOM_ARRAYS && (c.mom != MOM_VIRTUAL || c.mom_version != c.f_version))
     return fail(ctx, MFC_ERR_STATE, "rho/u requested after the field changed since macrovar");
   const bool fill = c.mom != MOM_ARRAYS && c.arrays_version != c.mom_version;
-  if (fill) c.arrays_version = c.mom_version;
   double* part = c.sums_scratch;
   double* res = part + nsum;
   HIPCHK(launch_field_sums(c, fill, part, res));
+  if (fill) c.arrays_version = c.mom_version;
   HIPCHK(hipMemcpyAsync(out6, res, sizeof(double) * 6, hipMemcpyDeviceToDevice, c.stream));
   return MFC_OK;
 }
