@@ -468,8 +468,9 @@ __global__ void __launch_bounds__(PB)
 // lists in memory, a grid for the sum, a grid to write the links and find the
 // nodes to refill) the rebuild and the refill took 88 us at 256^3 with 300
 // spheres of radius 8, 82 us with 900 of radius 4, 284 us with 2500 of radius
-// 6 and 33 us at 64^3 in FP64 with 8 of radius 4; now 68, 58, 248 and 21
-// us.  Of that the scan was 66, 52, 220 and 13.5 us while each node searched the
+// 6 and 33 us at 64^3 in FP64 with 8 of radius 4; with slots 68, 58, 248 and 21
+// us, and 62 to 70, 49, 189 and 17 with the segment sizes chosen since and no list
+// of contact links.  Of the slots' times the scan was 66, 52, 220 and 13.5 us while each node searched the
 // rows' starts for its row and took the image of the centre by itself and each
 // direction squared its own offsets: 44, 34, 144 and 11.3 us with the rows'
 // numbers and geometry in LDS and the squares shared.
