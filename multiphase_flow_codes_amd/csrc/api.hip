@@ -811,6 +811,9 @@ int mfc_macrovar(mfc_ctx* ctx) {
   if (c.phase != PHASE_POST_STREAM) return fail(ctx, MFC_ERR_STATE, "macrovar expects the streamed field");
   c.mom = MOM_VIRTUAL;
   c.mom_version = c.f_version;
+  // what the arrays hold is of an earlier macrovar: the field may be the same,
+  // but not the arrays (overwritten since), the forcing or the spheres
+  c.arrays_version = 0;
   c.ft.mac = c.ft.cur;
   return MFC_OK;
 }

@@ -170,7 +170,7 @@ struct Ctx {
   double *rho = nullptr, *ux = nullptr, *uy = nullptr, *uz = nullptr;
   int mom = MOM_NONE;
   uint64_t mom_version = 0;
-  uint64_t arrays_version = 0;      // MOM_VIRTUAL: the macrovar whose rho/u the arrays hold (0: none)
+  uint64_t arrays_version = 0;      // MOM_VIRTUAL: mom_version if the arrays hold that macrovar's rho/u (0: not)
   ForceTables ft;
   // host forcing state (gaussian.f90 FORCING)
   int32_t iseedf = 0, iyf = 0, ivf[32] = {0};
