@@ -159,8 +159,9 @@ hipError_t wait_flag(const uint32_t* flag, uint32_t value, hipStream_t s) {
 }
 
 // Copies the parts to the host after the work queued on the context's stream
-// and waits for them.
+// and waits for them (no parts: for that work).
 hipError_t copy_to_host(Ctx& c, const HostPart* part, int nparts) {
+  if (nparts == 0) return hipStreamSynchronize(c.stream);
   CopyJob j{};
   uint32_t units = 0;
   bool plain = c.pipe_dev < 0;

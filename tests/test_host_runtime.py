@@ -1,0 +1,70 @@
+"""What the host side of the library allocates, copies and launches, seen by a
+HIP runtime that runs on the CPU and computes nothing (tests/native/fake_hip.cpp):
+libmfc_lbm.so is loaded in a process of its own, behind that runtime."""
+import os
+import shutil
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PREAMBLE = """
+import ctypes as C, os, sys
+sys.path[:0] = [{root!r}, {here!r}]
+fake = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
+fake.fake_max_lds.restype = fake.fake_allocated.restype = C.c_size_t
+fake.fake_set_free.argtypes = [C.c_size_t]
+import numpy as np
+from helpers import small_params
+from multiphase_flow_codes_amd.lbm import Lattice, lib, _dp
+def lattice(n=(20, 18, 16), precision="fp64", storage="ab", **kw):
+    return Lattice(small_params(n=n, forcing=False, **kw), precision, storage=storage)
+def fields(n, seed=0):
+    rng = np.random.default_rng(seed)
+    return [rng.normal(size=n[::-1]) for _ in range(4)]
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """Runs a piece of code behind the CPU runtime."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    fake = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run([gxx, "-O1", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Werror", "-o", fake,
+                    os.path.join(HERE, "native", "fake_hip.cpp")], check=True, timeout=300)
+
+    def go(code, **env):
+        pre = PREAMBLE.format(root=ROOT, here=HERE, fake=fake)
+        r = subprocess.run([sys.executable, "-c", pre + textwrap.dedent(code) + "\nprint('done')"],
+                           capture_output=True, text=True, timeout=300, env=dict(os.environ, **env))
+        assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+
+    return go
+
+
+def test_fields_come_back(run):
+    run("""
+        for n in ((4, 4, 4), (17, 16, 8), (64, 64, 32), (75, 71, 73)):
+            lat, a = lattice(n), fields(n)
+            lat.upload_macro(*a)
+            for x, y in zip(lat.download_macro(), a):
+                assert np.array_equal(x, y)
+    """)
+
+
+def test_download_of_nothing_succeeds(run):
+    """Each target of mfc_download_macro may be null, all of them too."""
+    run("""
+        lat, a = lattice(), fields((20, 18, 16))
+        lat.upload_macro(*a)
+        assert lib().mfc_download_macro(lat.h, None, None, None, None) == 0
+        uy = np.empty_like(a[2])
+        assert lib().mfc_download_macro(lat.h, None, None, _dp(uy), None) == 0
+        assert np.array_equal(uy, a[2])
+    """)
