@@ -530,6 +530,7 @@ int mfc_status(mfc_ctx* ctx, int32_t* out16) {
   NEEDCTX;
   if (!out16) return MFC_ERR_ARG;
   Ctx& c = ctx->c;
+  const OnDevice here(c.pipe_dev);
   HIPCHK(launch_link_totals(c));
   const HostPart part = {c.h_status, c.d_status, sizeof(int32_t) * ST_COUNT};
   HIPCHK(copy_to_host(c, &part, 1));

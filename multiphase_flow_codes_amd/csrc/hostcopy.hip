@@ -15,7 +15,9 @@
 // 2.5 ms) but starved beside a program's own thread pool (17.7 MB 0.6 to 5 ms).
 //
 // The windows belong to a device and are shared by its contexts: allocated at
-// the first copy, freed with the last context.  A copy that finds them in use by
+// the first copy, freed with the last context.  The calling thread's current
+// device may be another one (a thread starts on device 0): it is the context's
+// while a copy allocates and launches.  A copy that finds them in use by
 // another host thread takes the runtime's path.
 #include <mutex>
 #include <thread>
@@ -127,6 +129,17 @@ bool prepare(Pipe& P, int windows, hipStream_t s) {
 
 }  // namespace
 
+OnDevice::OnDevice(int dev) {
+  int now = -1;
+  ok = dev >= 0 && hipGetDevice(&now) == hipSuccess;
+  if (!ok || now == dev) return;
+  ok = hipSetDevice(dev) == hipSuccess;
+  if (ok) was = now;
+}
+OnDevice::~OnDevice() {
+  if (was >= 0) (void)hipSetDevice(was);
+}
+
 void host_pipe_ref(int dev) {
   std::lock_guard<std::mutex> lk(g_pipe[dev].mu);
   ++g_pipe[dev].refs;
@@ -175,6 +188,8 @@ hipError_t copy_to_host(Ctx& c, const HostPart* part, int nparts) {
   }
   j.unit0[nparts] = units;
   j.nparts = nparts;
+  const OnDevice here(plain ? -1 : c.pipe_dev);
+  plain = plain || !here.ok;
   std::unique_lock<std::mutex> own;
   if (!plain) {
     own = std::unique_lock<std::mutex>(g_pipe[c.pipe_dev].use, std::try_to_lock);

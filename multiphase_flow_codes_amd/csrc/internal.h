@@ -272,6 +272,16 @@ struct HostPart {
   size_t bytes;
 };
 constexpr int kMaxParts = 4;
+// the device is current for the calling thread while the object lives
+struct OnDevice {
+  explicit OnDevice(int dev);
+  ~OnDevice();
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+  bool ok = false;   // false: it could not be set
+ private:
+  int was = -1;
+};
 hipError_t copy_to_host(Ctx& c, const HostPart* part, int nparts);   // waits
 hipError_t wait_flag(const uint32_t* flag, uint32_t value, hipStream_t s);
 void host_pipe_ref(int dev);     // a context of the device was created

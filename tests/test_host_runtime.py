@@ -68,3 +68,38 @@ def test_download_of_nothing_succeeds(run):
         assert lib().mfc_download_macro(lat.h, None, None, _dp(uy), None) == 0
         assert np.array_equal(uy, a[2])
     """)
+
+
+def test_results_of_another_device(run):
+    """Contexts of device 1 read by threads whose current device is 0: what such
+    a read allocates and launches is on device 1, and 0 stays current."""
+    run("""
+        import threading
+        a, got = fields((20, 18, 16)), []
+        fake.hipSetDevice(1)
+        lat = lattice(npart=2, rad=3.0)
+        lat.prt_init(2)
+        lat.upload_macro(*a)
+        lat.prt_set("ypglb", np.array([[5.0, 5.0, 5.0], [14.0, 12.0, 11.0]]))
+        lat.beads_links()
+        fake.fake_reset()
+
+        def read():
+            lat.sync()
+            lat.status()
+            got.extend(lat.download_macro())
+            got.append(lat.prt_get("ypglb"))
+            d = C.c_int(-1)
+            fake.hipGetDevice(C.byref(d))
+            got.append(d.value)
+
+        t = threading.Thread(target=read)
+        t.start()
+        t.join()
+        assert len(got) == 6 and got[5] == 0
+        for x, y in zip(got, a):
+            assert np.array_equal(x, y)
+        assert got[4][1, 0] == 14.0
+        assert fake.fake_launches(b"k_copy_out") == 4 and fake.fake_launches(b"k_link_totals") == 1
+        assert fake.fake_foreign() == 0
+    """)
