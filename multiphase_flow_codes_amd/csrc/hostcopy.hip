@@ -171,21 +171,45 @@ hipError_t wait_flag(const uint32_t* flag, uint32_t value, hipStream_t s) {
   }
 }
 
+// Is the target left to the runtime's own copy?  Memory the thread cannot be
+// relied on to write (a device's, managed) always, pinned memory where the bus
+// alone is the faster: four arrays of 2.1 MB 185 us against 308 through the
+// windows, of 885 KB 102 against 165, of 262 KB 55 against 53, of 85 KB 42 against 24.
+static bool runtime_target(const HostPart& part) {
+  constexpr size_t kPinnedFrom = (size_t)1 << 19;
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, part.host) != hipSuccess) {
+    (void)hipGetLastError();   // ordinary memory
+    return false;
+  }
+  if (a.type == hipMemoryTypeHost) return part.bytes >= kPinnedFrom;
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 // Copies the parts to the host after the work queued on the context's stream
 // and waits for them (no parts: for that work).
-hipError_t copy_to_host(Ctx& c, const HostPart* part, int nparts) {
-  if (nparts == 0) return hipStreamSynchronize(c.stream);
+hipError_t copy_to_host(Ctx& c, const HostPart* all, int nall) {
   CopyJob j{};
+  HostPart part[kMaxParts];
+  int nparts = 0;
   uint32_t units = 0;
   bool plain = c.pipe_dev < 0;
-  for (int k = 0; k < nparts; ++k) {
-    j.dev[k] = (const char*)part[k].dev;
-    j.bytes[k] = part[k].bytes;
-    j.unit0[k] = units;
-    const uint64_t n = (part[k].bytes + kUnit - 1) / kUnit;
-    if (n == 0 || n > (1u << 24) || part[k].bytes % 4 != 0) plain = true;
+  for (int k = 0; k < nall; ++k) {
+    if (runtime_target(all[k])) {
+      const hipError_t e = hipMemcpyAsync(all[k].host, all[k].dev, all[k].bytes, hipMemcpyDeviceToHost, c.stream);
+      if (e != hipSuccess) return e;
+      continue;
+    }
+    part[nparts] = all[k];
+    j.dev[nparts] = (const char*)all[k].dev;
+    j.bytes[nparts] = all[k].bytes;
+    j.unit0[nparts] = units;
+    const uint64_t n = (all[k].bytes + kUnit - 1) / kUnit;
+    if (n == 0 || n > (1u << 24) || all[k].bytes % 4 != 0) plain = true;
     units += (uint32_t)n;
+    ++nparts;
   }
+  if (nparts == 0) return hipStreamSynchronize(c.stream);
   j.unit0[nparts] = units;
   j.nparts = nparts;
   const OnDevice here(plain ? -1 : c.pipe_dev);

@@ -103,3 +103,30 @@ def test_results_of_another_device(run):
         assert fake.fake_launches(b"k_copy_out") == 4 and fake.fake_launches(b"k_link_totals") == 1
         assert fake.fake_foreign() == 0
     """)
+
+
+@pytest.mark.parametrize("alloc,n,copies", [
+    ("hipHostMalloc", (64, 60, 62), 1),   # large: the bus reaches pinned memory without the thread's copy
+    ("hipHostMalloc", (20, 18, 16), 0),   # small: the windows are faster
+    ("hipMalloc", (64, 60, 62), 1),
+    ("hipMalloc", (20, 18, 16), 1),       # the thread may not be able to write it
+])
+def test_targets_the_runtime_knows(run, alloc, n, copies):
+    """Results for memory of the runtime's own are left to its copy, those for
+    ordinary memory beside them still go through the windows."""
+    run(f"""
+        n = {n}
+        size = n[0] * n[1] * n[2]
+        lat, a = lattice(n), fields(n)
+        lat.upload_macro(*a)
+        p, out = C.c_void_p(), np.empty(n[::-1])
+        assert fake.{alloc}(C.byref(p), C.c_size_t(8 * size), 0) == 0
+        p = C.cast(p, C.POINTER(C.c_double))
+        for target in (None, _dp(out)):
+            fake.fake_reset()
+            assert lib().mfc_download_macro(lat.h, None, p, None, target) == 0
+            assert np.array_equal(np.ctypeslib.as_array(p, (size,)), a[1].ravel())
+            assert fake.fake_copies() == {copies}
+            assert (fake.fake_launches(b"k_copy_out") > 0) == (target is not None or not {copies})
+        assert np.array_equal(out, a[3])
+    """)
