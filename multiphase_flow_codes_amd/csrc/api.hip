@@ -33,16 +33,24 @@ constexpr int kTimingPool = 8192;
 constexpr int64_t kOrderCap = int64_t(1) << 16;
 
 // Elements from one direction's row to the next in the row-interleaved layout:
-// nx rounded up to whole 128-B lines where that adds at most a tenth, else to
-// 64 B, so that a wavefront's run of a row starts on a line and two rows never
-// share one.  Two buffers only: in place the unwritten ends of the lines cost
-// more than the shared ones (150 x 141 x 162 FP64 240 us padded, 200 not).
-// Fluid steps, two buffers: 150 x 141 x 162 FP32 111-149 us unpadded and 98
-// padded, 1000 x 400 x 128 FP32 1562 us at 64 B and 1385 at 128 B.
+// nx rounded up to whole 128-B lines, else to 64 B, where that adds little, so
+// that a wavefront's run of a row starts on a line and two rows never share one.
+// Two buffers only: in place the unwritten ends of the lines cost more than the
+// shared ones (150 x 141 x 162 FP64 240 us padded, 200 not).  The padding is
+// memory and traffic too.  It pays in rows of more than a tile of 64 nodes
+// (fluid steps, us, unpadded / 64 B / 128 B, 24 million nodes unless said: FP32
+// nx = 300 944 / 679 / 643, 150 888 / 776 / 777, 115 867 / 830 / 847, 90 854 / 883 / 842
+// and 66 / 58 / 58 with 2 million; 150 x 141 x 162 FP32 111-149 unpadded, 98 padded,
+// 1000 x 400 x 128 FP32 1562 at 64 B, 1385 at 128 B) while it adds up to an
+// eighth, in rows of up to 112 nodes up to a fourteenth (FP32 nx = 100, 12 %,
+// 825 / 900, 70, 14 %, 830 / 995, FP64 66, 9 %, 1452 / 1663).  In rows of one tile
+// it never does (FP32 nx = 60, 7 %, 656 / 1046, 33 714 / 1606, 17 987 / 2395, FP64
+// 50, 12 %, 1244 / 1729, 36 1331 / 1881).
 uint64_t row_pitch(uint64_t nx, size_t tsize, bool two_buffers) {
-  if (!two_buffers) return nx;
+  if (!two_buffers || nx <= (uint64_t)kTileX) return nx;
   const uint64_t b = nx * tsize, line = (b + 127) / 128 * 128, half = (b + 63) / 64 * 64;
-  return (10 * line <= 11 * b ? line : half) / tsize;
+  if (nx <= 112) return (14 * line <= 15 * b ? line : (14 * half <= 15 * b ? half : b)) / tsize;
+  return (10 * line <= 11 * b ? line : (8 * half <= 9 * b ? half : b)) / tsize;
 }
 
 int fail(mfc_ctx* ctx, int code, const char* what, hipError_t e = hipSuccess) {
@@ -392,13 +400,12 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
   }
   {
     // Population layout.  By default the 19 planes' rows of one (y, z) lie
-    // side by side (pitch = nx, rs = 19 nx): a collide workgroup's 38
-    // streams then fall in a few neighbouring pages instead of 38 planes
-    // 4 GB apart.  Measured against the plane-major layout, alternating in
+    // side by side (pitch = nx, in two buffers padded as row_pitch says; rs =
+    // 19 pitch): a collide workgroup's 38 streams then fall in a few
+    // neighbouring pages instead of 38 planes 4 GB apart.  Measured against the plane-major layout, alternating in
     // one box: FP32 collide 2.6 % faster at 1024^3 and 8 % at 256^3 (step
     // 2.5 % and 5 %), FP64 in place 2.3 % faster at 1024^3, FP64 and FP32
-    // storage with FP64 collision unchanged at 256^3.  Rows are padded as
-    // row_pitch says.
+    // storage with FP64 collision unchanged at 256^3.
     // MFC_POP_LAYOUT=planes selects plane-major planes instead, 512 B
     // further apart than the node count (a power-of-two plane size would
     // start every stream at the same offset of each page; 512 B measured
@@ -412,6 +419,14 @@ int mfc_create(const mfc_params* p, mfc_ctx** out) {
       c.g.rs = (uint64_t)c.g.nx;
     } else {
       c.g.pitch = row_pitch((uint64_t)c.g.nx, c.tsize, c.g.lay == LAY_AB);
+      // a box that takes most of the memory stays unpadded: what fits without
+      // the padding is not refused for it (the rest of a box, its fields above
+      // all, is less than half of its two populations)
+      size_t room = 0, total = 0;
+      if (c.g.pitch > (uint64_t)c.g.nx &&
+          (hipMemGetInfo(&room, &total) != hipSuccess ||
+           3 * (2 * NPOP * c.tsize * c.g.pitch * (ncell / c.g.nx)) > 2 * (uint64_t)room))
+        c.g.pitch = (uint64_t)c.g.nx;
       c.g.rs = (uint64_t)NPOP * c.g.pitch;
     }
   }

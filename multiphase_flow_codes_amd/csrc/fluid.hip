@@ -2,10 +2,9 @@
 //
 // Storage: populations are SoA, direction i of node (x, y, z) at
 // pop[i * pitch + x + rs * (y + ny*z)]: by default the 19 directions' rows of
-// one (y, z) side by side (pitch = nx, rs = 19 nx), else whole planes
-// (rs = nx, pitch = the node count plus 512 B); in FP64 or FP32 (deviations
-// f_i - w_i*rho0).  The resident buffer holds the
-// post-collision (pre-streaming) field; streaming is never a separate pass:
+// one (y, z) side by side (pitch = nx or a little more, rs = 19 pitch), else
+// whole planes (rs = nx, pitch = the node count plus 512 B); in FP64 or FP32
+// (deviations f_i - w_i*rho0).  The resident buffer holds the post-collision (pre-streaming) field; streaming is never a separate pass:
 // every consumer pulls f_i(x) = buf[i][x - c_i] (half-way bounce-back at the
 // y walls when they are on).  One kernel therefore streams, takes moments,
 // evaluates the forcing field and collides, reading 19 and writing 19

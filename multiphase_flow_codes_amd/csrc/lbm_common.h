@@ -97,8 +97,8 @@ struct Grid {
   // Population element of (plane q, node x + nx*(y + ny*z)):
   //   q * pitch + x + rs * (y + ny*z).
   // Plane-major layout: pitch >= ncell, rs = nx (each plane a contiguous
-  // field).  Row-interleaved layout: pitch = nx, rs = 19*nx (the 19 planes'
-  // rows of one (y, z) side by side).
+  // field).  Row-interleaved layout: pitch = nx or a little more (row_pitch),
+  // rs = 19*pitch (the 19 planes' rows of one (y, z) side by side).
   uint64_t pitch;     // elements from one population plane to the next
   uint64_t rs;        // elements from one row of a plane to the next row
   FastDiv dx, dy;     // division by nx and ny

@@ -93,9 +93,16 @@ class BoxCase:
         t = 8 if precision == "fp64" else 4
         n, np_, r = self.n, self.npart, self.rad
         ncell = n ** 3
-        # rows padded to whole 128-B lines where that adds at most a tenth, else to 64 B
-        line, half = -(-n * t // 128) * 128, -(-n * t // 64) * 64
-        allocs = [19 * n * n * (line if 10 * line <= 11 * n * t else half)] * 2 + [8 * 18 * n * n] * 4 + [8 * 6 * n, 64, 64] + [8 * ncell] * 4
+        # rows padded as the library's row_pitch does
+        b = n * t
+        line, half = -(-b // 128) * 128, -(-b // 64) * 64
+        if n <= 64:
+            row = b
+        elif n <= 112:
+            row = line if 14 * line <= 15 * b else half if 14 * half <= 15 * b else b
+        else:
+            row = line if 10 * line <= 11 * b else half if 8 * half <= 9 * b else b
+        allocs = [19 * n * n * row] * 2 + [8 * 18 * n * n] * 4 + [8 * 6 * n, 64, 64] + [8 * ncell] * 4
         if np_ > 0:
             allocs += [8 * 3 * np_] * 16
             maxcnt = math.ceil(2.0 * (r + 2.0) + 1.0) + 4

@@ -130,3 +130,36 @@ def test_targets_the_runtime_knows(run, alloc, n, copies):
             assert (fake.fake_launches(b"k_copy_out") > 0) == (target is not None or not {copies})
         assert np.array_equal(out, a[3])
     """)
+
+
+def test_padding_of_rows_is_bounded(run):
+    """Two buffers take at most an eighth more than their 19 values per node,
+    rows of up to 64 nodes no more than those; and a lattice that fits the
+    memory without padding is made (and read back) however little is left."""
+    run("""
+        def populations(n, precision):
+            before = fake.fake_allocated()
+            lat = lattice(n, precision)
+            got = fake.fake_allocated() - before
+            # forcing tables, phase tables and the rest of a context
+            rest = 4 * 8 * 18 * n[1] * n[2] + 16 * sum(n) + 8 * (16384 + 1024) + 4096
+            lat.close()
+            return got, rest
+
+        for precision, size in (("fp32", 4), ("fp64", 8), ("fp32x", 4)):
+            for nx in list(range(4, 40)) + [48, 50, 63, 64, 65, 66, 70, 75, 90, 96, 100, 111, 112, 113, 115, 120,
+                                            129, 130, 150, 170, 200, 257, 262, 300, 1000]:
+                n = (nx, 24, 20)
+                need = 2 * 19 * size * nx * n[1] * n[2]
+                got, rest = populations(n, precision)
+                assert need <= got <= (need if nx <= 64 else need * 9 // 8) + rest, (precision, nx, got, need)
+
+        n = (150, 24, 20)
+        size = 8 * n[0] * n[1] * n[2]
+        tight = 2 * 19 * size + 4 * 8 * 18 * n[1] * n[2] + 4 * size + (1 << 19)
+        a = fields(n)
+        fake.fake_set_free(tight)
+        lat = lattice(n)
+        lat.upload_macro(*a)
+        assert all(np.array_equal(x, y) for x, y in zip(lat.download_macro(), a))
+    """)
