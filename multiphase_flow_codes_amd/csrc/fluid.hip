@@ -607,7 +607,11 @@ CollideArgs collide_args(Ctx& c) {
 //  waves   4 wavefronts per workgroup, 3 where rows are a multiple of three
 //          tiles, so that workgroups hold whole rows (192 x 176 x 208 FP32 step
 //          with spheres 282 against 284); 1 where the lattice has at most
-//          16 tiles per CU (48^3 FP64 f 8.7 against 9.1).
+//          16 tiles per CU (48^3 FP64 f 8.7 against 9.1), and in FP64 rows of
+//          up to three quarters of a tile, whose idle lanes leave the wavefront
+//          slots as the bound (24 million nodes: nx = 5 f 5.62 against 6.79 ms,
+//          17 1.87 against 2.20, 48 1.15 against 1.21; nx = 50 1.32 against
+//          1.24; FP32 nx = 17 0.96 and 0.99).
 //  cached  plain stores where both buffers stay in the 256 MiB last-level
 //          cache between steps: from 48 MiB (64^3 FP32, 38 MiB, s 13.1 against
 //          11.6 non-temporal; 64^3 FP64, 76 MiB, s 18.6 against 20.2, f 14.0
@@ -616,7 +620,12 @@ CollideArgs collide_args(Ctx& c) {
 //  ntl     non-temporal loads.  Small lattices (up to 48 MiB: 48^3 FP32 f 5.6
 //          against 6.3).  FP64 with spheres (256^3 s 860 against 897, 448 x
 //          256 x 256 s 1536 against 1570; without them f 877 against 875, 262
-//          x 257 x 227 f 841 against 811).  FP32 storage with FP64 arithmetic
+//          x 257 x 227 f 841 against 811; in ragged rows with spheres it is
+//          nearly even: 262 x 257 x 227 s 937 against 929, 200 x 190 x 210 s 518
+//          against 530, 150 x 141 x 162 s 241 against 243), and large FP64
+//          lattices without spheres in rows of whole 64-B half lines (64 x 160
+//          x 1000 f 494 against 518, 192 x 256 x 488 1174 against 1187; 75 x 256 x
+//          1250 1346-1480 and 1412-1515).  FP32 storage with FP64 arithmetic
 //          with spheres (256^3 s 454 against 474, 262 x 257 x 227 s 486
 //          against 491) and in rows of whole workgroups (256^3 f 442 against
 //          451, but 262 x 257 x 227 f 468 against 450).  FP32 with spheres
@@ -628,7 +637,12 @@ CollideArgs collide_args(Ctx& c) {
 //          FP32 f 3.36 against 3.45-3.61 ms, 1024^3 26.6 against 29.1 ms; 320
 //          x 288 x 304 FP32 f 759 against 719), and in lattices up to 128 MiB,
 //          whose nodes then meet the same L2 in the next step (40^3 FP32 f 5.0
-//          against 6.2).  In place: always (1024^3 FP64 f 52.5 against 64 ms,
+//          against 6.2).  FP64 without spheres from 2.5 GiB (64 x 256 x 1464 f
+//          1173 against 1280 us, 100 x 256 x 937 1306 against 1453, 256^3 822
+//          against 867; 200^3, 2.3 GiB, 426 against 413), in rows of more than four
+//          tiles from 6 GiB (384 x 256 x 256 1261 against 1315; 262 x 200 x 200
+//          575 against 545), in rows of 32 nodes or more (20 x 256 x 2000 771
+//          against 721).  In place: always (1024^3 FP64 f 52.5 against 64 ms,
 //          130 x 118 x 126 FP32 47 against 58), but rows of up to four tiles
 //          that outgrow the last-level cache (200 x 190 x 210 FP64 f 461
 //          against 441).
@@ -649,7 +663,8 @@ static CollideShape collide_shape(const Ctx& c, bool spheres) {
   const uint32_t tpr = (uint32_t)((c.g.nx + kTileX - 1) / kTileX);
   s.t.tpr = fast_div(tpr);
   s.t.ntiles = tpr * (uint32_t)c.g.ny * (uint32_t)c.g.nz;
-  s.t.waves = s.t.ntiles <= 4096 ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
+  const bool all64 = sizeof(T) == 8;
+  s.t.waves = s.t.ntiles <= 4096 || (all64 && c.g.nx <= 48) ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
   s.block = (unsigned)kTileX * s.t.waves;
   s.grid = (s.t.ntiles + s.t.waves - 1) / s.t.waves;
   const bool ab = c.g.lay == LAY_AB;
@@ -658,15 +673,17 @@ static CollideShape collide_shape(const Ctx& c, bool spheres) {
   const uint64_t plane = (uint64_t)NPOP * sizeof(T) * (uint64_t)c.g.nx * (uint64_t)c.g.ny;
   const bool small = 2 * buf <= 48 * mib;
   s.cached = ab && !small && 2 * buf <= 260 * mib;
+  const bool streams64 = ab && all64 && !spheres && c.g.nx >= 32 && 2 * buf >= (tpr <= 4 ? 2560 : 6144) * mib;
   if (sizeof(T) != sizeof(R))
     s.ntl = small || spheres || c.g.nx % 256 == 0;
   else
-    s.ntl = small || (spheres && (sizeof(T) == 8 || (c.g.nx % kTileX == 0 && s.t.waves % tpr == 0)));
+    s.ntl = small || (streams64 && c.g.nx % 8 == 0) ||
+            (spheres && (all64 || (c.g.nx % kTileX == 0 && s.t.waves % tpr == 0)));
   bool ranges;
   if (c.xcd_remap >= 0)
     ranges = c.xcd_remap != 0;
   else if (ab)
-    ranges = plane >= 18 * mib || 2 * buf <= 128 * mib;
+    ranges = plane >= 18 * mib || 2 * buf <= 128 * mib || streams64;
   else
     ranges = !(tpr <= 4 && buf > 256 * mib);
   s.t.per = ranges ? s.grid / kXcds : 0;
