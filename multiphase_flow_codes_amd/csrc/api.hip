@@ -1246,7 +1246,7 @@ int step_overlapped(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       }
       if ((he = hipStreamWaitEvent(sB, c.ev_coll, 0)) != hipSuccess) break;
       // beads_collision with beads_lubforce and the map clearing in its grid
-      c.old_version = 0;   // the next collide is writing the other buffer
+      if (more) c.old_version = 0;   // the next collide is writing the other buffer
       if ((he = launch_bounce_back(c, true)) != hipSuccess) break;
       if ((he = hipEventRecord(c.ev_bb, sB)) != hipSuccess) break;
       c.f_version++;
@@ -1254,10 +1254,13 @@ int step_overlapped(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       if ((he = launch_move(c, it == c.p.irelease ? 1 : 0, 1, true)) != hipSuccess) break;
       P.map_old = P.map_cur;
       if ((prc = links_now(ctx, 1, it))) break;
-      if ((he = launch_filling(c, true, nullptr)) != hipSuccess) break;
+      if ((he = launch_filling(c, wants_contacts(c), nullptr)) != hipSuccess) break;
       c.f_version++;
       if ((prc = mfc_macrovar(ctx))) break;
-      he = hipEventRecord(c.ev_part, sB);
+      if ((he = hipEventRecord(c.ev_part, sB)) != hipSuccess) break;
+      // the contact links the next bounce-back then takes from their list, beside
+      // the collide of the near tiles
+      if (more) he = ensure_contacts(c);
     } while (false);
     c.stream = sA;
     if (he != hipSuccess) return fail(ctx, MFC_ERR_HIP, "overlapped particle phase", he);
@@ -1286,7 +1289,7 @@ int step_overlapped(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
     else
       c.g.lay = c.g.lay == LAY_AA_ODD ? LAY_AA_EVEN : LAY_AA_ODD;
     c.phase = PHASE_PRE_STREAM;
-    c.f_version++;
+    c.old_version = ++c.f_version;
   }
   return MFC_OK;
 }
@@ -1332,14 +1335,15 @@ int mfc_step(mfc_ctx* ctx, int32_t istep, int32_t nsteps) {
       // with its overlap check fused in (reported by mfc_sync)
       HIPCHK(launch_move(c, it == c.p.irelease ? 1 : 0, 1, true));
       P.map_old = P.map_cur;
-      // links, then the refill with the contact links listed in its grid
+      // links, then the refill (the contact links listed in its grid where the
+      // bounce-back takes them from the list)
       if ((rc = links_now(ctx, 1, it))) return rc;
       if (s + 1 < nsteps && c.p.xkf > 0.0) {
         forcing_modes_host(c);
         drawn = true;
         drawn_rc = prepare_modes(ctx, job);
       }
-      HIPCHK(launch_filling(c, true, drawn && !drawn_rc && job.nblk > 0 ? &job : nullptr));
+      HIPCHK(launch_filling(c, wants_contacts(c), drawn && !drawn_rc && job.nblk > 0 ? &job : nullptr));
       c.f_version++;
     }
     if ((rc = mfc_macrovar(ctx))) return rc;

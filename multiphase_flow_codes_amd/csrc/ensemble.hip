@@ -198,7 +198,7 @@ int build_step(mfc_ens* e, StepTabs& T) {
       st[3].lds = std::max(st[3].lds, scan_lds(c));
       P.map_np[target] = P.np;
       P.map_cur = target;
-      const FillKArgs fa = fill_args(c, true, true, &nb);
+      const FillKArgs fa = fill_args(c, true, wants_contacts(c), &nb);
       st[4].add(&fa, nb);
       c.f_version++;
     }

@@ -240,7 +240,7 @@ int segment_capacity(double rad, int slab);
 int segment_planes(double rad, int npart, int want);
 int segment_links(double rad, int slab);
 hipError_t launch_links(Ctx& c, int target, int overlap_check, int istep);
-// does the bounce-back need the list of contact links (else it may)?
+// does the bounce-back of a plain step need the list of contact links?
 bool wants_contacts(const Ctx& c);
 hipError_t ensure_contacts(Ctx& c);
 // ST_NLINKS and ST_NSOLID of the current build
@@ -254,7 +254,7 @@ hipError_t launch_map_clear(Ctx& c, int buf);
 hipError_t launch_move(Ctx& c, int first, int wrap, bool from_seg = false);
 hipError_t launch_redistribute(Ctx& c, int istep);
 struct TableJob;
-// contacts: the grid also lists the contact links, if they are wanted; job: a forcing table
+// contacts: the grid also lists the contact links; job: a forcing table
 // evaluated by extra blocks of it
 hipError_t launch_filling(Ctx& c, bool contacts = false, const TableJob* job = nullptr);
 hipError_t launch_initpartvel(Ctx& c);

@@ -1897,7 +1897,7 @@ FillKArgs fill_args(Ctx& c, bool refill, bool contacts, int* blocks) {
   FillKArgs a;
   a.fa = FillArgs{};
   a.nfill = refill && make_fill_args(c, P.map_old, P.map_cur, a.fa) ? P.map_np[P.map_old] * P.nseg : 0;
-  a.nct = contacts && wants_contacts(c) ? P.np * P.nseg : 0;
+  a.nct = contacts ? P.np * P.nseg : 0;
   if (a.nct) P.ct_ok = true;
   a.ct = contact_args(P);
   a.A = c.pop[c.cur];

@@ -125,6 +125,8 @@ size_t fake_max_lds(const char* part) {
     if (l.name.find(part) != std::string::npos) m = std::max(m, l.lds);
   return m;
 }
+// the i-th launch since the last reset ("" past the end)
+const char* fake_launch(int i) { return (size_t)i < launches.size() ? launches[i].name.c_str() : ""; }
 void fake_reset() {
   launches.clear();
   copies = syncs = foreign = 0;

@@ -163,3 +163,36 @@ def test_padding_of_rows_is_bounded(run):
         lat.upload_macro(*a)
         assert all(np.array_equal(x, y) for x, y in zip(lat.download_macro(), a))
     """)
+
+
+@pytest.mark.parametrize("mode", ["1", "2"])
+@pytest.mark.parametrize("storage", ["ab", "aa"])
+def test_overlapped_step_does_not_wait_for_the_contact_list(run, mode, storage):
+    """Contact links are listed behind the refill (in its grid in place, by a grid
+    beside the near collide with two buffers), not ahead of the bounce-back,
+    except the first one after links built on their own; a call's last
+    bounce-back takes them from the other buffer where there is one."""
+    run(f"""
+        lat = lattice((40, 36, 32), "fp32", "{storage}", npart=2, rad=3.0)
+        lat.upload_macro(*fields((40, 36, 32)))
+        lat.initpop()
+        lat.macrovar()
+        lat.prt_init(2)
+        lat.prt_set("ypglb", np.array([[9.0, 9.0, 9.0], [28.0, 20.0, 21.0]]))
+        lat.beads_links()
+        fake.fake_launch.restype = C.c_char_p
+        ahead = []
+        for first, n in ((1, 6), (7, 3), (10, 1)):
+            fake.fake_reset()
+            lat.step(first, n)
+            names = []
+            while fake.fake_launch(len(names)):
+                names.append(fake.fake_launch(len(names)).decode())
+            names = [x for x in names if any(k in x for k in ("k_contacts", "k_tile_mark", "k_bounce_back", "k_fill"))]
+            assert sum("k_bounce_back" in x for x in names) == n
+            # listed behind the refill, or where the next step's bounce-back starts
+            ahead.append(sum("k_tile_mark" in a and "k_contacts" in b for a, b in zip(names, names[1:])))
+            behind = sum("k_fill" in a and "k_contacts" in b for a, b in zip(names, names[1:]))
+            assert behind == (n - 1 if "{storage}" == "ab" else 0)
+        assert ahead == ([1, 1, 0] if "{storage}" == "ab" else [1, 0, 0])
+    """, MFC_OVERLAP=mode)
