@@ -123,7 +123,8 @@ int mfc_forcing(mfc_ctx* ctx);          /* BOX/gaussian.f90:182-372 */
 int mfc_collision_mrt(mfc_ctx* ctx);    /* BOX/collision.f90:8-210 */
 int mfc_streaming(mfc_ctx* ctx);        /* BOX/streaming.f90:2-171 */
 /* rhoupdat (BOX/collision.f90:213-229); optionally also returns
- * max|rho_new - rho_old|, the pre-relaxation residual of BOX/main.f90:91-96. */
+ * max|rho_new - rho_old|, the pre-relaxation residual of BOX/main.f90:91-96,
+ * over the nodes where that is a number (NaN if at none), as maxval takes it. */
 int mfc_rhoupdat(mfc_ctx* ctx, double* max_abs_change);
 /* The pre-relaxation loop (BOX/main.f90:86-108): collision_MRT, streaming and
  * rhoupdat until its residual is at most eps or the iteration count, from 0,

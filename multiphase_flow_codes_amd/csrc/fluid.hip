@@ -62,6 +62,13 @@ __device__ __forceinline__ void force_row(const double* __restrict__ t, R c1, R 
 }
 
 
+// A density change as an integer whose maximum is the residual's: one above the
+// bits of a non-negative double, which order as integers; 0 for a change that is
+// no number, so that those count only where there is no other.
+__device__ __forceinline__ uint64_t residual_bits(double change) {
+  return change == change ? (uint64_t)__double_as_longlong(change) + 1 : 0;
+}
+
 // Fused stream + macro + forcing + MRT collision.
 //
 // One wavefront per tile of 64 consecutive x nodes of a row (kTileX):
@@ -83,7 +90,7 @@ __device__ __forceinline__ void force_row(const double* __restrict__ t, R c1, R 
 // NTL, NTS: non-temporal loads of the two-buffer field, non-temporal stores
 // (CollideShape says when).
 // RES (with ARR): the density is taken from the populations as rhoupdat takes it
-// and stored; `diff` receives the bits of its change.
+// and stored; `diff` receives the residual_bits of its change.
 template <typename T, typename R, bool ARR, bool WALLS, int LAY, bool NTL, bool NTS, bool RES = false>
 __device__ __forceinline__ void collide_node(const CollideArgs& a, int x, int y, int z, uint64_t* diff = nullptr) {
   const T* __restrict__ A = (const T*)a.A;
@@ -148,7 +155,7 @@ __device__ __forceinline__ void collide_node(const CollideArgs& a, int x, int y,
 #pragma unroll
         for (int i = 1; i < NPOP; ++i) r = r + (double)f[i];
         const double old = a.rho[n];
-        *diff = (uint64_t)__double_as_longlong(fabs(r - old));
+        *diff = residual_bits(fabs(r - old));
         a.rho[n] = r;
         rho = (R)r;
       } else {
@@ -245,7 +252,7 @@ __global__ void __launch_bounds__(256)
 // Pre-relaxation at frozen velocity: the rhoupdat that ends one iteration and
 // the collide that begins the next in one pass over the populations.  Each
 // wavefront leaves its largest density change in one of kRelaxSlots words
-// (as in rhoupdat: NaN above all), zero before.  The collide is wasted once, when
+// (as in rhoupdat), zero before.  The collide is wasted once, when
 // the change has become small enough.  Bound: the populations read and written,
 // rho and u read, rho written.  An iteration of two grids took 843 us at 256^3
 // FP32, 1536 in FP64, 150 at 128 x 120 x 110 FP64 and 17.9 at 32^3 FP32; now
@@ -428,9 +435,8 @@ __global__ void __launch_bounds__(kSumThreads) k_macro_sums(MacroArgs a, double*
 
 // rhoupdat (collision.f90:213-229) plus the pre-relaxation residual
 // max|rho_new - rho_old| (main.f90:91-96): each workgroup walks its share of
-// the nodes and leaves one maximum in part.  The maxima are taken on the bits
-// of |rho_new - rho_old| (non-negative doubles order as integers, NaN above
-// all), so a NaN anywhere is a NaN residual.  Bound: 19 populations and rho
+// the nodes and leaves one maximum in part.  A node whose change is no number
+// is passed over, as maxval passes it over.  Bound: 19 populations and rho
 // read, rho written.  One atomic per 256 nodes on a single word, behind a
 // barrier tree in LDS, set the time before: 796 us at 256^3 FP32 and 88 us at
 // 128 x 120 x 110 FP64, now 338 and 48 us (4.6 and 5.9 TB/s).  16384
@@ -462,7 +468,7 @@ __global__ void __launch_bounds__(256)
     double r = f[0];
 #pragma unroll
     for (int i = 1; i < NPOP; ++i) r = r + f[i];
-    d = max(d, (uint64_t)__double_as_longlong(fabs(r - old)));
+    d = max(d, residual_bits(fabs(r - old)));
     rho[n] = r;
   }
   d = block_max(d);
@@ -483,7 +489,7 @@ __global__ void __launch_bounds__(256)
   }
   d = block_max(d);
   if (threadIdx.x == 0) {
-    *out = d;
+    *out = d ? d - 1 : 0x7ff8000000000000ull;   // no number anywhere: NaN
     __hip_atomic_store((uint32_t*)(out + 1), seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
