@@ -286,10 +286,31 @@ class Lattice:
         collision_MRT, streaming, rhoupdat until max|rho - rho_prev| <= rhoepsl or
         the iteration count passes max_iter; then macrovar.  Returns
         (iterations, final residual)."""
-        it, err = C.c_int32(), C.c_double()
-        self._chk(lib().mfc_prerelax(self.h, float(rhoepsl), math.floor(min(max(max_iter, -1), 2**31 - 2)), C.byref(it), C.byref(err)))
+        if [getattr(getattr(self, f.__name__), "__func__", None) for f in _PRERELAX] != _PRERELAX:
+            it = 0   # replaced ones (a subclass's) are called
+            while True:
+                self.collision_mrt()
+                self.streaming()
+                err = self.rhoupdat()
+                if err <= rhoepsl or it > max_iter:
+                    break
+                it += 1
+            self.macrovar()
+            return it, err
+        # in batches, so that an interrupt is not kept waiting; the first iteration
+        # of a batch costs half of one more than the others
+        it, n, err = 0, C.c_int32(), C.c_double()
+        while True:
+            batch = 128
+            if max_iter - it < batch - 2:
+                batch = max(math.floor(max_iter - it) + 2, 1)
+            self._chk(lib().mfc_prerelax(self.h, float(rhoepsl), batch - 2, C.byref(n), C.byref(err)))
+            it += n.value
+            if err.value <= rhoepsl or it > max_iter:
+                break
+            it += 1
         self.macrovar()
-        return it.value, err.value
+        return it, err.value
 
     # -- particles ---------------------------------------------------------------
     def prt_init(self, npart: int):
@@ -392,6 +413,10 @@ class Lattice:
         n = C.c_int64()
         self._chk(lib().mfc_get_timing(self.h, C.byref(t), C.byref(n)))
         return t.value, n.value
+
+
+# the single calls that prerelax's batches stand for
+_PRERELAX = [Lattice.collision_mrt, Lattice.streaming, Lattice.rhoupdat]
 
 
 class Ensemble:

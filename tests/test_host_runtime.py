@@ -196,3 +196,57 @@ def test_overlapped_step_does_not_wait_for_the_contact_list(run, mode, storage):
             assert behind == (n - 1 if "{storage}" == "ab" else 0)
         assert ahead == ([1, 1, 0] if "{storage}" == "ab" else [1, 0, 0])
     """, MFC_OVERLAP=mode)
+
+
+def test_prerelax_answers_an_interrupt(run):
+    """A signal handler's exception ends the loop after a batch of iterations, not
+    after all of them; counts and stops as one iteration after the other."""
+    run("""
+        import math, signal
+        lat = lattice((8, 8, 8))
+        def start():
+            lat.upload_macro(*fields((8, 8, 8)))
+            lat.initpop()
+            fake.fake_reset()
+        start()
+        # the CPU runtime's residual is 0
+        assert lat.prerelax(0.0, 5) == (0, 0.0)
+        for m in (-3, -1, 0, 1, 2.5, 125, 126, 127, 128, 129, 254.9, 300):
+            start()
+            it, err = lat.prerelax(-1.0, m)
+            assert (it, err) == (max(math.floor(m) + 1, 0), 0.0), (m, it)
+            assert fake.fake_launches(b"k_rho_residual") == it + 1
+        def stop(*_):
+            raise KeyboardInterrupt
+        signal.signal(signal.SIGALRM, stop)
+        for limit in (300000, math.inf, math.nan):
+            start()
+            signal.setitimer(signal.ITIMER_REAL, 0.03)
+            try:
+                lat.prerelax(-1.0, limit)
+                raise AssertionError
+            except KeyboardInterrupt:
+                pass
+            assert fake.fake_launches(b"k_rho_residual") < 290000
+    """)
+
+
+def test_prerelax_calls_replaced_methods(run):
+    run("""
+        class Counting(Lattice):
+            n = 0
+            def rhoupdat(self):
+                self.n += 1
+                return super().rhoupdat() + (1.0 if self.n < 4 else 0.0)
+        lat = Counting(small_params(n=(8, 8, 8), forcing=False), "fp64")
+        lat.upload_macro(*fields((8, 8, 8)))
+        lat.initpop()
+        assert lat.prerelax(0.5) == (3, 0.0) and lat.n == 4
+        lat = lattice((8, 8, 8))
+        lat.upload_macro(*fields((8, 8, 8)))
+        lat.initpop()
+        seen = []
+        step = lat.streaming
+        lat.streaming = lambda: (seen.append(1), step())
+        assert lat.prerelax(-1.0, 2) == (3, 0.0) and len(seen) == 4
+    """)
