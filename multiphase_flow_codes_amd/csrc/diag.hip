@@ -357,6 +357,11 @@ __device__ __forceinline__ void small_pass(const FftArgs& a, const double2* src,
   }
 }
 
+// LDS entries from one index of k_fft_any's lines to the next: x lines are
+// loaded along j, so the rows of several are padded.
+template <int AXIS>
+__host__ __device__ constexpr int any_row(int tx) { return AXIS == AXIS_X && tx > 1 ? tx + 1 : tx; }
+
 // Any length: passes over the factors of n (4, 2, 3, 5, then the remaining
 // primes by their sums, outputs m and r - m together) between two LDS buffers.
 // Bound: those sums.  A spectrum of 150 x 141 x 162 nodes (141 = 3 x 47) takes
@@ -367,7 +372,7 @@ __global__ void __launch_bounds__(256)
     k_fft_any(FftArgs a) {
   extern __shared__ double2 lbuf[];
   const int n = a.n;
-  const int row = AXIS == AXIS_X ? a.tx + 1 : a.tx;   // x lines are loaded along j: pad the tile's rows
+  const int row = any_row<AXIS>(a.tx);
   auto slot = [&](int j, int t) { return j * row + t; };
   double* bins = (double*)(lbuf + 2 * (size_t)n * row);
   if (AXIS == AXIS_Z) {
@@ -545,7 +550,9 @@ static hipError_t launch_fft(const Grid& g, FftArgs a, int comps, hipStream_t s,
   a.n = AXIS == AXIS_X ? g.nx : (AXIS == AXIS_Y ? g.ny : g.nz);
   const bool pow2 = ilog2_exact(a.n) >= 3;
   // lines per tile: eight (runs of 128 B), more where eight are too few to
-  // fill a wavefront, fewer where the tile would outgrow 80 KB of LDS
+  // fill a wavefront, fewer where they would be more than 4096 (two buffers:
+  // 2048) entries: at most 72 KB of LDS and the shells of the z pass, along x
+  // 96 KB (two padded lines of 1023 entries)
   const int most = pow2 ? 4096 : 2048;
   a.ltx = 3;
   while ((a.n << a.ltx) < 512) ++a.ltx;
@@ -563,7 +570,7 @@ static hipError_t launch_fft(const Grid& g, FftArgs a, int comps, hipStream_t s,
   for (int r = 4, m = a.n; m > 1; r = r == 4 ? 2 : (r == 2 ? 3 : r + 2))
     for (; m % r == 0; m /= r) a.f[a.nf++] = r;
   size_t lds = sizeof(double2) * (pow2 ? (size_t)(a.n + a.n / 8) * a.tx
-                                       : 2 * (size_t)a.n * (AXIS == AXIS_X ? a.tx + 1 : a.tx));
+                                       : 2 * (size_t)a.n * any_row<AXIS>(a.tx));
   int nb = a.tiles;
   if (AXIS == AXIS_Z) {
     lds += sizeof(double) * a.nek;

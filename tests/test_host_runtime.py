@@ -250,3 +250,27 @@ def test_prerelax_calls_replaced_methods(run):
         lat.streaming = lambda: (seen.append(1), step())
         assert lat.prerelax(-1.0, 2) == (3, 0.0) and len(seen) == 4
     """)
+
+
+def test_spectrum_stays_within_its_lds(run):
+    """Transform tiles of lines of up to 2048 entries take at most 96 KB of LDS
+    along x, and 72 KB along y and z with 8 B more per shell along z."""
+    run("""
+        def spectrum(n, nek):
+            lat = lattice(n, "fp32")
+            lat.upload_macro(*fields(n))
+            fake.fake_reset()
+            ek = np.zeros(nek)
+            assert lib().mfc_diag_spectrum(lat.h, nek, _dp(ek)) == 0
+            assert fake.fake_launches(b"invalid") == 0
+            return fake.fake_max_lds(b"k_fft")
+
+        sizes = [4, 5, 7, 12, 64, 100, 127, 128, 250, 256, 500, 512, 1000, 682, 683, 1023, 1024, 1025, 1536, 2047, 2048]
+        for m in sizes:
+            for axis in range(3):
+                n = [4, 4, 4]
+                n[axis] = m
+                for nek in (8, 4096):
+                    got = spectrum(tuple(n), nek)
+                    assert got <= max(96 * 1024, 72 * 1024 + 8 * nek), (n, nek, got)
+    """)
