@@ -171,7 +171,8 @@ int mfc_beads_collision(mfc_ctx* ctx);  /* BOX/partlib.f90:1064-1717 */
 int mfc_set_bb_order(mfc_ctx* ctx, int32_t order);
 /* Lattice planes per unit of particle work (1, 2, 4 or 8; 0: by size), before
  * mfc_prt_init.  By size, few spheres are cut into many units so that they
- * fill the GPU on their own; 4 suits a box that shares it with many others. */
+ * fill the GPU on their own; 4 suits a box that shares it with many others
+ * (dozens in one ensemble: 3-5 % of a step). */
 int mfc_set_segment_planes(mfc_ctx* ctx, int32_t planes);
 int mfc_beads_lubforce(mfc_ctx* ctx);   /* BOX/partlib.f90:2211-2292 */
 int mfc_beads_move(mfc_ctx* ctx, int32_t istep);         /* BOX/partlib.f90:2295-2394 */

@@ -3,12 +3,13 @@
 // Each member is an ordinary context (its own size, spheres, rates and body
 // force; state created and initialised through the single-box API).  One
 // ensemble step runs the time-loop body of every member with one grid per
-// stage for all of them: collide, contact links (members in the
-// reference's order only), bounce-back (+ lubrication, map clearing), move, link scan, refill (+ contact search).  Each grid reads its members' argument blocks from a
-// per-stage table and finds its member from a block-offset table
-// (off[c] <= blockIdx.x < off[c+1]).  The sequence and the per-member state
-// transitions are exactly those of mfc_step, so a member advanced in the
-// ensemble is bitwise identical to the same box advanced alone.
+// stage for all of them: collide, contact links (members in the reference's
+// order only), bounce-back (+ lubrication, map clearing), move, link scan,
+// refill (+ contact search for those members).  Each grid reads its members'
+// argument blocks from a per-stage table and finds its member from a
+// block-offset table (off[c] <= blockIdx.x < off[c+1]).  The sequence and the
+// per-member state transitions are exactly those of mfc_step, so a member
+// advanced in the ensemble is bitwise identical to the same box advanced alone.
 //
 // Steps go in chunks of up to kChunk: the host builds the tables of all the
 // chunk's steps into one pinned buffer and uploads them with ONE plain copy;

@@ -319,8 +319,8 @@ __device__ __forceinline__ int case_of_block(const int* __restrict__ off, int nc
 // ARR_ANY: some member takes its moments from the rho/u arrays (a.arr, its
 // first step after joining); without it only the recomputing path is built.
 // remap = 1 deals the grid to the 8 XCDs in contiguous ranges: consecutive
-// node ranges, whose neighbour rows overlap, then share one L2.  The block-to-nodes map is a bijection either way, so results do
-// not depend on it.
+// node ranges, whose neighbour rows overlap, then share one L2.  The
+// block-to-nodes map is a bijection either way, so results do not depend on it.
 // NTL: non-temporal loads, where most nodes lie in rows of whole 64-B half lines (32
 // boxes of 32 to 128 nodes an edge FP64 1697 us a step against 1748 plain, FP32 928
 // against 935).  In other rows neighbouring blocks need the same lines: plain

@@ -27,7 +27,7 @@
 namespace mfc {
 
 constexpr int PB = 256;  // threads per particle workgroup
-// A segment is one z-slab (G.slab planes, 4 or 8) of one particle's bounding
+// A segment is one z-slab (G.slab planes: 1, 2, 4 or 8) of one particle's bounding
 // box: the unit of work of every box-scan kernel, so a sphere spreads over
 // several workgroups.  Segment s of particle p is block p * nseg + s.
 
@@ -433,7 +433,7 @@ __device__ __forceinline__ void block_place2(bool fa, bool fb, int (*wt)[PB / 64
 // (the marks come in a later grid), so each listed node's id and its whole
 // 32-node mask word are stored as zero: no read, no atomic; a word or a node
 // listed by several spheres receives the same zero from each.
-__device__ void clear_segment(int b, int nseg, int seg_cap, const uint32_t* __restrict__ sol_list,
+__device__ void clear_segment(int b, int seg_cap, const uint32_t* __restrict__ sol_list,
                               const int32_t* __restrict__ sol_cnt, int32_t* __restrict__ isn,
                               uint32_t* __restrict__ mask) {
   const int cnt = sol_cnt[b];
@@ -446,10 +446,10 @@ __device__ void clear_segment(int b, int nseg, int seg_cap, const uint32_t* __re
 }
 
 __global__ void __launch_bounds__(PB)
-    k_map_clear(int nseg, int seg_cap, const uint32_t* __restrict__ sol_list,
+    k_map_clear(int seg_cap, const uint32_t* __restrict__ sol_list,
                 const int32_t* __restrict__ sol_cnt, int32_t* __restrict__ isn,
                 uint32_t* __restrict__ mask) {
-  clear_segment(blockIdx.x, nseg, seg_cap, sol_list, sol_cnt, isn, mask);
+  clear_segment(blockIdx.x, seg_cap, sol_list, sol_cnt, isn, mask);
 }
 
 // beads_links (partlib.f90:934-1043) for one segment of a particle's box:
@@ -1102,7 +1102,7 @@ __device__ __forceinline__ void bounce_back_body(int b_, const BounceArgs& a) {
   const int u = b_ - a.nlub;
   if (u >= nunits) {
     if (u - nunits < a.nclr) {
-      clear_segment(u - nunits, a.nseg, a.seg_cap, a.clr_list, a.clr_cnt, a.clr_isn, a.clr_mask);
+      clear_segment(u - nunits, a.seg_cap, a.clr_list, a.clr_cnt, a.clr_isn, a.clr_mask);
     } else {   // the counts of the pair-search cells the coming move fills
       const int i = (u - nunits - a.nclr) * PB + (int)threadIdx.x;
       if (i < a.ncell) a.clr_cells[i] = 0;
@@ -1653,7 +1653,6 @@ static PGeom pgeom(const Ctx& c) {
   G.radp2 = c.p.rad * 1.0 + 2.0;
   G.r2 = (c.p.rad * 1.0) * (c.p.rad * 1.0);
   G.rlink2 = (c.p.rad + 1.5) * (c.p.rad + 1.5);
-  G.rsolid2 = (c.p.rad + 0.5) * (c.p.rad + 0.5);
   G.slab = c.pt.slab;
   G.dseg = fast_div((uint32_t)c.pt.nseg);
   return G;
@@ -1680,8 +1679,9 @@ int segment_capacity(double rad, int slab) {
 // diagonal), and a direction across the planes as many as lines meet the sphere
 // or the part of its surface in the segment, whichever is fewer (a band of
 // height h has the projected area pi r h, a cap 2 pi r h; sqrt(2) lines per unit
-// area along a diagonal), each with a margin of a node.  1.9 to 3 times the
-// largest count met over radii from 2 to 27 and random centres.
+// area along a diagonal), each with a margin of a node.  Over radii from 2 to 27
+// and random centres it is 1.7 (8 planes) to 5.7 times (1 plane, radius 2) the
+// largest count met.
 int segment_links(double rad, int slab) {
   const double r = rad + 1.0, disc = M_PI * r * r, h = slab + 1.0;
   const double in_plane = slab * (4.0 * (2.0 * r) + 4.0 * (2.0 * sqrt(2.0) * rad + 2.0));
@@ -1728,7 +1728,7 @@ int segment_planes(double rad, int npart, int want) {
 hipError_t launch_map_clear(Ctx& c, int buf) {
   Particles& P = c.pt;
   if (P.map_np[buf] > 0)
-    hipLaunchKernelGGL(k_map_clear, dim3(P.map_np[buf] * P.nseg), dim3(PB), 0, c.stream, P.nseg, P.seg_cap,
+    hipLaunchKernelGGL(k_map_clear, dim3(P.map_np[buf] * P.nseg), dim3(PB), 0, c.stream, P.seg_cap,
                        P.sol_list[buf], P.sol_cnt[buf], P.isn[buf], P.mask[buf]);
   P.map_np[buf] = 0;
   return hipGetLastError();
@@ -1833,7 +1833,6 @@ size_t scan_lds(const Ctx& c) {
          sizeof(SegRow) * (size_t)(c.pt.slab * box_candidates(c.p.rad));
 }
 
-// fused: the lubrication forces ride in the same grid
 // fused (mfc_step): lubrication blocks, and the map buffer the coming links
 // rebuild (map_cur ^ 1, built two steps ago) cleared in the same grid and
 // marked empty

@@ -33,8 +33,6 @@ struct PGeom {
   // solid nor has a link, since every lattice vector is shorter than 1.5
   // (the margin over sqrt(2) dwarfs any rounding of the squared distances)
   double rlink2;
-  // (r + 0.5)^2: no solid node lies farther out than this
-  double rsolid2;
   // z planes per segment (Particles::slab)
   int slab;
   FastDiv dseg;   // division by the segments per particle
