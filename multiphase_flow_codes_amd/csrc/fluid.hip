@@ -617,7 +617,12 @@ CollideArgs collide_args(Ctx& c) {
 //          up to three quarters of a tile, whose idle lanes leave the wavefront
 //          slots as the bound (24 million nodes: nx = 5 f 5.62 against 6.79 ms,
 //          17 1.87 against 2.20, 48 1.15 against 1.21; nx = 50 1.32 against
-//          1.24; FP32 nx = 17 0.96 and 0.99).
+//          1.24; FP32 nx = 17 0.96 and 0.99).  In place with FP64 arithmetic one
+//          or two tiles of a row, with ranges: FP32 storage (24 x 256 x 3906 f
+//          1207 against 1297 us, 64 x 256 x 1464 676 against 703, 128 x 256 x 732
+//          681 against 719, 128 x 160 x 400 s 316 against 323), FP64 from a GiB a
+//          tile (64 x 256 x 600 s 590 against 669, 128 x 256 x 732 f 1346 against
+//          1358; 100 x 256 x 500, 1.8 GiB, 749 against 717).
 //  cached  plain stores where both buffers stay in the 256 MiB last-level
 //          cache between steps: from 48 MiB (64^3 FP32, 38 MiB, s 13.1 against
 //          11.6 non-temporal; 64^3 FP64, 76 MiB, s 18.6 against 20.2, f 14.0
@@ -651,7 +656,7 @@ CollideArgs collide_args(Ctx& c) {
 //          against 721).  In place: always (1024^3 FP64 f 52.5 against 64 ms,
 //          130 x 118 x 126 FP32 47 against 58), but rows of up to four tiles
 //          that outgrow the last-level cache (200 x 190 x 210 FP64 f 461
-//          against 441).
+//          against 441) up to 2 GiB of FP64 (256 x 256 x 320 f 1052 against 1173).
 // One workgroup per row or 256-node chunk of a row, the shape before, left
 // half of its lanes idle where a row ends in a short chunk: 320 x 288 x 304
 // FP32 f 912 us (now 715) and FP64 in place 1790 (now 1575), 262 x 257 x 227
@@ -669,13 +674,15 @@ static CollideShape collide_shape(const Ctx& c, bool spheres) {
   const uint32_t tpr = (uint32_t)((c.g.nx + kTileX - 1) / kTileX);
   s.t.tpr = fast_div(tpr);
   s.t.ntiles = tpr * (uint32_t)c.g.ny * (uint32_t)c.g.nz;
-  const bool all64 = sizeof(T) == 8;
-  s.t.waves = s.t.ntiles <= 4096 || (all64 && c.g.nx <= 48) ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
-  s.block = (unsigned)kTileX * s.t.waves;
-  s.grid = (s.t.ntiles + s.t.waves - 1) / s.t.waves;
-  const bool ab = c.g.lay == LAY_AB;
+  const bool ab = c.g.lay == LAY_AB, all64 = sizeof(T) == 8;
   const uint64_t mib = (uint64_t)1 << 20;
   const uint64_t buf = (uint64_t)NPOP * sizeof(T) * c.g.ncell;
+  // in place with FP64 arithmetic: a workgroup per row
+  const bool row_groups = !ab && sizeof(R) == 8 && tpr <= 2 && (!all64 || c.g.nx <= 48 || buf >= tpr * 1024 * mib);
+  s.t.waves = s.t.ntiles <= 4096 || (all64 && c.g.nx <= 48) ? 1 : (tpr % 4 != 0 && tpr % 3 == 0 ? 3 : 4);
+  if (row_groups && s.t.ntiles > 4096) s.t.waves = tpr;
+  s.block = (unsigned)kTileX * s.t.waves;
+  s.grid = (s.t.ntiles + s.t.waves - 1) / s.t.waves;
   const uint64_t plane = (uint64_t)NPOP * sizeof(T) * (uint64_t)c.g.nx * (uint64_t)c.g.ny;
   const bool small = 2 * buf <= 48 * mib;
   s.cached = ab && !small && 2 * buf <= 260 * mib;
@@ -691,7 +698,7 @@ static CollideShape collide_shape(const Ctx& c, bool spheres) {
   else if (ab)
     ranges = plane >= 18 * mib || 2 * buf <= 128 * mib || streams64;
   else
-    ranges = !(tpr <= 4 && buf > 256 * mib);
+    ranges = row_groups || !(tpr <= 4 && buf > 256 * mib) || (all64 && buf >= 2048 * mib);
   s.t.per = ranges ? s.grid / kXcds : 0;
   return s;
 }
